@@ -38,6 +38,8 @@ constexpr int CPML_NM = 45;  // complete C-PML memories per point and field
 
 enum { ASM_COLORED = 0, ASM_ATOMIC = 1, ASM_GATHER = 2 };
 
+struct ClusterHead;  // cluster.hpp
+
 struct ElemArgs {
     // geometry, SoA over element points in the solver's element order
     const float* __restrict__ G;        // [9][P]: dxi_dx[m*3+a] * sqrt(J w_i w_j w_k)
@@ -84,6 +86,14 @@ struct ElemArgs {
     const float* __restrict__ att_c;
     float* __restrict__ zeta;
     float* __restrict__ devp;
+    // clusters (GATHER, wavefront form): heads, point lists, entries of the
+    // nodes shared with other clusters, and what the interior update needs
+    const ClusterHead* __restrict__ cl_head;
+    const uint16_t* __restrict__ cl_ent;
+    const int32_t* __restrict__ cl_bdst;
+    const float* __restrict__ minv;
+    float* Uw;
+    float* Ww;
     float D[25];
 };
 
@@ -1279,14 +1289,6 @@ __global__ void __launch_bounds__(64 * WPB) k_element_wave(ElemArgs A, int e0, i
     wave_body<WPB, MODE, DIAG>(A, e0, ne, xcd_block(blockIdx.x, gridDim.x));
 }
 
-// One launch for the element ranges of several solvers, wavefront form.
-template <int WPB, int MODE, bool DIAG>
-__global__ void __launch_bounds__(64 * WPB)
-    k_element_wave_grp(const ElemArgs* __restrict__ tab, const int4* __restrict__ map) {
-    const int4 E = map[xcd_block(blockIdx.x, gridDim.x)];
-    wave_body<WPB, MODE, DIAG>(const_row(tab, E.x), E.y, E.z, E.w);
-}
-
 // Fixed-order sum of a node's element contributions (GATHER assembly): the
 // node's first point (its entry at the node id) added to 0, then the other
 // points' entries (slots [kb, ke) of the node) in increasing solver order.
@@ -1362,6 +1364,106 @@ struct Vec3 {
     float v[3];
 };
 
+// What a special node keeps over the fields.
+struct SpecialNode {
+    float mi, dmp;
+    bool pml;
+    bool use[3];  // C-PML memory directions in use
+    float C[5], al[9];
+};
+
+__device__ __forceinline__ SpecialNode special_node(const NodeArgs& A, int64_t g) {
+    SpecialNode N;
+    N.mi = A.minv[g];
+    N.dmp = A.damp ? A.damp[g] : 0.f;
+    N.pml = A.pml_nodal && g < A.Gpml;
+#pragma unroll
+    for (int q = 0; q < 5; ++q) N.C[q] = N.pml ? A.pc[q * A.Gpml + g] : 0.f;
+#pragma unroll
+    for (int q = 0; q < 9; ++q) N.al[q] = N.pml ? A.palpha[q * A.Gpml + g] : 0.f;
+    const uint32_t mk = N.pml ? A.pmask[g] : 0u;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) N.use[d] = (mk >> d) & 1u;
+    return N;
+}
+
+// One field's state of a special node.  C-PML memory of unused directions is
+// zero and stays zero (alpha = (1, 0, 0), C = 0): neither read nor written.
+struct SpecialState {
+    float U[3], W[3], an[3], pn[3], m[9];
+};
+
+__device__ __forceinline__ void load_special(const NodeArgs& A, const SpecialNode& N, int64_t g, int f, SpecialState& S) {
+    const int64_t o = int64_t(f) * A.fstride + g * 3;
+    const int64_t oa = int64_t(f) * A.astride + g * 3;
+    const float* pmem = A.pmem + int64_t(f) * 9 * A.Gpml;
+    const float* pnew = A.pnew + int64_t(f) * 3 * A.Gpml;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        S.U[c] = A.U[o + c];
+        S.W[c] = A.W[o + c];
+        S.an[c] = A.Aacc[oa + c];
+        S.pn[c] = N.pml ? pnew[c * A.Gpml + g] : 0.f;
+    }
+#pragma unroll
+    for (int q = 0; q < 9; ++q) S.m[q] = (N.pml && N.use[q % 3]) ? pmem[q * A.Gpml + g] : 0.f;
+}
+
+// C-PML terms, legacy damping, massless rule, corrector and next predictor of
+// one special node and field from its assembled residual R; a_n kept.
+__device__ __forceinline__ void update_special(const NodeArgs& A, const SpecialNode& N, int64_t g, int f,
+                                               const SpecialState& S, float* R) {
+    const float dt = A.dt, hdt = 0.5f * dt, hdt2 = 0.5f * dt * dt;
+    const int64_t o = int64_t(f) * A.fstride + g * 3;
+    const int64_t oa = int64_t(f) * A.astride + g * 3;
+    float* pmem = A.pmem + int64_t(f) * 9 * A.Gpml;
+    float* pnew = A.pnew + int64_t(f) * 3 * A.Gpml;
+    float un[3], vn[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        un[c] = S.U[c] - dt * S.W[c];
+        vn[c] = S.W[c] - hdt * S.an[c];
+    }
+    if (N.pml) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const float oldv = S.pn[c] + A.c2 * S.an[c];  // pml.cpp:91-109
+            const float newv = un[c] + A.c1 * vn[c];      // pml.cpp:72-89
+            R[c] += N.C[0] * vn[c] + N.C[1] * un[c] + N.C[2] * S.m[c * 3 + 0] + N.C[3] * S.m[c * 3 + 1] +
+                    N.C[4] * S.m[c * 3 + 2];  // pml.cpp:209-212, assembled over PML elements
+#pragma unroll
+            for (int d = 0; d < 3; ++d)  // pml.cpp:133-146
+                if (N.use[d])
+                    pmem[(c * 3 + d) * A.Gpml + g] =
+                        N.al[d * 3 + 0] * S.m[c * 3 + d] + N.al[d * 3 + 1] * newv + N.al[d * 3 + 2] * oldv;
+            pnew[c * A.Gpml + g] = newv;
+        }
+    }
+    Vec3 nu, nw, na;  // stored as 12-byte words
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        // legacy ramp v -= d v before the corrector (solver.cpp:565-573)
+        const float vp = (N.dmp > 0.f) ? vn[c] - N.dmp * vn[c] : vn[c];
+        float u1, a1, v1;
+        if (N.mi > 0.f) {
+            u1 = (N.dmp > 0.f) ? un[c] + dt * vp + hdt2 * S.an[c] : S.U[c];
+            a1 = R[c] * N.mi;
+            v1 = vp + hdt * (S.an[c] + a1);
+        } else {  // m <= 0: a = 0, u and v kept (solver.cpp:57-61)
+            u1 = un[c];
+            a1 = 0.f;
+            v1 = vp;
+        }
+        const float w1 = v1 + hdt * a1;
+        nu.v[c] = u1 + dt * w1;
+        nw.v[c] = w1;
+        na.v[c] = a1;
+    }
+    *reinterpret_cast<Vec3*>(A.U + o) = nu;
+    *reinterpret_cast<Vec3*>(A.W + o) = nw;
+    *reinterpret_cast<Vec3*>(A.Aacc + oa) = na;
+}
+
 // Special nodes [0, Ga): C-PML terms, legacy damping, massless rule, a_n kept.
 // FG field groups per workgroup: the 256 lanes cover 256/FG nodes, and lane
 // group fy handles fields fy, fy + FG, ... (each wavefront stays on one field
@@ -1379,21 +1481,7 @@ __device__ __forceinline__ void node_special_body(const NodeArgs& A, int blk) {
     const bool staged = STAGE && A.gather;  // uniform over the workgroup
     if (!active && !staged) return;
     const int64_t g = active ? g0 : A.Ga - 1;
-    const float mi = A.minv[g];
-    const float dt = A.dt, hdt = 0.5f * dt, hdt2 = 0.5f * dt * dt;
-    const float dmp = A.damp ? A.damp[g] : 0.f;
-    const bool pml = A.pml_nodal && g < A.Gpml;
-    float C[5] = {0.f, 0.f, 0.f, 0.f, 0.f}, al[9];
-    bool use[3] = {false, false, false};
-    if (pml) {
-#pragma unroll
-        for (int q = 0; q < 5; ++q) C[q] = A.pc[q * A.Gpml + g];
-#pragma unroll
-        for (int q = 0; q < 9; ++q) al[q] = A.palpha[q * A.Gpml + g];
-        const uint32_t mk = A.pmask[g];
-#pragma unroll
-        for (int dd = 0; dd < 3; ++dd) use[dd] = (mk >> dd) & 1u;
-    }
+    const SpecialNode N = special_node(A, g);
     int kb[2] = {0, 0};
     int64_t s0 = 0, s1 = 0;
     bool ids = false;
@@ -1408,24 +1496,10 @@ __device__ __forceinline__ void node_special_body(const NodeArgs& A, int blk) {
         }
     }
     for (int f = fy; f < A.nf; f += FG) {
-        const int64_t o = int64_t(f) * A.fstride + g * 3;
-        const int64_t oa = int64_t(f) * A.astride + g * 3;
-        float* pmem = A.pmem + int64_t(f) * 9 * A.Gpml;
-        float* pnew = A.pnew + int64_t(f) * 3 * A.Gpml;
-        float U[3], W[3], R[3], an[3], un[3], vn[3];
-        // this field's node state first, so that its loads overlap the slot sums;
-        // C-PML memory of unused directions is zero and stays zero (alpha = (1, 0, 0),
-        // C = 0): neither read nor written
-        float m[9], pn[3];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            U[c] = A.U[o + c];
-            W[c] = A.W[o + c];
-            an[c] = A.Aacc[oa + c];
-            pn[c] = pml ? pnew[c * A.Gpml + g] : 0.f;
-        }
-#pragma unroll
-        for (int q = 0; q < 9; ++q) m[q] = (pml && use[q % 3]) ? pmem[q * A.Gpml + g] : 0.f;
+        // this field's node state first, so that its loads overlap the slot sums
+        SpecialState S;
+        load_special(A, N, g, f, S);
+        float R[3];
         if (staged) {
             const Vec3 rm = *reinterpret_cast<const Vec3*>(A.Rl + (int64_t(f) * A.PR + g) * 3);
             const float main[3] = {rm.v[0], rm.v[1], rm.v[2]};
@@ -1435,51 +1509,9 @@ __device__ __forceinline__ void node_special_body(const NodeArgs& A, int blk) {
             gather_r(A, f, g, kb[0], kb[1], R);
         } else {
 #pragma unroll
-            for (int c = 0; c < 3; ++c) R[c] = A.R[o + c];
+            for (int c = 0; c < 3; ++c) R[c] = A.R[int64_t(f) * A.fstride + g * 3 + c];
         }
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            un[c] = U[c] - dt * W[c];
-            vn[c] = W[c] - hdt * an[c];
-        }
-        if (pml) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                const float oldv = pn[c] + A.c2 * an[c];  // pml.cpp:91-109
-                const float newv = un[c] + A.c1 * vn[c];                 // pml.cpp:72-89
-                R[c] += C[0] * vn[c] + C[1] * un[c] + C[2] * m[c * 3 + 0] + C[3] * m[c * 3 + 1] +
-                        C[4] * m[c * 3 + 2];  // pml.cpp:209-212, assembled over PML elements
-#pragma unroll
-                for (int d = 0; d < 3; ++d)  // pml.cpp:133-146
-                    if (use[d])
-                        pmem[(c * 3 + d) * A.Gpml + g] =
-                            al[d * 3 + 0] * m[c * 3 + d] + al[d * 3 + 1] * newv + al[d * 3 + 2] * oldv;
-                pnew[c * A.Gpml + g] = newv;
-            }
-        }
-        Vec3 nu, nw, na;  // stored as 12-byte words
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            // legacy ramp v -= d v before the corrector (solver.cpp:565-573)
-            const float vp = (dmp > 0.f) ? vn[c] - dmp * vn[c] : vn[c];
-            float u1, a1, v1;
-            if (mi > 0.f) {
-                u1 = (dmp > 0.f) ? un[c] + dt * vp + hdt2 * an[c] : U[c];
-                a1 = R[c] * mi;
-                v1 = vp + hdt * (an[c] + a1);
-            } else {  // m <= 0: a = 0, u and v kept (solver.cpp:57-61)
-                u1 = un[c];
-                a1 = 0.f;
-                v1 = vp;
-            }
-            const float w1 = v1 + hdt * a1;
-            nu.v[c] = u1 + dt * w1;
-            nw.v[c] = w1;
-            na.v[c] = a1;
-        }
-        *reinterpret_cast<Vec3*>(A.U + o) = nu;
-        *reinterpret_cast<Vec3*>(A.W + o) = nw;
-        *reinterpret_cast<Vec3*>(A.Aacc + oa) = na;
+        update_special(A, N, g, f, S, R);
     }
 }
 
@@ -1688,12 +1720,35 @@ __global__ void __launch_bounds__(((EPB * NP + 63) / 64) * 64) k_record(RecArgs 
 // node's slots summed in increasing slot order, starting from 0 -- the sum the
 // node kernels form in registers, so a corrector reading R gives the same
 // bits.  One lane per node of [0, G4); nodes without slots get 0.
-__global__ void __launch_bounds__(256) k_scatter_slots(NodeArgs A) {
+// new_cluster (may be null): 1 at the slots where the points of a node's next
+// cluster begin; each cluster's points are then summed first, and the clusters'
+// sums after them, as the cluster kernel and the node kernels do together.
+__global__ void __launch_bounds__(256) k_scatter_slots(NodeArgs A, const uint8_t* __restrict__ new_cluster) {
     const int64_t n = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     const int f = blockIdx.y;
     if (n >= A.G4) return;
     float r[3];
-    gather_r(A, f, n, A.off[n], A.off[n + 1], r);
+    if (new_cluster) {
+        const float* Rl = A.Rl + int64_t(f) * A.PR * 3;
+        float p[3];
+        for (int k = 0; k < 3; ++k) {
+            r[k] = 0.f;
+            p[k] = 0.f + Rl[n * 3 + k];
+        }
+        for (int q = A.off[n]; q < A.off[n + 1]; ++q) {
+            const float* c = Rl + int64_t(A.pts[q]) * 3;
+            for (int k = 0; k < 3; ++k) {
+                if (new_cluster[q]) {
+                    r[k] += p[k];
+                    p[k] = 0.f;
+                }
+                p[k] += c[k];
+            }
+        }
+        for (int k = 0; k < 3; ++k) r[k] += p[k];
+    } else {
+        gather_r(A, f, n, A.off[n], A.off[n + 1], r);
+    }
     float* o = A.R + int64_t(f) * A.fstride + n * 3;
     o[0] = r[0];
     o[1] = r[1];

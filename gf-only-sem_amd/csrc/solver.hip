@@ -17,6 +17,7 @@
 #include <numeric>
 
 #include "common.hpp"
+#include "cluster.hpp"
 #include "kernels.hpp"
 
 #include "device.hpp"
@@ -34,7 +35,25 @@ struct ElemRange {
     bool diag;
     bool pml;
     int ax;  // complete C-PML: the axes (bit 0 x, 1 y, 2 z) with d != 0 at some point of the range's elements
+    int cb, ce;  // GATHER: the range's clusters
 };
+
+// Where GATHER assembly leaves residuals: node n sums the entries
+// pts_host[off_host[n], off_host[n+1]) of Rl, the first being entry n itself;
+// on the device off / pts list all but that first one.  Two forms: one entry
+// per element point (rdst[point]; every element kernel but the cluster form),
+// or one per cluster and node (the cluster kernel).
+struct GatherPlan {
+    bool ready = false;
+    int64_t PR = 0;  // entries per field
+    std::vector<int32_t> off_host, pts_host;
+    DevBuf<int32_t> off, pts, rdst;
+    DevBuf<uint8_t> new_cluster;  // point form: slots where a node's next cluster begins
+    DevBuf<float> Rl;
+};
+
+// Which buffer holds the last step's residual.
+enum { R_ASSEMBLED = 0, R_POINTS = 1, R_CLUSTERS = 2 };
 
 struct FieldSource {
     int direction = -1;
@@ -81,16 +100,20 @@ struct gfx_solver {
     gfx::DevBuf<float> pc, palpha, pabar, pmem, pnew;
     gfx::DevBuf<uint8_t> pmask;  // nodal C-PML: memory directions in use (bits x, y, z)
     gfx::DevBuf<int32_t> pml_slot, src_off;
-    gfx::DevBuf<float> U, W, R, Aacc, Rl;
-    // GATHER assembly: node n owns slots [goff_host[n], goff_host[n+1]); slot q
-    // sums the entry gpts_host[q] of Rl (increasing in solver order per node;
-    // the first is the node's own index).  On the device goff / gpts list
-    // every slot but the first, which the node kernels read at the node id.
-    gfx::DevBuf<int32_t> goff, gpts;
-    std::vector<int32_t> goff_host, gpts_host;
-    // entry of each element point in Rl ([P]) and entries per field (G4 + P - G)
-    gfx::DevBuf<int32_t> rdst;
-    int64_t PR = 0;
+    gfx::DevBuf<float> U, W, R, Aacc;
+    // GATHER assembly: residual entries per element point (built when a kernel
+    // needs it) and per cluster
+    gfx::GatherPlan by_point, by_cluster;
+    // clusters of elements (GATHER): cluster c is the solver elements
+    // [cl_begin[c], cl_begin[c+1]); the regular nodes of one cluster only come
+    // last, from Gi on, and take their update in the cluster kernel.  cl_ok:
+    // that kernel's preconditions hold (nodal or no C-PML, elastic).
+    bool cl_ok = false;
+    int64_t Gi = 0;
+    std::vector<int32_t> cl_begin;
+    gfx::DevBuf<gfx::dev::ClusterHead> cl_head;
+    gfx::DevBuf<uint16_t> cl_ent;
+    gfx::DevBuf<int32_t> cl_bdst;
     std::vector<gfx::FieldSource> sources;
     gfx::DevBuf<int4> src_ent;
     gfx::DevBuf<float> src_w, stf;
@@ -108,10 +131,10 @@ struct gfx_solver {
     // cells (solver numbering) and weights of the last injection
     int stage = 0;
     bool stage_zeroed = false;
-    // GATHER: R (not the slot sums of Rl) holds the last step's assembled
-    // residual, as after a step driven stage by stage (the exchange may have
-    // changed it after the scatter)
-    bool r_in_R = false;
+    // GATHER: what holds the last step's residual: the entries of one of the
+    // plans, or R itself, as after a step driven stage by stage (the exchange
+    // may have changed it after the scatter)
+    int r_src = gfx::R_ASSEMBLED;
     gfx::DevBuf<int32_t> inj_cells;
     gfx::DevBuf<float> inj_w;
     // timing
@@ -274,12 +297,27 @@ std::vector<char> cpml_rigid_nodes(const gfx_solver_desc& d, int E, int G) {
     return rigid;
 }
 
+// The element stage runs the cluster kernel: GATHER assembly and the wavefront form.
+bool uses_clusters(const gfx_solver& S) {
+    return S.assembly == GFX_ASSEMBLY_GATHER && S.cl_ok && S.kernel == GFX_ELEMENT_WAVE;
+}
+
+int active_plan(const gfx_solver& S) {
+    if (S.assembly != GFX_ASSEMBLY_GATHER) return R_ASSEMBLED;
+    return uses_clusters(S) ? R_CLUSTERS : R_POINTS;
+}
+
+const GatherPlan& plan_of(const gfx_solver& S, int r_src) {
+    return r_src == R_CLUSTERS ? S.by_cluster : S.by_point;
+}
+
 void init_state(gfx_solver& S) {
     S.U.zero(S.stream);
     S.W.zero(S.stream);
     S.R.zero(S.stream);
     S.Aacc.zero(S.stream);
-    S.Rl.zero(S.stream);
+    S.by_point.Rl.zero(S.stream);
+    S.by_cluster.Rl.zero(S.stream);
     S.pmem.zero(S.stream);
     S.pnew.zero(S.stream);
     S.zeta.zero(S.stream);
@@ -290,7 +328,7 @@ void init_state(gfx_solver& S) {
     S.n_snap = 0;
     S.stage = 0;
     S.stage_zeroed = false;
-    S.r_in_R = false;
+    S.r_src = R_ASSEMBLED;  // R is zero
 }
 
 // Launchers.  DIAG selects the axis-aligned geometry form for a range whose
@@ -444,6 +482,16 @@ void launch_cpml(gfx_solver& S, const dev::ElemArgs& a, int ax, int b, int n) {
     }
 }
 
+template <int OUT>
+void launch_clusters(gfx_solver& S, const dev::ElemArgs& a, const ElemRange& rg) {
+    const int grid = rg.ce - rg.cb;
+    if (grid == 0) return;
+    if (rg.diag)
+        dev::k_cluster<true, OUT><<<grid, dev::CLUSTER_THREADS, 0, S.stream>>>(a, rg.cb);
+    else
+        dev::k_cluster<false, OUT><<<grid, dev::CLUSTER_THREADS, 0, S.stream>>>(a, rg.cb);
+}
+
 void launch_element(gfx_solver& S, const dev::ElemArgs& a, const ElemRange& rg) {
     const int b = rg.b, n = rg.e - rg.b;
     if (S.n_sls > 0 && !rg.pml) {  // shear attenuation: one kernel form for every range
@@ -466,6 +514,8 @@ void launch_element(gfx_solver& S, const dev::ElemArgs& a, const ElemRange& rg) 
         }
     } else if (ref_elem_pml(S)) {
         launch_element_p<true, false>(S, a, b, n);  // element-local C-PML: block kernel, general form
+    } else if (uses_clusters(S)) {
+        launch_clusters<dev::CL_FUSED>(S, a, rg);
     } else if (rg.diag) {
         launch_element_d<true>(S, a, b, n);
     } else {
@@ -499,7 +549,20 @@ void launch_node_regular(gfx_solver& S, const dev::NodeArgs& na, int grid) {
         launch_node_regular_t<false>(S, na, grid);
 }
 
+// Fields per workgroup of the cluster form's node launch: all of them where the
+// nodes alone fill the device's 2,048 workgroup places eight times over, fewer
+// where they do not (not below four: the C-PML coefficients, 56 bytes per node,
+// are read again for every chunk).  24 fields on 23,328 elements: 482 us in six
+// chunks against 578 us for the two launches over all fields they replace.
+constexpr int NODE_BLOCKS = 16384;
+int node_chunk(int blocks, int nf) {
+    const int want = std::max(1, NODE_BLOCKS / std::max(blocks, 1));  // field chunks
+    const int chunk = std::max((nf + want - 1) / want, std::min(nf, 4));
+    return chunk;
+}
+
 struct StepArgs {
+    bool clusters = false;  // cluster form: one launch for all nodes
     dev::ElemArgs ea{};
     dev::NodeArgs na{};
     dev::RecArgs ra{};
@@ -509,8 +572,16 @@ struct StepArgs {
 };
 constexpr int REPB = 2;  // recording cells per workgroup
 
-StepArgs make_step_args(gfx_solver& S) {
+void require_plan(gfx_solver& S, int which);
+
+// Arguments of one step; points = true: with the residuals left per element
+// point whatever the element kernel (the per-stage entry points).
+StepArgs make_step_args(gfx_solver& S, bool points = false) {
     StepArgs a;
+    const bool clusters = !points && uses_clusters(S);
+    a.clusters = clusters;
+    require_plan(S, S.assembly != GFX_ASSEMBLY_GATHER ? R_ASSEMBLED : clusters ? R_CLUSTERS : R_POINTS);
+    const GatherPlan& gp = clusters ? S.by_cluster : S.by_point;
     const double theta = 1.0 / 8.0;  // pml.cpp:35, coefficients pml.cpp:63-64
     const float c1 = float((1.0 - 2.0 * theta) * 0.5 * S.dt);
     const float c2 = float((1.0 - theta) * 0.5 * S.dt * S.dt);
@@ -525,9 +596,15 @@ StepArgs make_step_args(gfx_solver& S) {
     ea.fstride = S.fstride;
     ea.U = S.U.p;
     ea.R = S.R.p;
-    ea.Rl = S.Rl.p;
-    ea.rdst = S.rdst.p;
-    ea.PR = S.PR;
+    ea.Rl = gp.Rl.p;
+    ea.rdst = gp.rdst.p;
+    ea.PR = gp.PR;
+    ea.cl_head = S.cl_head.p;
+    ea.cl_ent = S.cl_ent.p;
+    ea.cl_bdst = S.cl_bdst.p;
+    ea.minv = S.minv.p;
+    ea.Uw = S.U.p;
+    ea.Ww = S.W.p;
     ea.W = S.W.p;
     ea.Aacc = S.Aacc.p;
     ea.astride = S.astride;
@@ -559,16 +636,16 @@ StepArgs make_step_args(gfx_solver& S) {
     na.G = S.G;
     na.Ga = S.Ga;
     na.Gpml = S.Gpml;
-    na.G4 = S.G4;
+    na.G4 = clusters ? S.Gi : S.G4;  // the nodes from Gi on are updated by the cluster kernel
     na.P = int64_t(S.E) * NP;
     na.nf = S.nf;
     na.fstride = S.fstride;
     na.astride = S.astride;
     na.gather = (S.assembly == GFX_ASSEMBLY_GATHER) ? 1 : 0;
-    na.Rl = S.Rl.p;
-    na.PR = S.PR;
-    na.off = S.goff.p;
-    na.pts = S.gpts.p;
+    na.Rl = gp.Rl.p;
+    na.PR = gp.PR;
+    na.off = gp.off.p;
+    na.pts = gp.pts.p;
     na.minv = S.minv.p;
     na.damp = S.has_cpml ? nullptr : S.damp.p;
     na.U = S.U.p;
@@ -585,8 +662,13 @@ StepArgs make_step_args(gfx_solver& S) {
     na.c2 = c2;
     na.dt = float(S.dt);
     const int fg = S.node_fg;
-    a.spec_grid = int((S.Ga + 256 / fg - 1) / (256 / fg));
-    a.reg_grid = int(((S.G4 - S.Ga) / 4 + 256 / fg - 1) / (256 / fg));
+    if (clusters) {  // one node per lane
+        a.spec_grid = int((S.Ga + 255) / 256);
+        a.reg_grid = int((na.G4 - S.Ga + 255) / 256);
+    } else {
+        a.spec_grid = int((S.Ga + 256 / fg - 1) / (256 / fg));
+        a.reg_grid = int(((na.G4 - S.Ga) / 4 + 256 / fg - 1) / (256 / fg));
+    }
     a.r4 = int64_t(S.nf) * S.fstride / 4;
     a.zero_grid = int((a.r4 + 255) / 256);
 
@@ -632,14 +714,32 @@ void enqueue_step(gfx_solver& S, const StepArgs& a, bool record, hipEvent_t* ev)
     if (ev && pml_tail == nr) GFX_HIP(hipEventRecord(ev[0], S.stream));
     GFX_HIP(hipGetLastError());
     if (ev) GFX_HIP(hipEventRecord(ev[1], S.stream));
-    if (a.spec_grid > 0) launch_node_special(S, a.na, a.spec_grid);
+    const bool rec = record && a.recording && a.rec_grid > 0;
+    const bool split = ev != nullptr;  // per-kernel timing: special and regular nodes apart
+    int* const close = a.clusters && !rec ? S.ctr.p : nullptr;  // the node launch closes the step
+    bool closed = false;
+    auto nodes = [&](bool special, bool regular) {
+        if (!a.clusters) {
+            if (special && a.spec_grid > 0) launch_node_special(S, a.na, a.spec_grid);
+            if (regular && a.reg_grid > 0) launch_node_regular(S, a.na, a.reg_grid);
+            return;
+        }
+        const int sg = special ? a.spec_grid : 0, rg = regular ? a.reg_grid : 0;
+        if (sg + rg == 0) return;
+        const int chunk = node_chunk(a.spec_grid + a.reg_grid, S.nf);
+        const dim3 grid(unsigned(sg + rg), unsigned((S.nf + chunk - 1) / chunk));
+        int* const c = regular ? close : nullptr;
+        dev::k_cluster_nodes<<<grid, 256, 0, S.stream>>>(a.na, sg, chunk, c, S.stride);
+        closed = closed || c;
+    };
+    if (!split) nodes(true, true);
+    else nodes(true, false);
     if (ev) GFX_HIP(hipEventRecord(ev[2], S.stream));
-    if (a.reg_grid > 0) launch_node_regular(S, a.na, a.reg_grid);
+    if (split) nodes(false, true);
     GFX_HIP(hipGetLastError());
     if (ev) GFX_HIP(hipEventRecord(ev[3], S.stream));
-    if (record && a.recording && a.rec_grid > 0)
-        dev::k_record<REPB><<<a.rec_grid, a.rec_threads, 0, S.stream>>>(a.ra);
-    dev::k_advance<<<1, 64, 0, S.stream>>>(S.ctr.p, S.stride);
+    if (rec) dev::k_record<REPB><<<a.rec_grid, a.rec_threads, 0, S.stream>>>(a.ra);
+    if (!closed) dev::k_advance<<<1, 64, 0, S.stream>>>(S.ctr.p, S.stride);
     GFX_HIP(hipGetLastError());
     if (ev) GFX_HIP(hipEventRecord(ev[4], S.stream));
 }
@@ -670,7 +770,7 @@ void ensure_graph(gfx_solver& S) {
 }
 
 void run_steps(gfx_solver& S, int nsteps) {
-    if (nsteps > 0) S.r_in_R = false;
+    if (nsteps > 0) S.r_src = active_plan(S);
     if (S.use_graph && !S.timing) {
         ensure_graph(S);
         for (int t = 0; t < nsteps; ++t) {
@@ -774,6 +874,207 @@ struct DeviceWork {
     }
 };
 
+// Clusters of the solver elements [b, e), appended to `begin`: up to CE elements
+// whose keys differ in the lowest three bits only (a 2 x 2 x 2 block of the
+// element lattice), blocks with fewer joined while they fit.  Where that leaves
+// more than a fifth of the places empty (thin or unstructured meshes, no
+// centroids), runs of CE elements along the curve instead.
+void cluster_range(const std::vector<uint64_t>& key, const std::vector<int32_t>& elem_of_int, int b, int e, bool lattice,
+                   std::vector<int32_t>& begin) {
+    const size_t at = begin.size();
+    if (lattice) {
+        int cb = b;  // first element of the open cluster
+        for (int i = b; i < e;) {
+            int j = i + 1;
+            while (j < e && j - i < dev::CE && (key[elem_of_int[j]] >> 3) == (key[elem_of_int[i]] >> 3)) ++j;
+            if (i > cb && j - cb > dev::CE) {
+                begin.push_back(cb);
+                cb = i;
+            }
+            i = j;
+        }
+        if (e > cb) begin.push_back(cb);
+        if (5 * int64_t(e - b) >= 4 * int64_t(dev::CE) * int64_t(begin.size() - at)) return;
+        begin.resize(at);
+    }
+    for (int i = b; i < e; i += dev::CE) begin.push_back(i);
+}
+
+struct HostPlan {
+    int64_t PR = 0;
+    std::vector<int32_t> off, pts, xoff, xpts, rdst;
+    std::vector<uint8_t> new_cluster;
+    std::vector<dev::ClusterHead> head;
+    std::vector<uint16_t> ent;
+    std::vector<int32_t> bdst;
+};
+
+// Device slot lists: every slot but the node's first (read at the node id).
+void device_slots(int64_t G4, HostPlan& h) {
+    h.xoff.assign(G4 + 1, 0);
+    h.xpts.reserve(h.pts.size());
+    for (int64_t n = 0; n < G4; ++n) {
+        for (int32_t q = h.off[n] + 1; q < h.off[n + 1]; ++q) h.xpts.push_back(h.pts[q]);
+        h.xoff[n + 1] = int32_t(h.xpts.size());
+    }
+}
+
+// Residual entries per element point: each node owns the contiguous slots
+// [off[n], off[n+1]), filled with its element points in increasing solver order
+// (the fixed summation order).  A node's first point (lowest solver order) has
+// its entry at the node's own index, the other points after the nodes, element
+// by element, ordered by node id inside each element (the points a node-kernel
+// workgroup gathers from one element then sit together).  Entry positions do
+// not change the sums: each node adds its slots in increasing solver point order.
+HostPlan point_plan(const gfx_solver& S, const std::vector<uint32_t>& hib) {
+    HostPlan h;
+    const int64_t E = S.E, P = E * NP, G4 = S.G4;
+    std::vector<int32_t>&off = h.off, &pts = h.pts, &rdst = h.rdst;
+    off.assign(G4 + 1, 0);
+    pts.resize(P);
+    for (int64_t q = 0; q < P; ++q) ++off[hib[q] + 1];
+    for (int64_t n = 0; n < G4; ++n) off[n + 1] += off[n];
+    require(off[G4] == P, "internal: gather slots do not cover every element point");
+    std::vector<int32_t> fill(off.begin(), off.end() - 1);
+    for (int64_t q = 0; q < P; ++q) pts[fill[hib[q]]++] = int32_t(q);
+    if (S.cl_ok) {  // slots (without each node's first) where the next cluster's points begin
+        std::vector<int32_t> cl(E, 0);
+        for (int c = 0; c + 1 < int(S.cl_begin.size()); ++c)
+            for (int e = S.cl_begin[c]; e < S.cl_begin[c + 1]; ++e) cl[e] = c;
+        for (int64_t n = 0; n < G4; ++n)
+            for (int32_t q = off[n] + 1; q < off[n + 1]; ++q)
+                h.new_cluster.push_back(cl[pts[q] / NP] != cl[pts[q - 1] / NP]);
+    }
+    rdst.assign(P, -1);
+    for (int64_t n = 0; n < G4; ++n)
+        if (off[n + 1] > off[n]) rdst[pts[off[n]]] = int32_t(n);
+    int64_t k = G4;
+    for (int64_t e = 0; e < E; ++e) {
+        int64_t rest[NP];
+        int nr = 0;
+        for (int p = 0; p < NP; ++p)
+            if (rdst[e * NP + p] < 0) rest[nr++] = e * NP + p;
+        std::sort(rest, rest + nr, [&](int64_t a, int64_t b) { return hib[a] < hib[b] || (hib[a] == hib[b] && a < b); });
+        for (int q = 0; q < nr; ++q) rdst[rest[q]] = int32_t(k++);
+    }
+    require(k == G4 + P - S.G, "internal: residual entries do not match the point count");
+    h.PR = (k + 3) / 4 * 4;  // 16-byte aligned field stride
+    for (int64_t q = 0; q < P; ++q) pts[q] = rdst[pts[q]];
+    device_slots(G4, h);
+    return h;
+}
+
+// Residual entries per cluster and node, and the cluster kernel's tables.  A
+// node sums its clusters in increasing order; the first has its entry at the
+// node id, the others after the nodes, cluster by cluster in list order.
+HostPlan cluster_plan(const gfx_solver& S, const std::vector<uint32_t>& hib) {
+    HostPlan h;
+    const int nc = int(S.cl_begin.size()) - 1;
+    const int64_t P = int64_t(S.E) * NP, G4 = S.G4;
+    std::vector<int32_t> first(G4, -1);  // lowest cluster of each node
+    for (int c = 0; c < nc; ++c)
+        for (int64_t q = int64_t(S.cl_begin[c]) * NP; q < int64_t(S.cl_begin[c + 1]) * NP; ++q)
+            if (first[hib[q]] < 0) first[hib[q]] = c;
+    h.head.assign(nc, dev::ClusterHead{});
+    h.ent.resize(P);
+    std::vector<std::vector<int32_t>> shared(nc);  // the nodes of each cluster's second list
+    std::atomic<bool> bad{false};
+    parallel_for(nc, [&](int64_t c) {
+        dev::ClusterHead& H = h.head[c];
+        H.e0 = S.cl_begin[c];
+        H.ne = S.cl_begin[c + 1] - H.e0;
+        const int np = H.ne * NP;
+        const int64_t q0 = int64_t(H.e0) * NP;
+        std::vector<uint64_t> at(np);  // (node, point), by node then point
+        for (int q = 0; q < np; ++q) at[q] = (uint64_t(hib[q0 + q]) << 16) | uint64_t(q);
+        std::sort(at.begin(), at.end());
+        struct Node {
+            int32_t id, b, n;
+        };
+        std::vector<Node> list[2];
+        for (int q = 0; q < np;) {
+            int e = q + 1;
+            while (e < np && (at[e] >> 16) == (at[q] >> 16)) ++e;
+            const int32_t id = int32_t(at[q] >> 16);
+            list[id >= S.Gi ? 0 : 1].push_back({id, q, e - q});
+            q = e;
+        }
+        uint16_t* out = h.ent.data() + q0;
+        for (int k = 0; k < 2; ++k) {
+            std::stable_sort(list[k].begin(), list[k].end(), [](const Node& x, const Node& y) { return x.n > y.n; });
+            int cnt[dev::CE] = {};
+            for (const Node& x : list[k]) {
+                if (x.n > dev::CE) bad = true;
+                for (int m = 0; m < std::min<int>(x.n, dev::CE); ++m) ++cnt[m];
+            }
+            if (bad) return;
+            for (int m = 0; m < dev::CE; ++m) H.cnt[m] |= uint32_t(cnt[m]) << (16 * k);
+            for (int m = 0; m < dev::CE; ++m)
+                for (int t = 0; t < cnt[m]; ++t) *out++ = uint16_t(at[list[k][t].b + m] & 0xffff);
+        }
+        if (out != h.ent.data() + q0 + np) bad = true;
+        H.ibase = list[0].empty() ? 0 : list[0][0].id;
+        for (size_t t = 0; t < list[0].size(); ++t)
+            if (list[0][t].id != H.ibase + int32_t(t)) bad = true;
+        for (const Node& x : list[1]) shared[c].push_back(x.id);
+    });
+    require(!bad, "internal: cluster lists do not match the node numbering");
+    std::vector<int32_t>&off = h.off, &pts = h.pts;
+    off.assign(G4 + 1, 0);
+    for (int64_t n = 0; n < G4; ++n) off[n + 1] = n >= S.Gi && first[n] >= 0;
+    int64_t nb = 0;
+    for (int c = 0; c < nc; ++c) {
+        h.head[c].boff = int32_t(nb);
+        nb += int64_t(shared[c].size());
+        for (int32_t n : shared[c]) ++off[n + 1];
+    }
+    for (int64_t n = 0; n < G4; ++n) off[n + 1] += off[n];
+    pts.resize(off[G4]);
+    h.bdst.resize(nb);
+    std::vector<int32_t> fill(off.begin(), off.end() - 1);
+    for (int64_t n = S.Gi; n < G4; ++n)
+        if (first[n] >= 0) pts[fill[n]++] = int32_t(n);
+    int64_t k = G4;
+    for (int c = 0; c < nc; ++c)
+        for (size_t t = 0; t < shared[c].size(); ++t) {
+            const int32_t n = shared[c][t];
+            const int32_t dst = first[n] == c ? n : int32_t(k++);
+            h.bdst[h.head[c].boff + t] = dst;
+            pts[fill[n]++] = dst;
+        }
+    h.PR = (k + 3) / 4 * 4;  // 16-byte aligned field stride
+    device_slots(G4, h);
+    return h;
+}
+
+// Builds the residual entries a launch needs if they are not there yet (a
+// solver switched to another element kernel, or driven stage by stage).
+void require_plan(gfx_solver& S, int which) {
+    if (which == R_ASSEMBLED) return;
+    GatherPlan& gp = which == R_CLUSTERS ? S.by_cluster : S.by_point;
+    if (gp.ready) return;
+    std::vector<uint32_t> hib(size_t(S.E) * NP);
+    GFX_HIP(hipStreamSynchronize(S.stream));
+    GFX_HIP(hipMemcpy(hib.data(), S.ibool.p, hib.size() * 4, hipMemcpyDeviceToHost));
+    HostPlan h = which == R_CLUSTERS ? cluster_plan(S, hib) : point_plan(S, hib);
+    gp.PR = h.PR;
+    gp.off.upload(h.xoff);
+    gp.pts.upload(h.xpts);
+    gp.rdst.upload(h.rdst);
+    gp.new_cluster.upload(h.new_cluster);
+    if (which == R_CLUSTERS) {
+        S.cl_head.upload(h.head);
+        S.cl_ent.upload(h.ent);
+        S.cl_bdst.upload(h.bdst);
+    }
+    gp.Rl.alloc(size_t(S.nf) * gp.PR * 3);
+    gp.Rl.zero(S.stream);
+    GFX_HIP(hipStreamSynchronize(S.stream));
+    gp.off_host = std::move(h.off);
+    gp.pts_host = std::move(h.pts);
+    gp.ready = true;
+}
+
 void create(const gfx_solver_desc& d, gfx_solver& S) {
     require(d.ngll == 5, "the device solver supports NGLL = 5 (polynomial order 4) only");
     require(d.n_elem > 0 && d.n_rank_node > 0, "empty mesh");
@@ -841,6 +1142,31 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
             key[e] = m;
         }
     }
+    // The cluster kernel (GATHER assembly, elastic, without the complete C-PML)
+    // works on elements that lie together: the curve then runs over the lattice of element-sized cells instead (the element
+    // size per axis from grad xi at the element centres), so that its lowest
+    // three bits number the elements of a 2 x 2 x 2 block
+    const bool by_cluster = S.assembly == GFX_ASSEMBLY_GATHER && d.n_sls == 0 && !S.cpml_complete;
+    if (by_cluster && d.elem_centroid) {
+        double lo[3] = {1e300, 1e300, 1e300}, h[3] = {0, 0, 0};
+        for (int e = 0; e < E; ++e)
+            for (int c = 0; c < 3; ++c) {
+                const double* x = d.dxi_dx + (int64_t(e) * NP + NP / 2) * 9 + c * 3;
+                lo[c] = std::min(lo[c], d.elem_centroid[e * 3 + c]);
+                h[c] += 2.0 / std::sqrt(x[0] * x[0] + x[1] * x[1] + x[2] * x[2]) / E;
+            }
+        if (std::isfinite(h[0]) && std::isfinite(h[1]) && std::isfinite(h[2]))
+            for (int e = 0; e < E; ++e) {
+                uint64_t q[3], m = 0;
+                for (int c = 0; c < 3; ++c) {
+                    const double t = std::floor((d.elem_centroid[e * 3 + c] - lo[c]) / h[c] + 0.5);
+                    q[c] = uint64_t(std::min(std::max(t, 0.0), 2097151.0));
+                }
+                for (int b = 20; b >= 0; --b)
+                    for (int c = 2; c >= 0; --c) m = (m << 1) | ((q[c] >> b) & 1ULL);
+                key[e] = m;
+            }
+    }
     // axis-aligned elements: dxi_a/dx_m = 0 for a != m at every point, up to FP64
     // round-off of the input (|off-diagonal| <= 1e-12 x the largest diagonal
     // entry); they run the diagonal geometry form of the element kernels
@@ -888,10 +1214,16 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
             if (i == E || col[elem_of_int[i]] != col[e0] || pml_el[elem_of_int[i]] != pml_el[e0] ||
                 pml_ax[elem_of_int[i]] != pml_ax[e0] || diag_el[elem_of_int[i]] != diag_el[e0]) {
                 const bool pml = pml_el[e0] != 0;
-                S.ranges.push_back({b, i, diag_el[e0] != 0 && !pml, pml, int(pml_ax[e0])});
+                S.ranges.push_back({b, i, diag_el[e0] != 0 && !pml, pml, int(pml_ax[e0]), 0, 0});
+                if (by_cluster) {
+                    S.ranges.back().cb = int(S.cl_begin.size());
+                    cluster_range(key, elem_of_int, b, i, d.elem_centroid != nullptr, S.cl_begin);
+                    S.ranges.back().ce = int(S.cl_begin.size());
+                }
                 b = i;
             }
         }
+        if (by_cluster) S.cl_begin.push_back(E);
         S.n_colors = S.assembly == GFX_ASSEMBLY_COLORED ? (*std::max_element(col.begin(), col.end()) + 1) : 1;
         S.n_diag = 0;
         for (const ElemRange& rg : S.ranges)
@@ -968,15 +1300,54 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
             }
         }
     }
+    // regular nodes of one cluster only form a class of their own (-1) behind the
+    // other regular nodes
+    if (by_cluster) {
+        std::vector<int32_t> seen(G, -1), in_elem(G, -1);
+        std::vector<char> shared(G, 0);
+        S.cl_ok = true;
+        for (int c = 0; c + 1 < int(S.cl_begin.size()); ++c)
+            for (int i = S.cl_begin[c]; i < S.cl_begin[c + 1]; ++i)
+                for (int p = 0; p < NP; ++p) {
+                    const int g = d.ibool[int64_t(elem_of_int[i]) * NP + p];
+                    if (in_elem[g] == i) S.cl_ok = false;  // a node twice in one element: one entry per point only
+                    in_elem[g] = i;
+                    if (seen[g] >= 0 && seen[g] != c) shared[g] = 1;
+                    seen[g] = c;
+                }
+        for (int g = 0; g < G; ++g)
+            if (cls[g] == 0 && seen[g] >= 0 && !shared[g]) cls[g] = -1;
+    }
     // numbering: C-PML nodes, other special nodes, regular nodes; first touch
     // in solver element order inside each class; C-PML nodes grouped by their
-    // direction mask (first touch inside a group), so wavefronts share a mask
+    // direction mask (first touch inside a group), so wavefronts share a mask;
+    // with clusters: cluster by cluster, the nodes of most of the cluster's elements
+    // first (the order of the cluster kernel's lists)
     // (-1 = not yet seen, -2 = queued in this class, >= 0 = numbered)
     S.node_new_of_old.assign(G, -1);
     int next = 0;
-    for (int pass = 2; pass >= 0; --pass) {
+    for (int pass = 2; pass >= -1; --pass) {
         std::vector<int> order;
+        if (by_cluster) {
+            std::vector<uint8_t> held(G, 0);  // elements of the cluster that hold the node
+            for (int c = 0; c + 1 < int(S.cl_begin.size()); ++c) {
+                const size_t b = order.size();
+                for (int i = S.cl_begin[c]; i < S.cl_begin[c + 1]; ++i)
+                    for (int p = 0; p < NP; ++p) {
+                        const int g = d.ibool[int64_t(elem_of_int[i]) * NP + p];
+                        if (cls[g] != pass) continue;
+                        if (S.node_new_of_old[g] == -1) {
+                            S.node_new_of_old[g] = -2;
+                            held[g] = 0;
+                            order.push_back(g);
+                        }
+                        ++held[g];
+                    }
+                std::stable_sort(order.begin() + b, order.end(), [&](int x, int y) { return held[x] > held[y]; });
+            }
+        }
         for (int i = 0; i < E; ++i) {
+            if (by_cluster) break;
             const int64_t e = elem_of_int[i];
             for (int p = 0; p < NP; ++p) {
                 const int g = d.ibool[e * NP + p];
@@ -996,6 +1367,7 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
                              [&](int a, int b) { return pm_old[a] < pm_old[b]; });
         for (int g : order) S.node_new_of_old[g] = next++;
         if (pass == 2) S.Gpml = next;
+        if (pass == 0) S.Gi = next;
     }
     // every node numbered exactly once: the numbering is a permutation of [0, G)
     require(next == G, "internal: node numbering is not a permutation");
@@ -1008,9 +1380,10 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
         }
     }
     int64_t n_special = 0;
-    for (int g = 0; g < G; ++g) n_special += cls[g] ? 1 : 0;
+    for (int g = 0; g < G; ++g) n_special += cls[g] > 0 ? 1 : 0;
     S.Ga = std::min<int64_t>(((n_special + 3) / 4) * 4, ((int64_t(G) + 3) / 4) * 4);
     S.G4 = ((int64_t(G) + 3) / 4) * 4;
+    S.Gi = std::min<int64_t>((S.Gi + 3) / 4 * 4, S.G4);
 
     // ---- geometry / material, FP64 -> FP32 SoA, first-touch flags ----
     std::vector<float> hG(size_t(9) * P), hlam(P), hmu(P);
@@ -1250,49 +1623,28 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
     dv.alloc(S.R, fs);
     dv.alloc(S.Aacc, size_t(S.astride) * S.nf);
     if (S.assembly == GFX_ASSEMBLY_GATHER) {
-        // each node owns the contiguous slots [off[n], off[n+1]), filled with its
-        // element points in increasing solver order (the fixed summation order);
-        // the element kernels store each point's residual at the point itself
-        std::vector<int32_t> off(S.G4 + 1, 0), pts(P);
-        for (int64_t q = 0; q < P; ++q) ++off[hib[q] + 1];
-        for (int64_t n = 0; n < S.G4; ++n) off[n + 1] += off[n];
-        require(off[S.G4] == P, "internal: gather slots do not cover every element point");
-        std::vector<int32_t> fill(off.begin(), off.end() - 1);
-        for (int64_t q = 0; q < P; ++q) pts[fill[hib[q]]++] = int32_t(q);
-        // residual entry of each point: a node's first point (lowest solver order) at
-        // the node's own index, the other points after the nodes, element by element,
-        // ordered by node id inside each element (the points a node-kernel workgroup
-        // gathers from one element then sit together); a node's slots list entries,
-        // the first one being the node itself.  Entry positions do not change the
-        // sums: each node adds its slots in increasing solver point order.
-        std::vector<int32_t> rdst(P, -1);
-        for (int64_t n = 0; n < S.G4; ++n)
-            if (off[n + 1] > off[n]) rdst[pts[off[n]]] = int32_t(n);
-        int64_t k = S.G4;
-        for (int64_t e = 0; e < E; ++e) {
-            int64_t rest[NP];
-            int nr = 0;
-            for (int p = 0; p < NP; ++p)
-                if (rdst[e * NP + p] < 0) rest[nr++] = e * NP + p;
-            std::sort(rest, rest + nr, [&](int64_t a, int64_t b) { return hib[a] < hib[b] || (hib[a] == hib[b] && a < b); });
-            for (int q = 0; q < nr; ++q) rdst[rest[q]] = int32_t(k++);
-        }
-        require(k == S.G4 + P - S.G, "internal: residual entries do not match the point count");
-        S.PR = (k + 3) / 4 * 4;  // 16-byte aligned field stride
-        for (int64_t q = 0; q < P; ++q) pts[q] = rdst[pts[q]];
-        // device slot lists: every point but the node's first (read at the node id)
-        std::vector<int32_t> xoff(S.G4 + 1, 0), xpts;
-        xpts.reserve(size_t(P - S.G));
-        for (int64_t n = 0; n < S.G4; ++n) {
-            for (int32_t q = off[n] + 1; q < off[n + 1]; ++q) xpts.push_back(pts[q]);
-            xoff[n + 1] = int32_t(xpts.size());
-        }
-        S.goff_host = off;
-        S.gpts_host = pts;
-        dv.upload(S.goff, std::move(xoff));
-        dv.upload(S.gpts, std::move(xpts));
-        dv.upload(S.rdst, std::move(rdst));
-        dv.alloc(S.Rl, size_t(S.nf) * S.PR * 3);
+        // (the cluster kernels address a field's nodes and entries, at most P + 4, by 32-bit byte offsets)
+        S.cl_ok = S.cl_ok && (!S.has_cpml || S.pml_nodal) && (P + 8) * 12 < (int64_t(1) << 32);
+        // the first cluster or point of every node holds its entry at the node id
+        std::vector<char> touched(G, 0);
+        for (int64_t q = 0; q < P; ++q) touched[hib[q]] = 1;
+        require(std::find(touched.begin(), touched.end(), 0) == touched.end(),
+                "internal: residual entries do not match the point count");
+        // the plan of the element kernel in use now; another form's is built when it is first run
+        GatherPlan& gp = uses_clusters(S) ? S.by_cluster : S.by_point;
+        HostPlan h = uses_clusters(S) ? cluster_plan(S, hib) : point_plan(S, hib);
+        gp.PR = h.PR;
+        gp.off_host = std::move(h.off);
+        gp.pts_host = std::move(h.pts);
+        dv.upload(gp.off, std::move(h.xoff));
+        dv.upload(gp.pts, std::move(h.xpts));
+        dv.upload(gp.rdst, std::move(h.rdst));
+        dv.upload(gp.new_cluster, std::move(h.new_cluster));
+        dv.upload(S.cl_head, std::move(h.head));
+        dv.upload(S.cl_ent, std::move(h.ent));
+        dv.upload(S.cl_bdst, std::move(h.bdst));
+        dv.alloc(gp.Rl, size_t(S.nf) * gp.PR * 3);
+        gp.ready = true;
     }
     std::vector<uint32_t>().swap(hib);
 
@@ -1455,12 +1807,13 @@ extern "C" gfx_status gfx_solver_get_state(const gfx_solver* s, int field, doubl
         const std::vector<float> hU = fetch(s, s->U.p + int64_t(field) * s->fstride, n3);
         const std::vector<float> hW = fetch(s, s->W.p + int64_t(field) * s->fstride, n3);
         std::vector<float> hR;
-        if (s->assembly == GFX_ASSEMBLY_GATHER && !s->r_in_R) {
+        if (s->r_src != R_ASSEMBLED) {
             // assembled r of the last step: fixed-order sum of the node's slots, as the
             // node kernels form it
-            const std::vector<float> hl = fetch(s, s->Rl.p + int64_t(field) * s->PR * 3, size_t(s->PR) * 3);
-            const std::vector<int32_t>& off = s->goff_host;
-            const std::vector<int32_t>& pts = s->gpts_host;
+            const GatherPlan& gp = plan_of(*s, s->r_src);
+            const std::vector<float> hl = fetch(s, gp.Rl.p + int64_t(field) * gp.PR * 3, size_t(gp.PR) * 3);
+            const std::vector<int32_t>& off = gp.off_host;
+            const std::vector<int32_t>& pts = gp.pts_host;
             hR.assign(size_t(s->G4) * 3, 0.f);
             for (int64_t n = 0; n < s->G; ++n)
                 for (int q = off[n]; q < off[n + 1]; ++q)
@@ -1521,14 +1874,11 @@ extern "C" gfx_status gfx_solver_set_state(gfx_solver* s, int field, const doubl
         if (!hA.empty())
             GFX_HIP(hipMemcpy(s->Aacc.p + int64_t(field) * s->astride, hA.data(), hA.size() * 4,
                               hipMemcpyHostToDevice));
-        if (s->assembly == GFX_ASSEMBLY_GATHER) {  // r = m a at the first entry of each node
-            std::vector<float> hl(size_t(s->PR) * 3, 0.f);
-            for (int64_t n = 0; n < s->G; ++n)
-                if (s->goff_host[n + 1] > s->goff_host[n])
-                    for (int c = 0; c < 3; ++c)
-                        hl[int64_t(s->gpts_host[s->goff_host[n]]) * 3 + c] = hR[n * 3 + c];
-            GFX_HIP(hipMemcpy(s->Rl.p + int64_t(field) * s->PR * 3, hl.data(), hl.size() * 4,
-                              hipMemcpyHostToDevice));
+        if (s->r_src != R_ASSEMBLED) {  // r = m a at the first entry of each node (the node's own index)
+            const GatherPlan& gp = plan_of(*s, s->r_src);
+            std::vector<float> hl(size_t(gp.PR) * 3, 0.f);
+            std::copy(hR.begin(), hR.end(), hl.begin());
+            GFX_HIP(hipMemcpy(gp.Rl.p + int64_t(field) * gp.PR * 3, hl.data(), hl.size() * 4, hipMemcpyHostToDevice));
         }
     });
 }
@@ -1627,9 +1977,14 @@ extern "C" gfx_status gfx_step_element_residual(gfx_solver* s, int ngll, int n_e
         require(n_elem == s->E, "n_elem differs from the solver's element count");
         require(s->stage_zeroed || s->assembly != GFX_ASSEMBLY_ATOMIC,
                 "ATOMIC assembly adds into the residual: call gfx_step_zero_residual first");
-        StepArgs a = make_step_args(*s);
+        StepArgs a = make_step_args(*s, true);
         a.ea.nstf = 0;  // sources come from gfx_step_source_injection
-        for (const auto& rg : s->ranges) launch_element(*s, a.ea, rg);
+        for (const auto& rg : s->ranges) {
+            if (uses_clusters(*s))
+                launch_clusters<dev::CL_POINTS>(*s, a.ea, rg);
+            else
+                launch_element(*s, a.ea, rg);
+        }
         GFX_HIP(hipGetLastError());
         s->stage = STAGE_ELEMENT;
     });
@@ -1666,9 +2021,10 @@ extern "C" gfx_status gfx_step_source_injection(gfx_solver* s, int field, int di
         if (s->inj_w.n < w.size()) s->inj_w.alloc(w.size());
         GFX_HIP(hipMemcpy(s->inj_cells.p, cells.data(), cells.size() * 4, hipMemcpyHostToDevice));
         GFX_HIP(hipMemcpy(s->inj_w.p, w.data(), w.size() * 4, hipMemcpyHostToDevice));
-        dev::k_inject<<<1, 128, 0, s->stream>>>(s->Rl.p, s->rdst.p, s->R.p, s->ibool.p, s->inj_cells.p, s->inj_w.p,
+        const GatherPlan& gp = s->by_point;
+        dev::k_inject<<<1, 128, 0, s->stream>>>(gp.Rl.p, gp.rdst.p, s->R.p, s->ibool.p, s->inj_cells.p, s->inj_w.p,
                                                int(cells.size()), direction, float(stf_val),
-                                               s->PR, s->fstride, field,
+                                               gp.PR, s->fstride, field,
                                                s->assembly == GFX_ASSEMBLY_GATHER ? 1 : 0);
         GFX_HIP(hipGetLastError());
     });
@@ -1678,9 +2034,10 @@ extern "C" gfx_status gfx_step_scatter_to_rank(gfx_solver* s) {
     return guarded([&] {
         stage_require(s, STAGE_ELEMENT, "gfx_step_scatter_to_rank", "gfx_step_element_residual");
         if (s->assembly == GFX_ASSEMBLY_GATHER) {
-            const StepArgs a = make_step_args(*s);
+            const StepArgs a = make_step_args(*s, true);
             dim3 grid(unsigned((s->G4 + 255) / 256), unsigned(s->nf));
-            dev::k_scatter_slots<<<grid, 256, 0, s->stream>>>(a.na);
+            dev::k_scatter_slots<<<grid, 256, 0, s->stream>>>(a.na,
+                                                             uses_clusters(*s) ? s->by_point.new_cluster.p : nullptr);
             GFX_HIP(hipGetLastError());
         }
         // COLORED and ATOMIC assemble into R inside the element stage
@@ -1693,7 +2050,7 @@ extern "C" gfx_status gfx_step_newmark_correct(gfx_solver* s, double dt, double 
         stage_require(s, STAGE_ASSEMBLED, "gfx_step_newmark_correct", "gfx_step_scatter_to_rank");
         check_newmark(s, dt, beta);
         require(gamma == 0.5, "the solver's Newmark scheme has gamma = 1/2");
-        StepArgs a = make_step_args(*s);
+        StepArgs a = make_step_args(*s, true);
         a.na.gather = 0;  // R holds the assembled residual (k_scatter_slots, or the exchange)
         if (a.spec_grid > 0) launch_node_special(*s, a.na, a.spec_grid);
         if (a.reg_grid > 0) launch_node_regular(*s, a.na, a.reg_grid);
@@ -1703,7 +2060,7 @@ extern "C" gfx_status gfx_step_newmark_correct(gfx_solver* s, double dt, double 
         GFX_HIP(hipGetLastError());
         advance_host(*s);
         s->stage = STAGE_IDLE;
-        s->r_in_R = true;
+        s->r_src = R_ASSEMBLED;
     });
 }
 
@@ -1855,16 +2212,17 @@ extern "C" gfx_status gfx_solver_checkpoint_save(const gfx_solver* s, void* host
         get(s->devp.p, s->devp.n);
         // assembled residual of the last step (what get_state reads for a at
         // regular nodes): R itself, or the fixed-order slot sums
-        if (s->assembly != GFX_ASSEMBLY_GATHER || s->r_in_R) {
+        if (s->r_src == R_ASSEMBLED) {
             get(s->R.p, fl);
         } else {
             std::fill(p, p + fl, 0.f);
             for (int f = 0; f < s->nf; ++f) {
-                const std::vector<float> hl = fetch(s, s->Rl.p + int64_t(f) * s->PR * 3, size_t(s->PR) * 3);
+                const GatherPlan& gp = plan_of(*s, s->r_src);
+                const std::vector<float> hl = fetch(s, gp.Rl.p + int64_t(f) * gp.PR * 3, size_t(gp.PR) * 3);
                 float* r = p + int64_t(f) * s->fstride;
                 for (int64_t n = 0; n < s->G; ++n)
-                    for (int q = s->goff_host[n]; q < s->goff_host[n + 1]; ++q)
-                        for (int c = 0; c < 3; ++c) r[n * 3 + c] += hl[int64_t(s->gpts_host[q]) * 3 + c];
+                    for (int q = gp.off_host[n]; q < gp.off_host[n + 1]; ++q)
+                        for (int c = 0; c < 3; ++c) r[n * 3 + c] += hl[int64_t(gp.pts_host[q]) * 3 + c];
             }
         }
     });
@@ -1898,21 +2256,20 @@ extern "C" gfx_status gfx_solver_checkpoint_load(gfx_solver* s, const void* host
         if (s->assembly != GFX_ASSEMBLY_GATHER) {
             put(s->R.p, fl);
         } else {
-            // the sum at the first point of each node, zeros elsewhere: get_state
-            // then forms the same r
-            std::vector<float> hl(size_t(s->PR) * 3);
+            // the sum at each node's first entry (its own index), zeros elsewhere:
+            // get_state then forms the same r
+            require_plan(*s, active_plan(*s));
+            const GatherPlan& gp = plan_of(*s, active_plan(*s));
+            std::vector<float> hl(size_t(gp.PR) * 3, 0.f);
             for (int f = 0; f < s->nf; ++f) {
-                std::fill(hl.begin(), hl.end(), 0.f);
                 const float* r = p + int64_t(f) * s->fstride;
-                for (int64_t n = 0; n < s->G; ++n)
-                    if (s->goff_host[n + 1] > s->goff_host[n])
-                        for (int c = 0; c < 3; ++c) hl[int64_t(s->gpts_host[s->goff_host[n]]) * 3 + c] = r[n * 3 + c];
-                GFX_HIP(hipMemcpy(s->Rl.p + int64_t(f) * s->PR * 3, hl.data(), hl.size() * 4, hipMemcpyHostToDevice));
+                std::copy(r, r + size_t(s->G) * 3, hl.begin());
+                GFX_HIP(hipMemcpy(gp.Rl.p + int64_t(f) * gp.PR * 3, hl.data(), hl.size() * 4, hipMemcpyHostToDevice));
             }
         }
         s->step = int(hdr[5]);
         s->n_snap = int(hdr[6]);
-        s->r_in_R = false;
+        s->r_src = active_plan(*s);
         s->stage = 0;
         upload_counters(*s);
     });
@@ -1997,8 +2354,8 @@ extern "C" gfx_status gfx_autotune(const gfx_solver_desc* base, int trial_steps,
         gfx_solver_desc pick = *base;
         const int asms[2] = {GFX_ASSEMBLY_COLORED, GFX_ASSEMBLY_GATHER};
         constexpr int NL = 9;
-        const int launch[NL][2] = {{GFX_ELEMENT_BLOCK, 1}, {GFX_ELEMENT_BLOCK, 2}, {GFX_ELEMENT_BLOCK, 4},
-                                   {GFX_ELEMENT_WAVE, 2},  {GFX_ELEMENT_WAVE, 4},  {GFX_ELEMENT_WAVE, 8},
+        const int launch[NL][2] = {{GFX_ELEMENT_WAVE, 8},  {GFX_ELEMENT_WAVE, 2},  {GFX_ELEMENT_WAVE, 4},
+                                   {GFX_ELEMENT_BLOCK, 1}, {GFX_ELEMENT_BLOCK, 2}, {GFX_ELEMENT_BLOCK, 4},
                                    {GFX_ELEMENT_PAIR, 1},  {GFX_ELEMENT_PAIR, 2},  {GFX_ELEMENT_PENCIL, 0}};
         auto time_steps = [&](gfx_solver& S) {
             run_steps(S, 1);  // warm-up
@@ -2034,6 +2391,8 @@ extern "C" gfx_status gfx_autotune(const gfx_solver_desc* base, int trial_steps,
                 const auto& lc = launch[li];
                 if (lc[0] != GFX_ELEMENT_BLOCK && ref_elem_pml(*S)) continue;
                 if (lc[0] == GFX_ELEMENT_PAIR && S->nf < 2) continue;
+                // the cluster kernel is one form for every elements-per-block request
+                if (lc[0] == GFX_ELEMENT_WAVE && lc[1] != 8 && S->assembly == GFX_ASSEMBLY_GATHER && S->cl_ok) continue;
                 S->kernel = lc[0];
                 S->epb = resolve_epb(lc[0], lc[1]);
                 const double per = time_steps(*S);
@@ -2047,7 +2406,7 @@ extern "C" gfx_status gfx_autotune(const gfx_solver_desc* base, int trial_steps,
             S->epb = resolve_epb(launch[best_lc][0], launch[best_lc][1]);
             int best_fg = fg0;
             for (int fg : {1, 2, 4, 8}) {
-                if (fg == fg0 || fg > 2 * S->nf) continue;
+                if (fg == fg0 || fg > 2 * S->nf || uses_clusters(*S)) continue;
                 S->node_fg = fg;
                 const double per = time_steps(*S);
                 if (per < best_here) {
@@ -2197,7 +2556,7 @@ bool groupable(const gfx_batch& B, const std::vector<char>& active) {
         if (!active[i]) continue;
         const gfx_solver& S = *B.s[i];
         if (S.assembly != GFX_ASSEMBLY_GATHER || (S.has_cpml && !S.pml_nodal) || S.n_sls > 0) return false;
-        if (S.kernel != GFX_ELEMENT_BLOCK && S.kernel != GFX_ELEMENT_WAVE) return false;
+        if (S.kernel != GFX_ELEMENT_BLOCK && !uses_clusters(S)) return false;
         if (first && (S.kernel != first->kernel || S.epb != first->epb || S.node_fg != first->node_fg)) return false;
         if (!first) first = &S;
     }
@@ -2209,12 +2568,7 @@ void launch_element_grp(int kernel, int epb, gfx_batch::Group& c, const gfx::Dev
                         hipStream_t st) {
     constexpr int M = dev::ASM_GATHER;
     if (kernel == GFX_ELEMENT_WAVE) {
-        switch (epb) {
-            case 1: dev::k_element_wave_grp<1, M, DIAG><<<grid, 64, 0, st>>>(c.etab.p, map.p); break;
-            case 2: dev::k_element_wave_grp<2, M, DIAG><<<grid, 128, 0, st>>>(c.etab.p, map.p); break;
-            case 4: dev::k_element_wave_grp<4, M, DIAG><<<grid, 256, 0, st>>>(c.etab.p, map.p); break;
-            default: dev::k_element_wave_grp<8, M, DIAG><<<grid, 512, 0, st>>>(c.etab.p, map.p); break;
-        }
+        dev::k_cluster_grp<DIAG><<<grid, dev::CLUSTER_THREADS, 0, st>>>(c.etab.p, map.p);
     } else {
         constexpr auto T = [](int e) { return ((e * NP + 63) / 64) * 64; };
         switch (epb) {
@@ -2231,6 +2585,8 @@ void launch_nodes_grp(gfx_batch::Group& c, hipStream_t st) {
     if (c.bs > 0) dev::k_node_special_grp<FG><<<c.bs, 256, 0, st>>>(c.ntab.p, c.map_spec.p);
     if (c.br > 0) dev::k_node_regular_grp<true, FG><<<c.br, 256, 0, st>>>(c.ntab.p, c.map_reg.p);
 }
+
+constexpr int GROUP_CHUNK = 4;  // fields per workgroup of a group's node launch (cluster form)
 
 // Argument tables and entries of a group of solvers, uploaded before the
 // capture that records the group's launches.
@@ -2252,10 +2608,20 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
         for (const auto& rg : S.ranges) {
             const int n = rg.e - rg.b;
             auto& m = rg.diag ? ed : eg;
+            if (kernel == GFX_ELEMENT_WAVE) {
+                for (int cl = rg.cb; cl < rg.ce; ++cl) m.push_back(make_int4(t, cl, 0, 0));
+                continue;
+            }
             for (int w = 0; w < (n + S.epb - 1) / S.epb; ++w) m.push_back(make_int4(t, rg.b, n, w));
         }
-        for (int w = 0; w < args[i].spec_grid; ++w) es.push_back(make_int4(t, 0, 0, w));
-        for (int w = 0; w < args[i].reg_grid; ++w) er.push_back(make_int4(t, 0, 0, w));
+        if (args[i].clusters) {  // all nodes in the one launch of c.map_spec
+            for (int f = 0; f < S.nf; f += GROUP_CHUNK)
+                for (int w = 0; w < args[i].spec_grid + args[i].reg_grid; ++w)
+                    es.push_back(make_int4(t, args[i].spec_grid, f, w));
+        } else {
+            for (int w = 0; w < args[i].spec_grid; ++w) es.push_back(make_int4(t, 0, 0, w));
+            for (int w = 0; w < args[i].reg_grid; ++w) er.push_back(make_int4(t, 0, 0, w));
+        }
         ctr.push_back(S.ctr.p);
         strides.push_back(S.stride);
     }
@@ -2287,7 +2653,9 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
 void enqueue_group(gfx_batch::Group& c, const std::vector<StepArgs>& args, hipStream_t st) {
     if (c.bg > 0) launch_element_grp<false>(c.kernel, c.epb, c, c.map_gen, c.bg, st);
     if (c.bd > 0) launch_element_grp<true>(c.kernel, c.epb, c, c.map_diag, c.bd, st);
-    switch (c.fg) {
+    if (c.kernel == GFX_ELEMENT_WAVE && c.bs > 0)
+        dev::k_cluster_nodes_grp<<<c.bs, 256, 0, st>>>(c.ntab.p, c.map_spec.p, GROUP_CHUNK);
+    else switch (c.fg) {
         case 2: launch_nodes_grp<2>(c, st); break;
         case 4: launch_nodes_grp<4>(c, st); break;
         case 8: launch_nodes_grp<8>(c, st); break;
@@ -2413,7 +2781,10 @@ extern "C" gfx_status gfx_batch_run(gfx_batch* b, int n_steps, const int* until)
             if (!any) break;
             GFX_HIP(hipGraphLaunch(batch_graph(*b, active), b->stream));
             for (size_t i = 0; i < b->s.size(); ++i)
-                if (active[i]) advance_host(*b->s[i]);
+                if (active[i]) {
+                    b->s[i]->r_src = active_plan(*b->s[i]);
+                    advance_host(*b->s[i]);
+                }
         }
         GFX_HIP(hipStreamSynchronize(b->stream));
     });

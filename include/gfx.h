@@ -98,7 +98,10 @@ typedef enum {
 typedef enum {
     GFX_ELEMENT_AUTO = 0,  /* wave kernel when applicable, else block kernel */
     GFX_ELEMENT_BLOCK = 1, /* one lane per GLL point, workgroup barriers between stages */
-    GFX_ELEMENT_WAVE = 2,  /* one wavefront per element, two points per lane, no barriers */
+    GFX_ELEMENT_WAVE = 2,  /* one wavefront per element, two points per lane, no barriers; with
+                              GATHER assembly of elastic elements (nodal or no C-PML): clusters
+                              of up to eight elements per workgroup whatever elems_per_block,
+                              shared nodes summed per cluster, interior nodes updated in place */
     GFX_ELEMENT_PAIR = 3,  /* as BLOCK, two fields per pass (nodal C-PML only) */
     GFX_ELEMENT_PENCIL = 4 /* lane per 5-point pencil along k, ten elements per workgroup
                               (fixed; elems_per_block must be 0), k contractions in

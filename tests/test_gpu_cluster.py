@@ -1,0 +1,80 @@
+"""The cluster kernel (GATHER assembly, wavefront element form) at the sizes
+where its tables have edges: clusters of one element, of fewer than eight, odd
+element counts per axis, elements in caller order (no centroids, runs of eight),
+axis-aligned and general geometry, one and several fields, with and without
+C-PML, forces whose cells share nodes across clusters.
+
+Against the lane-per-point block kernel on the same mesh, which sums each
+node's points in another order: both round in FP32, so after a few dozen steps
+the states agree to some 1e-6 relative; the bars are 1e-5 for u and v and 1e-4
+for the acceleration, which is a difference of much larger element forces."""
+import numpy as np
+import pytest
+
+import meshcases as mc
+import pygfx
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(mesh, nf, kernel, has_cpml, morton, steps=30):
+    cells, w, stf = mc.buried_source(mesh, frac=(0.5, 0.5, 0.0), depth=0.4 * (mesh.bounds[5] - mesh.bounds[4]))
+    s = pygfx.Solver(mesh, n_fields=nf, assembly=pygfx.GFX_ASSEMBLY_GATHER, element_kernel=kernel, has_cpml=has_cpml,
+                     morton=morton, record_capacity=1, rec_cell=np.zeros(0, np.int32))
+    rng = np.random.default_rng(3)
+    for f in range(nf):
+        s.set_source(f, f % 3, cells, w, stf)
+        u, v = (rng.normal(size=mesh.n_node * 3) * k for k in (1e-3, 1e-2))
+        s.set_state(f, u, v, np.zeros_like(u))
+    s.run(steps)
+    return [s.get_state(f) for f in range(nf)]
+
+
+@pytest.mark.parametrize("nx,ny,nz,nf,jitter,has_cpml,morton", [
+    (1, 1, 1, 1, 0.0, False, True),    # one element, every node interior
+    (3, 1, 1, 2, 0.0, False, True),
+    (3, 3, 2, 1, 0.2, False, True),
+    (2, 2, 2, 3, 0.0, False, True),    # exactly one full cluster
+    (5, 7, 3, 3, 0.0, True, True),
+    (5, 4, 5, 1, 0.15, True, True),
+    (4, 5, 3, 25, 0.0, True, False),   # runs of eight in caller order
+    (9, 6, 7, 4, 0.1, True, False)])
+def test_cluster_kernel_matches_block_kernel(nx, ny, nz, nf, jitter, has_cpml, morton):
+    pml = 1 if has_cpml else 0
+    mesh = pygfx.build_box(nx=nx, ny=ny, nz=nz, lx=600.0 * nx, ly=600.0 * ny, lz=600.0 * nz,
+                           layers=[(900.0, 5000.0, 2900.0, 2500.0), (0.0, 6200.0, 3600.0, 2800.0)],
+                           pml_xmin=pml, pml_xmax=pml, pml_ymin=pml, pml_ymax=pml, pml_zmax=pml, f0_pml=1.5,
+                           jitter=jitter, jitter_seed=5, duration=1.0, record_depth_max=0.0)
+    print(f"case: {nx}x{ny}x{nz}, {nf} fields, jitter {jitter}, cpml {has_cpml}, centroids {morton}", flush=True)
+    a = _run(mesh, nf, pygfx.GFX_ELEMENT_AUTO, has_cpml, morton)
+    b = _run(mesh, nf, pygfx.GFX_ELEMENT_BLOCK, has_cpml, morton)
+    for x, y in zip(a, b):
+        for p, q, bar in zip(x, y, (1e-5, 1e-5, 1e-4)):
+            assert np.isfinite(p).all()
+            assert mc.rel_l2(p, q) <= bar
+
+
+def test_switching_the_element_kernel_keeps_the_state():
+    """A solver moved between the cluster and the block form mid-run (each has
+    its own residual entries) continues from the same state, and the
+    acceleration read after a switch is the last step's."""
+    mesh = mc.small_layered(duration=0.8)
+    cells, w, stf = mc.buried_source(mesh)
+    s = pygfx.Solver(mesh, assembly=pygfx.GFX_ASSEMBLY_GATHER, record_capacity=1)
+    s.set_source(0, 2, cells, w, stf)
+    s.run(12)
+    before = s.get_state(0)
+    s.set_launch(pygfx.GFX_ELEMENT_BLOCK, 1)
+    for x, y in zip(s.get_state(0), before):
+        assert np.array_equal(x, y)
+    image = s.checkpoint()
+    s.run(5)
+    s.set_launch(pygfx.GFX_ELEMENT_WAVE, 4)
+    after = s.get_state(0)
+    s.restore(image)
+    for x, y in zip(s.get_state(0), before):
+        assert np.array_equal(x, y)
+    s.set_launch(pygfx.GFX_ELEMENT_BLOCK, 1)
+    s.run(5)
+    for x, y in zip(s.get_state(0), after):
+        assert np.array_equal(x, y)

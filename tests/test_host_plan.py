@@ -71,3 +71,17 @@ def test_complete_cpml_plans_and_rejects_bad_inputs(assembly):
     no_profiles = mc.small_layered(nx=5, ny=4, nz=4, pml=1)
     with pytest.raises(ValueError, match="want_profiles"):
         pygfx.Solver(no_profiles, cpml_complete=True)
+
+
+@pytest.mark.parametrize("nx,ny,nz,morton", [(1, 1, 1, True), (3, 1, 2, True), (2, 2, 2, False), (5, 7, 3, True),
+                                             (9, 6, 7, False)])
+def test_cluster_tables_plan_at_every_size(nx, ny, nz, morton):
+    """The cluster form's tables (partial clusters, odd counts, caller order)
+    pass the plan's own checks: every point listed once, the interior nodes one
+    run of ids per cluster."""
+    mesh = pygfx.build_box(nx=nx, ny=ny, nz=nz, lx=600.0 * nx, ly=600.0 * ny, lz=600.0 * nz,
+                           layers=[(0.0, 6200.0, 3600.0, 2800.0)], pml_xmin=0, pml_xmax=0, pml_ymin=0, pml_ymax=0,
+                           pml_zmax=0, duration=1.0, record_depth_max=0.0)
+    with pytest.raises(pygfx.GfxError) as ei:
+        pygfx.Solver(mesh, assembly=pygfx.GFX_ASSEMBLY_GATHER, has_cpml=False, morton=morton, record_capacity=0)
+    assert ei.value.status == GFX_ERR_DEVICE, str(ei.value)
