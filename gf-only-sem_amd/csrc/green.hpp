@@ -5,6 +5,8 @@
 // element points at that node, postprocess/cpp/main.cpp:354-426).
 #pragma once
 
+#include <mutex>
+
 #include "device.hpp"
 #include "gfx.h"
 
@@ -27,6 +29,30 @@ struct gfx_green {
     std::vector<double> h_xyz, h_box;
     std::vector<int32_t> h_cell;
     hipStream_t stream = nullptr;
+    // device copies of an interpolation's queries and answers, kept between calls
+    // (up to KEEP queries, 26 MB) and held by one call at a time
+    struct Work {
+        static constexpr size_t KEEP = 262144;
+        gfx::DevBuf<double> q;
+        gfx::DevBuf<int32_t> t, c;
+        gfx::DevBuf<float> o;
+        void fit(size_t n) {
+            if (q.n >= n * 3) return;
+            q.alloc(n * 3);
+            t.alloc(n);
+            c.alloc(n);
+            o.alloc(n * 18);
+        }
+        void trim() {
+            if (t.n <= KEEP) return;
+            q.release();
+            t.release();
+            c.release();
+            o.release();
+        }
+    };
+    mutable std::mutex work_mu;
+    mutable Work work;
     ~gfx_green() {
         if (stream) (void)hipStreamDestroy(stream);
     }

@@ -10,9 +10,9 @@
 //
 // MLP: (x, y, z, t) scaled to [-1, 1] -> [sin, cos](2 pi B x) with B ~ N(0,
 // sigma^2) (n_freq x 4) -> depth x (Linear(width) + GELU) -> Linear(n_out).
-// Every product runs on v_mfma_f32_16x16x32_bf16 (LDS-tiled): operands
-// rounded to BF16 (round to nearest even), FP32 accumulation; master weights
-// and Adam moments stay FP32.
+// Every product runs on v_mfma_f32_16x16x32_bf16: operands rounded to BF16
+// (round to nearest even), FP32 accumulation; master weights and Adam moments
+// stay FP32.
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -97,59 +97,139 @@ __host__ __device__ inline int64_t region_of(int cell, int t, int n_time, int n_
     return int64_t(cell) * n_window + w;
 }
 
-// only (may be null): evaluate just the points whose region is marked there
-__global__ void k_judge(JudgeArgs A, int n, const double* __restrict__ q, const int32_t* __restrict__ tix,
-                        const uint8_t* __restrict__ only, int n_window, float* __restrict__ out,
-                        int32_t* __restrict__ cell_out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double p[3] = {q[3 * i], q[3 * i + 1], q[3 * i + 2]};
-    const int c = find_cell(A, p);
-    if (cell_out) cell_out[i] = c;
-    const int t = tix[i];
-    if (only && (c < 0 || !only[region_of(c, t, A.n_time, n_window)])) return;
-    float* o = out + int64_t(i) * 18;
+// Lanes of one wavefront exchange data through LDS.
+__device__ inline void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Q queries per wavefront: a lane each finds the cells, then the wavefront
+// evaluates one query after the other with the 125 nodes of its cell spread over
+// the lanes for the exact-node test and the weights; for the sum, 63 lanes take
+// seven nodes at a time, nine lanes of two values each.  Q = 1 up to 8,192
+// queries, which then all run at once, and grows beyond, so that the search is
+// not repeated by 64 lanes.  One lane per query took 97 us for 600 queries (its
+// 2,375 dependent loads run one after the other); this takes 14 us.
+// policy null: every point is evaluated, NaN where there is no cell or time.
+// policy [n_cell][n_window]: out holds other answers; a point keeps them where
+// its region says 0, becomes zero at 2, and is evaluated at 1 and outside all
+// cells (NaN there); *count is raised by the points evaluated.
+constexpr int JQ = 4;  // wavefronts per workgroup
+
+struct JudgeShared {
+    double lag[15], w[NP + 3], part[7][18];
+};
+
+__device__ inline void judge_eval(const JudgeArgs& A, JudgeShared& S, const double (&p)[3], int c, int t,
+                                  float* __restrict__ o) {
+    const int lane = threadIdx.x & 63;
     if (c < 0 || t < 0 || t >= A.n_time) {
-        for (int k = 0; k < 18; ++k) o[k] = __builtin_nanf("");
+        if (lane < 18) o[lane] = __builtin_nanf("");
         return;
     }
     const int32_t* ci = A.cell_idx + int64_t(c) * NP;
     const float* vt = A.val + int64_t(t) * A.n_node * 18;
-    // exact-node shortcut (gll_interpolator.py:172-177)
-    for (int k = 0; k < NP; ++k) {
-        const double* x = A.xyz + int64_t(ci[k]) * 3;
-        const double dx = x[0] - p[0], dy = x[1] - p[1], dz = x[2] - p[2];
-        if (dx * dx + dy * dy + dz * dz < EXACT_TOL * EXACT_TOL) {
-            const float* v = vt + int64_t(ci[k]) * 18;
-            for (int m = 0; m < 18; ++m) o[m] = v[m];
-            return;
+    // exact-node shortcut (gll_interpolator.py:172-177): the first such node
+    int hit = -1;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int k = lane + 64 * h;
+        bool at = false;
+        if (k < NP) {
+            const double* x = A.xyz + int64_t(ci[k]) * 3;
+            const double dx = x[0] - p[0], dy = x[1] - p[1], dz = x[2] - p[2];
+            at = dx * dx + dy * dy + dz * dz < EXACT_TOL * EXACT_TOL;
         }
+        const unsigned long long m = __ballot(at);
+        if (hit < 0 && m) hit = 64 * h + __ffsll(m) - 1;
     }
-    const double* bx = A.box + int64_t(c) * 6;
-    double xi[3];
-    for (int d = 0; d < 3; ++d) {
+    if (hit >= 0) {
+        if (lane < 18) o[lane] = vt[int64_t(ci[hit]) * 18 + lane];
+        return;
+    }
+    if (lane < 15) {  // lane (axis d, point a): its Lagrange polynomial at the query
+        const double g[5] = {-1.0, -0.6546536707079771, 0.0, 0.6546536707079771, 1.0};  // sqrt(3/7)
+        const int d = lane / 5, a = lane - 5 * d;
+        const double* bx = A.box + int64_t(c) * 6;
+        const double pd = d == 0 ? p[0] : d == 1 ? p[1] : p[2];
         const double lo = bx[2 * d], hi = bx[2 * d + 1];
-        xi[d] = fmin(1.0, fmax(-1.0, 2.0 * (p[d] - lo) / (hi - lo) - 1.0));
+        const double xi = fmin(1.0, fmax(-1.0, 2.0 * (pd - lo) / (hi - lo) - 1.0));
+        const double ga = a == 0 ? g[0] : a == 1 ? g[1] : a == 2 ? g[2] : a == 3 ? g[3] : g[4];
+        double v = 1.0;
+#pragma unroll
+        for (int j = 0; j < 5; ++j)
+            if (j != a) v *= (xi - g[j]) / (ga - g[j]);
+        S.lag[lane] = v;
     }
-    double lx[5], ly[5], lz[5];
-    lagrange5(xi[0], lx);
-    lagrange5(xi[1], ly);
-    lagrange5(xi[2], lz);
-    double sw = 0.0;
-    for (int a = 0; a < 5; ++a)
-        for (int b = 0; b < 5; ++b)
-            for (int k = 0; k < 5; ++k) sw += lx[a] * ly[b] * lz[k];
-    double acc[18];
-    for (int m = 0; m < 18; ++m) acc[m] = 0.0;
-    for (int a = 0; a < 5; ++a)
-        for (int b = 0; b < 5; ++b)
-            for (int k = 0; k < 5; ++k) {
-                const double w = lx[a] * ly[b] * lz[k] / sw;
-                const float* v = vt + int64_t(ci[(a * 5 + b) * 5 + k]) * 18;
-                for (int m = 0; m < 18; ++m) acc[m] += w * double(v[m]);
-            }
-    for (int m = 0; m < 18; ++m) o[m] = float(acc[m]);
+    wave_sync();
+    double w[2] = {0.0, 0.0}, sw;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int k = lane + 64 * h;
+        if (k < NP) w[h] = S.lag[k / 25] * S.lag[5 + (k / 5) % 5] * S.lag[10 + k % 5];
+    }
+    sw = w[0] + w[1];
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) sw += __shfl_xor(sw, s);
+    S.w[lane] = w[0] / sw;
+    if (lane + 64 < NP) S.w[lane + 64] = w[1] / sw;
+    wave_sync();
+    const int sub = lane / 9, pair = lane - 9 * sub;
+    if (sub < 7) {
+        double a0 = 0.0, a1 = 0.0;
+#pragma unroll 6
+        for (int k = sub; k < NP; k += 7) {
+            const float2 v = *reinterpret_cast<const float2*>(vt + int64_t(ci[k]) * 18 + 2 * pair);
+            a0 += S.w[k] * double(v.x);
+            a1 += S.w[k] * double(v.y);
+        }
+        S.part[sub][2 * pair] = a0;
+        S.part[sub][2 * pair + 1] = a1;
+    }
+    wave_sync();
+    if (lane < 18) {
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < 7; ++k) s += S.part[k][lane];
+        o[lane] = float(s);
+    }
+    wave_sync();  // S is rewritten by the next query
 }
+
+__global__ void __launch_bounds__(64 * JQ)
+    k_judge(JudgeArgs A, int n, int Q, const double* __restrict__ q, const int32_t* __restrict__ tix,
+            const uint8_t* __restrict__ policy, int n_window, float* __restrict__ out, int32_t* __restrict__ cell_out,
+            int* __restrict__ count) {
+    __shared__ JudgeShared sh[JQ];
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int64_t base = (int64_t(blockIdx.x) * JQ + wv) * Q;
+    const bool mine = lane < Q && base + lane < n;
+    double p[3] = {0.0, 0.0, 0.0};
+    int c = -1, t = 0, how = 0;
+    if (mine) {
+        const int64_t i = base + lane;
+        for (int d = 0; d < 3; ++d) p[d] = q[3 * i + d];
+        t = tix[i];
+        c = find_cell(A, p);
+        if (cell_out) cell_out[i] = c;
+        how = !policy || c < 0 ? 1 : policy[region_of(c, t, A.n_time, n_window)];
+        if (how == 2)
+            for (int k = 0; k < 18; ++k) out[i * 18 + k] = 0.f;
+    }
+    unsigned long long todo = __ballot(how == 1);
+    if (count && lane == 0 && todo) atomicAdd(count, __popcll(todo));
+    while (todo) {
+        const int l = __ffsll(todo) - 1;
+        todo &= todo - 1;
+        const double pq[3] = {__shfl(p[0], l), __shfl(p[1], l), __shfl(p[2], l)};
+        judge_eval(A, sh[wv], pq, __shfl(c, l), __shfl(t, l), out + (base + l) * 18);
+    }
+}
+
+// Queries per wavefront and workgroups for n queries.
+int judge_q(int n) { return std::min(64, std::max(1, (n + 8191) / 8192)); }
+int judge_blocks(int n) { return int((n + int64_t(JQ) * judge_q(n) - 1) / (int64_t(JQ) * judge_q(n))); }
 
 JudgeArgs judge_args(const gfx_green& G) {
     JudgeArgs a{};
@@ -175,180 +255,359 @@ JudgeArgs judge_args(const gfx_green& G) {
 }
 
 // -------------------------------- MLP -------------------------------------
+//
+// Every product is one form: C(m, n) = sum_k A[m][k] B[n][k] with both operands
+// BF16 and k-contiguous, leading dimensions padded to 64 with zeros.  Whoever
+// makes an operand (features, a layer's GELU, its gradient, Adam) rounds it to
+// BF16 once (nearest even) in the layout, or the two layouts, in which products
+// read it: activations and gradients [row][unit] for the next product along the
+// network and [unit][row] for the weight gradients, weights both ways.  Sums,
+// biases, pre-activations, master weights and moments stay FP32.
+//
+// Bound: at 131,072 rows a hidden layer takes 115 us, of which erff is more than
+// half (33.5 M values); its traffic would take 26 us.  At a training batch of
+// 8,192 rows the launches are latency bound (15 us a layer).  One Adam iteration
+// of the default network: 344 us, with FP32 operands rounded and transposed
+// while staging, separate bias and GELU passes and 256-term sums by single lanes
+// 1,380 us; 150,000 queries: 1.3 ms of kernels (2.9 ms).
 
-// C = op(A) op(B) with A(m,k) = TA ? A[k*lda+m] : A[m*lda+k] and
-// B(k,n) = TB ? B[n*ldb+k] : B[k*ldb+n], on gfx950's
-// v_mfma_f32_16x16x32_bf16, tiled through LDS: a workgroup of four wavefronts computes a 128 x 128 tile of C (each wavefront
-// 64 x 64 = 4 x 4 MFMA tiles, 16 accumulators of 4 floats), stepping K by 32.
-// Each step stages the A (128 x 32) and B (32 x 128) slices in LDS as BF16
-// (round to nearest even), both k-contiguous per row / column, so every MFMA
-// operand is one 16-byte LDS read; rows are padded to 40 BF16 (80 bytes), so
-// the 16 lanes of a read phase hit distinct banks.  Lane layout of the 16 x 16
-// x 32 BF16 MFMA: lane l feeds A row l % 16 and B column l % 16 with k =
-// 8 (l / 16) .. + 7, and receives D rows 4 (l / 16) .. + 3 of column l % 16.
-// The K range is split over gridDim.z (kc a multiple of 32); split z writes
-// C + z*M*ldc, summed later in a fixed order.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-constexpr int GT = 128, GK = 32, GKP = 40;
+constexpr int GK = 64;        // k per stage, and the padding of leading dimensions
+constexpr int GKP = GK + 8;   // LDS row: 144 bytes, so the 16 lanes of a read phase meet distinct banks
 
-template <bool TA, bool TB>
-__global__ void __launch_bounds__(256) k_gemm_lds(const float* __restrict__ A, int lda, const float* __restrict__ B,
-                                                  int ldb, float* __restrict__ C, int ldc, int M, int N, int K,
-                                                  int kc) {
-    __shared__ __attribute__((aligned(16))) uint16_t sA[GT * GKP];
-    __shared__ __attribute__((aligned(16))) uint16_t sB[GT * GKP];
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-    const int mb = blockIdx.y * GT, nb = blockIdx.x * GT;
-    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-    const int kbeg = blockIdx.z * kc, kend = min(K, kbeg + kc);
-    float* Cz = C + int64_t(blockIdx.z) * M * ldc;
-    f32x4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int r16 = lane & 15, kq = (lane >> 4) * 8;
-    for (int k0 = kbeg; k0 < kend; k0 += GK) {
-        __syncthreads();  // the previous slices have been read
-        // stage: 16 values of A and 16 of B per lane
-        if (!TA) {  // A(m, k) = A[m * lda + k]: lane -> row t / 2, k half (t & 1)
-            const int m = t >> 1, kk = (t & 1) * 16;
-            const int gm = mb + m;
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int k = k0 + kk + q;
-                const float v = (gm < M && k < kend) ? A[int64_t(gm) * lda + k] : 0.f;
-                sA[m * GKP + kk + q] = f2bf(v);
-            }
-        } else {  // A(m, k) = A[k * lda + m]: lane -> k = t / 8, 16 rows
-            const int kk = t >> 3, m0 = (t & 7) * 16;
-            const int k = k0 + kk;
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int gm = mb + m0 + q;
-                const float v = (gm < M && k < kend) ? A[int64_t(k) * lda + gm] : 0.f;
-                sA[(m0 + q) * GKP + kk] = f2bf(v);
-            }
-        }
-        if (TB) {  // B(k, n) = B[n * ldb + k]: lane -> column t / 2, k half (t & 1)
-            const int n = t >> 1, kk = (t & 1) * 16;
-            const int gn = nb + n;
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int k = k0 + kk + q;
-                const float v = (gn < N && k < kend) ? B[int64_t(gn) * ldb + k] : 0.f;
-                sB[n * GKP + kk + q] = f2bf(v);
-            }
-        } else {  // B(k, n) = B[k * ldb + n]: lane -> k = t / 8, 16 columns
-            const int kk = t >> 3, n0 = (t & 7) * 16;
-            const int k = k0 + kk;
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int gn = nb + n0 + q;
-                const float v = (gn < N && k < kend) ? B[int64_t(k) * ldb + gn] : 0.f;
-                sB[(n0 + q) * GKP + kk] = f2bf(v);
-            }
-        }
-        __syncthreads();
-        bf16x8 a[4], b[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) a[i] = *reinterpret_cast<const bf16x8*>(&sA[(wm + i * 16 + r16) * GKP + kq]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) b[j] = *reinterpret_cast<const bf16x8*>(&sB[(wn + j * 16 + r16) * GKP + kq]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int m = mb + wm + i * 16 + (lane >> 4) * 4 + q, n = nb + wn + j * 16 + r16;
-                if (m < M && n < N) Cz[int64_t(m) * ldc + n] = acc[i][j][q];
-            }
-}
+inline int pad64(int n) { return (n + 63) / 64 * 64; }
 
-// dst[i] = sum_z src[z*n + i], z in order
-__global__ void k_sum_splits(const float* __restrict__ src, int splits, int64_t n, float* __restrict__ dst) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float s = 0.f;
-    for (int z = 0; z < splits; ++z) s += src[int64_t(z) * n + i];
-    dst[i] = s;
-}
+// What a product's tile turns into.
+enum {
+    EPI_HIDDEN = 0,  // z = acc + bias; optionally Z = z; gelu(z) as BF16, one or two layouts
+    EPI_OUT = 1,     // acc + bias, FP32
+    EPI_BACK = 2,    // acc * gelu'(Z) as BF16, both layouts, and its column sums (bias gradient)
+    EPI_PART = 3     // acc, FP32 partial product of one k range
+};
+
+struct GemmArgs {
+    const uint16_t* A;
+    const uint16_t* B;
+    int lda, ldb;
+    int M, N, K;          // K a multiple of 64 (zero padded)
+    const float* bias;    // [N]
+    float* Z;             // [M][ldz] pre-activations (written by EPI_HIDDEN when set, read by EPI_BACK)
+    int ldz;              // padded to 64
+    uint16_t* H;          // [M][ldh], may be null
+    int ldh;
+    uint16_t* Ht;         // [N][ldt] transposed, rows m in [M, ldt) zero; may be null
+    int ldt;
+    float* out;           // EPI_OUT [M][N]; EPI_PART [z][M][N]; EPI_BACK [row tile][N] column sums
+};
+
+// The weight gradients of all layers as one launch: block -> (layer, tile).
+struct GradArgs {
+    static constexpr int MAX = 33;
+    GemmArgs g[MAX];
+    int tile0[MAX + 1];  // first block of each layer
+    int n, kc;           // layers; k per split
+};
+static_assert(sizeof(GradArgs) <= 4096, "kernel arguments");
 
 __device__ inline float gelu(float z) { return 0.5f * z * (1.f + erff(z * 0.70710678118654752f)); }
 __device__ inline float gelu_d(float z) {
     return 0.5f * (1.f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
 }
 
-// Z[b][n] += bias[n]; H = gelu(Z) (H may be null for the output layer)
-__global__ void k_bias_act(float* __restrict__ Z, const float* __restrict__ bias, float* __restrict__ H, int rows,
-                           int cols) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= int64_t(rows) * cols) return;
-    const float z = Z[i] + bias[i % cols];
-    Z[i] = z;
-    if (H) H[i] = gelu(z);
-}
-
-// dZ = dH * gelu'(Z) in place on dH
-__global__ void k_gelu_back(float* __restrict__ dH, const float* __restrict__ Z, int64_t n) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) dH[i] *= gelu_d(Z[i]);
-}
-
-// column sums of X[rows][cols] in a fixed order: partial sums over chunks of
-// 256 rows, then summed in chunk order
-constexpr int COLSUM_ROWS = 32;  // rows per partial column sum
-__global__ void k_colsum_part(const float* __restrict__ X, int rows, int cols, float* __restrict__ part) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    const int chunk = blockIdx.y;
-    if (c >= cols) return;
-    float s = 0.f;
-    const int r1 = min(rows, (chunk + 1) * COLSUM_ROWS);
-    for (int r = chunk * COLSUM_ROWS; r < r1; ++r) s += X[int64_t(r) * cols + c];
-    part[int64_t(chunk) * cols + c] = s;
-}
-
-// features: in [rows][n_in] scaled to [-1, 1]; Bf [n_freq][n_in]
-__global__ void k_fourier(const float* __restrict__ X, int rows, int n_in, const float* __restrict__ Bf, int n_freq,
-                          float* __restrict__ H) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= int64_t(rows) * n_freq) return;
-    const int r = int(i / n_freq), j = int(i % n_freq);
-    float v = 0.f;
-    for (int d = 0; d < n_in; ++d) v += Bf[j * n_in + d] * X[int64_t(r) * n_in + d];
-    v *= 6.283185307179586f;
-    H[int64_t(r) * 2 * n_freq + j] = sinf(v);
-    H[int64_t(r) * 2 * n_freq + n_freq + j] = cosf(v);
-}
-
-// mean squared error over rows x n_out of (out - y), gradient into out
-__global__ void k_mse(float* __restrict__ out, const float* __restrict__ y, int64_t n, float inv_n,
-                      float* __restrict__ part) {
-    __shared__ float sh[256];
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    float e = 0.f;
-    if (i < n) {
-        const float d = out[i] - y[i];
-        e = d * d;
-        out[i] = 2.f * d * inv_n;
-    }
-    sh[threadIdx.x] = e;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
+// One T x T tile of C (T = 128 or 64) by four wavefronts of T/2 x T/2 each, on
+// v_mfma_f32_16x16x32_bf16 with B as the first operand: lane l feeds row l % 16
+// of A and of B with k = 8 (l / 16) .. + 7 and receives row l % 16 of C, columns
+// 4 (l / 16) .. + 3.  A stage of 64 k comes in as 16-byte loads, one stage ahead
+// of the products.
+template <int EPI, int T>
+__device__ __forceinline__ void gemm_tile(const GemmArgs& G, int mt, int nt, int kbeg, int kend, int z) {
+    constexpr int F = T / 32;       // 16 x 16 tiles per wavefront and side
+    constexpr int L = T * GK / 8 / 256;  // 16-byte pieces per lane, operand and stage
+    // the stages of both operands; the epilogue's transposed tile and column sums
+    constexpr int STAGE = 2 * T * GKP, EPIL = T * (T + 8) + 4 * T;
+    __shared__ __attribute__((aligned(16))) uint16_t sA[STAGE > EPIL ? STAGE : EPIL];
+    uint16_t* const sB = sA + T * GKP;
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    const int mb = mt * T, nb = nt * T;
+    const int wm = (wave >> 1) * (T / 2), wn = (wave & 1) * (T / 2);
+    const int r16 = lane & 15, kq = (lane >> 4) * 8;
+    uint4 ra[L], rb[L];
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int q = 0; q < L; ++q) {
+            const int i = t + 256 * q, row = i >> 3, kk = (i & 7) * 8;
+            // rows past the end repeat the last one; their results are not stored
+            ra[q] = *reinterpret_cast<const uint4*>(G.A + int64_t(min(mb + row, G.M - 1)) * G.lda + k0 + kk);
+            rb[q] = *reinterpret_cast<const uint4*>(G.B + int64_t(min(nb + row, G.N - 1)) * G.ldb + k0 + kk);
+        }
+    };
+    f32x4 acc[F][F];
+#pragma unroll
+    for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    fetch(kbeg);
+    for (int k0 = kbeg; k0 < kend; k0 += GK) {
+        __syncthreads();  // the previous stage has been read
+#pragma unroll
+        for (int q = 0; q < L; ++q) {
+            const int i = t + 256 * q, row = i >> 3, kk = (i & 7) * 8;
+            *reinterpret_cast<uint4*>(&sA[row * GKP + kk]) = ra[q];
+            *reinterpret_cast<uint4*>(&sB[row * GKP + kk]) = rb[q];
+        }
         __syncthreads();
+        if (k0 + GK < kend) fetch(k0 + GK);
+#pragma unroll
+        for (int kk = 0; kk < GK; kk += 32) {
+            bf16x8 a[F], b[F];
+#pragma unroll
+            for (int i = 0; i < F; ++i) a[i] = *reinterpret_cast<const bf16x8*>(&sA[(wm + i * 16 + r16) * GKP + kk + kq]);
+#pragma unroll
+            for (int j = 0; j < F; ++j) b[j] = *reinterpret_cast<const bf16x8*>(&sB[(wn + j * 16 + r16) * GKP + kk + kq]);
+#pragma unroll
+            for (int i = 0; i < F; ++i)
+#pragma unroll
+                for (int j = 0; j < F; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+        }
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+    // a lane holds row m of the tile and four neighbouring columns: results go out
+    // in 8- and 16-byte pieces, the transposed copy through LDS
+    const bool back = EPI == EPI_BACK;
+    const bool transpose = (EPI == EPI_HIDDEN || back) && G.Ht;  // uniform
+    if (back || transpose) __syncthreads();  // the stages have been read
+    uint16_t* const sT = sA;                       // [T columns][T + 8 rows]
+    float* const sum = reinterpret_cast<float*>(sA + T * (T + 8));  // column sums of the two row halves
+#pragma unroll
+    for (int j = 0; j < F; ++j) {
+        const int nl = wn + j * 16 + (lane >> 4) * 4, n0 = nb + nl;
+        float bias[4], col[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            bias[q] = (EPI == EPI_HIDDEN || EPI == EPI_OUT) && n0 + q < G.N ? G.bias[n0 + q] : 0.f;
+            col[q] = 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < F; ++i) {
+            const int ml = wm + i * 16 + r16, m = mb + ml;
+            float v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = acc[i][j][q];
+            if (EPI == EPI_OUT || EPI == EPI_PART) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (m < G.M && n0 + q < G.N) G.out[(int64_t(z) * G.M + m) * G.N + n0 + q] = v[q] + bias[q];
+                continue;
+            }
+            const bool row = m < G.M;
+            if (EPI == EPI_HIDDEN) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] += bias[q];
+                if (row && G.Z && n0 < G.ldz) *reinterpret_cast<float4*>(G.Z + int64_t(m) * G.ldz + n0) = make_float4(v[0], v[1], v[2], v[3]);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] = row && n0 + q < G.N ? gelu(v[q]) : 0.f;
+            } else {
+                const float4 zz = row && n0 < G.ldz ? *reinterpret_cast<const float4*>(G.Z + int64_t(m) * G.ldz + n0) : make_float4(0.f, 0.f, 0.f, 0.f);
+                const float zq[4] = {zz.x, zz.y, zz.z, zz.w};
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    v[q] = row && n0 + q < G.N ? v[q] * gelu_d(zq[q]) : 0.f;
+                    col[q] += v[q];
+                }
+            }
+            uint32_t h[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) h[q] = f2bf(v[q]);
+            if (G.H && row && n0 < G.ldh)  // columns past N: zero
+                *reinterpret_cast<uint2*>(G.H + int64_t(m) * G.ldh + n0) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+            if (transpose)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) sT[(nl + q) * (T + 8) + ml] = uint16_t(h[q]);
+        }
+        if (back)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+#pragma unroll
+                for (int x = 1; x < 16; x <<= 1) col[q] += __shfl_xor(col[q], x);
+                if (r16 == 0) sum[(wave >> 1) * T + nl + q] = col[q];
+            }
+    }
+    if (back || transpose) __syncthreads();
+    if (transpose)
+        for (int c = t; c < T * T / 8; c += 256) {  // rows past M: zero, up to ldt
+            const int n = c / (T / 8), m = (c - n * (T / 8)) * 8;
+            if (nb + n < G.N && mb + m < G.ldt)
+                *reinterpret_cast<uint4*>(G.Ht + int64_t(nb + n) * G.ldt + mb + m) =
+                    *reinterpret_cast<const uint4*>(&sT[n * (T + 8) + m]);
+        }
+    if (back)
+        for (int n = t; n < T; n += 256)
+            if (nb + n < G.N) G.out[int64_t(mt) * G.N + nb + n] = sum[n] + sum[T + n];
+}
+
+template <int EPI, int T>
+__global__ void __launch_bounds__(256) k_gemm(GemmArgs G) {
+    gemm_tile<EPI, T>(G, blockIdx.y, blockIdx.x, 0, G.K, 0);
+}
+
+// dW = H^T dZ of every layer: the rows split over blockIdx.y, partial products
+// summed afterwards in split order.
+__global__ void __launch_bounds__(256) k_gemm_grads(GradArgs W) {
+    int l = 0;
+    while (l + 1 < W.n && int(blockIdx.x) >= W.tile0[l + 1]) ++l;
+    const GemmArgs& G = W.g[l];
+    const int tile = blockIdx.x - W.tile0[l], tn = (G.N + 63) / 64;
+    const int kbeg = blockIdx.y * W.kc;
+    gemm_tile<EPI_PART, 64>(G, tile / tn, tile % tn, kbeg, min(G.K, kbeg + W.kc), blockIdx.y);
+}
+
+// Gradient of every parameter from its partial sums, in order: W (layer l, i)
+// from `splits` products, b from the row tiles' column sums.
+struct ReduceArgs {
+    int n;                       // layers
+    int64_t w_off[GradArgs::MAX], b_off[GradArgs::MAX];
+    int64_t w_part[GradArgs::MAX];  // first partial product of the layer
+    int64_t b_part[GradArgs::MAX];
+    int size[GradArgs::MAX], cols[GradArgs::MAX], tiles[GradArgs::MAX];
+    int splits;
+};
+// 64 parameters per workgroup, four lanes each, so that the many row tiles of a
+// bias do not run as one serial chain; the four sums are added in lane order.
+__global__ void __launch_bounds__(256) k_reduce_grads(ReduceArgs R, const float* __restrict__ wp,
+                                                      const float* __restrict__ bp, float* __restrict__ g, int64_t n) {
+    __shared__ float sh[4][64];
+    const int c = threadIdx.x & 63, part = threadIdx.x >> 6;
+    const int64_t i = int64_t(blockIdx.x) * 64 + c;
+    float s = 0.f;
+    if (i < n) {
+        int l = 0;
+        while (l + 1 < R.n && i >= R.w_off[l + 1]) ++l;
+        const bool bias = i >= R.b_off[l];
+        const int cnt = bias ? R.tiles[l] : R.splits;
+        const int64_t stride = bias ? R.cols[l] : R.size[l];
+        const float* src = bias ? bp + R.b_part[l] + (i - R.b_off[l]) : wp + R.w_part[l] + (i - R.w_off[l]);
+        const int q = (cnt + 3) / 4;
+        for (int z = part * q; z < min(cnt, part * q + q); ++z) s += src[z * stride];
+    }
+    sh[part][c] = s;
+    __syncthreads();
+    if (part == 0 && i < n) g[i] = ((sh[0][c] + sh[1][c]) + sh[2][c]) + sh[3][c];
+}
+
+// features [sin, cos](2 pi B x) as BF16, [row][ld] (columns past 2 n_freq zero)
+// and, when set, transposed [feature][ldt] with rows past the end zero; X in
+// [rows][4] scaled to [-1, 1].  A lane makes eight frequencies of one row, so
+// that rows are written in 16-byte pieces (n_freq a multiple of 8) and the
+// transposed layout a wavefront's 64 rows at a time.
+__global__ void __launch_bounds__(256) k_fourier(const float* __restrict__ X, int rows, const float* __restrict__ Bf,
+                                                 int n_freq, uint16_t* __restrict__ H, int ld,
+                                                 uint16_t* __restrict__ Ht, int ldt) {
+    const int r = blockIdx.x * 64 + (threadIdx.x & 63);
+    if (r >= max(rows, Ht ? ldt : 0)) return;
+    const bool in = r < rows;
+    float x[4] = {0.f, 0.f, 0.f, 0.f};
+    if (in)
+        for (int d = 0; d < 4; ++d) x[d] = X[int64_t(r) * 4 + d];
+    uint16_t* const row = H + int64_t(r) * ld;
+    const bool wide = n_freq % 8 == 0;
+    const int first = (blockIdx.y * 4 + (threadIdx.x >> 6)) * 8;
+    for (int j0 = first; j0 < n_freq; j0 += gridDim.y * 32) {
+        uint32_t s[4] = {}, c[4] = {};
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int j = j0 + q;
+            if (j >= n_freq) break;
+            float v = 0.f;
+            for (int d = 0; d < 4; ++d) v += Bf[j * 4 + d] * x[d];
+            v *= 6.283185307179586f;
+            const uint32_t a = in ? f2bf(sinf(v)) : 0u, b = in ? f2bf(cosf(v)) : 0u;
+            s[q / 2] |= a << (16 * (q & 1));
+            c[q / 2] |= b << (16 * (q & 1));
+            if (!wide && in) {
+                row[j] = uint16_t(a);
+                row[n_freq + j] = uint16_t(b);
+            }
+            if (Ht) {
+                Ht[int64_t(j) * ldt + r] = uint16_t(a);
+                Ht[int64_t(n_freq + j) * ldt + r] = uint16_t(b);
+            }
+        }
+        if (wide && in) {
+            *reinterpret_cast<uint4*>(row + j0) = make_uint4(s[0], s[1], s[2], s[3]);
+            *reinterpret_cast<uint4*>(row + n_freq + j0) = make_uint4(c[0], c[1], c[2], c[3]);
+        }
+    }
+    if (in && first == 0)
+        for (int j = 2 * n_freq; j < ld; ++j) row[j] = 0;
+}
+
+// Squared error of 256 rows and its gradient as BF16 (both layouts), with the
+// gradient's column sums per 256 rows.  out, y: [rows][18].
+constexpr int NO = 18;
+constexpr int MSE_ROWS = 256;
+__global__ void __launch_bounds__(256) k_mse(const float* __restrict__ out, const float* __restrict__ y, int rows,
+                                             float inv_n, uint16_t* __restrict__ D, int ld, uint16_t* __restrict__ Dt,
+                                             int ldt, float* __restrict__ col, float* __restrict__ loss) {
+    __shared__ float sh[4];
+    __shared__ float sc[4][NO];
+    const int r = blockIdx.x * MSE_ROWS + threadIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    float e = 0.f;
+    for (int k = 0; k < NO; ++k) {
+        float d = 0.f;
+        if (r < rows) {
+            d = out[int64_t(r) * NO + k] - y[int64_t(r) * NO + k];
+            e += d * d;
+            d = 2.f * d * inv_n;
+            D[int64_t(r) * ld + k] = f2bf(d);
+        }
+        if (r < ldt) Dt[int64_t(k) * ldt + r] = f2bf(d);
+        float c = d;
+        for (int s = 32; s > 0; s >>= 1) c += __shfl_xor(c, s);
+        if (lane == 0) sc[wave][k] = c;
+    }
+    for (int s = 32; s > 0; s >>= 1) e += __shfl_xor(e, s);
+    if (lane == 0) sh[wave] = e;
+    __syncthreads();
+    if (threadIdx.x < NO)
+        col[int64_t(blockIdx.x) * NO + threadIdx.x] =
+            ((sc[0][threadIdx.x] + sc[1][threadIdx.x]) + sc[2][threadIdx.x]) + sc[3][threadIdx.x];
+    if (threadIdx.x == 0) loss[blockIdx.x] = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+}
+
+// The batch's loss in FP64: the workgroups' sums added in order.
+__global__ void k_loss(const float* __restrict__ part, int n, double inv_n, double* __restrict__ dst) {
+    if (threadIdx.x != 0) return;
+    double s = 0.0;
+    for (int i = 0; i < n; ++i) s += part[i];
+    *dst = s * inv_n;
+}
+
+// One layer's place in the parameter array and its BF16 copies: Wt [out][ld_in]
+// (forward) and Wn [in][ld_out] (backward).
+struct Layers {
+    int n;
+    int64_t w_off[GradArgs::MAX], b_off[GradArgs::MAX];
+    int in[GradArgs::MAX], out[GradArgs::MAX];
+    int64_t wt[GradArgs::MAX], wn[GradArgs::MAX];  // offsets in the copies' buffer
+};
+
+__device__ inline void round_weight(const Layers& Y, int64_t i, float w, uint16_t* __restrict__ copies) {
+    int l = 0;
+    while (l + 1 < Y.n && i >= Y.w_off[l + 1]) ++l;
+    if (i >= Y.b_off[l]) return;  // biases are added in FP32
+    const int q = int(i - Y.w_off[l]), a = q / Y.out[l], b = q - a * Y.out[l];
+    const uint16_t h = f2bf(w);
+    copies[Y.wt[l] + int64_t(b) * ((Y.in[l] + 63) / 64 * 64) + a] = h;
+    copies[Y.wn[l] + int64_t(a) * ((Y.out[l] + 63) / 64 * 64) + b] = h;
+}
+
+__global__ void k_round_weights(const float* __restrict__ w, int64_t n, Layers Y, uint16_t* __restrict__ copies) {
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n) round_weight(Y, i, w[i], copies);
 }
 
 __global__ void k_adam(float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m, float* __restrict__ v,
-                       int64_t n, float lr, float b1, float b2, float eps, float c1, float c2) {
+                       int64_t n, float lr, float b1, float b2, float eps, float c1, float c2, Layers Y,
+                       uint16_t* __restrict__ copies) {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float gi = g[i];
@@ -356,7 +615,9 @@ __global__ void k_adam(float* __restrict__ w, const float* __restrict__ g, float
     const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
     m[i] = mi;
     v[i] = vi;
-    w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    w[i] = wi;
+    round_weight(Y, i, wi, copies);
 }
 
 // Output envelope e(r), r = horizontal distance from (cx, cy): piecewise
@@ -411,13 +672,28 @@ __global__ void k_sample_tile(const float* __restrict__ val, const double* __res
     for (int k = 0; k < 18; ++k) Y[int64_t(r) * 18 + k] = v[k] * inv_scale[k] * ie;
 }
 
-// raw (x, y, z, t) -> scaled inputs
-__global__ void k_scale_in(const double* __restrict__ raw, int rows, const double* __restrict__ lo,
-                           const double* __restrict__ hi, float* __restrict__ X) {
+// raw (x, y, z, t) -> scaled inputs, the time retarded; t from t0 + tix dt when
+// tix is given (q then holds x, y, z).  No contraction: the values the host rounds.
+__global__ void k_inputs(const double* __restrict__ q, const int32_t* __restrict__ tix, double t0, double dt, int rows,
+                         const double* __restrict__ lo, const double* __restrict__ hi, Envelope E,
+                         float* __restrict__ X) {
+#pragma clang fp contract(off)
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= rows) return;
-    for (int d = 0; d < 4; ++d)
-        X[int64_t(r) * 4 + d] = float(2.0 * (raw[int64_t(r) * 4 + d] - lo[d]) / (hi[d] - lo[d]) - 1.0);
+    const double* p = q + int64_t(r) * (tix ? 3 : 4);
+    const double t = tix ? t0 + tix[r] * dt : p[3];
+    const double in[4] = {p[0], p[1], p[2], retarded_time(E, p[0], p[1], t)};
+    for (int d = 0; d < 4; ++d) X[int64_t(r) * 4 + d] = float(2.0 * (in[d] - lo[d]) / (hi[d] - lo[d]) - 1.0);
+}
+
+// network outputs -> values: times the output scale and the envelope
+__global__ void k_outputs(const float* __restrict__ out, const double* __restrict__ q, int stride, int rows,
+                          const double* __restrict__ scale, Envelope E, float* __restrict__ y) {
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= int64_t(rows) * NO) return;
+    const int64_t r = i / NO;
+    const double e = envelope_at(E, q[r * stride], q[r * stride + 1]);
+    y[i] = float(out[i] * scale[i - r * NO] * e);
 }
 
 }  // namespace sur
@@ -430,7 +706,7 @@ struct gfx_mlp {
     std::vector<int64_t> w_off, b_off;       // offsets in the flat parameter array
     int64_t n_params = 0;
     gfx::DevBuf<float> w, g, m, v, Bf;
-    gfx::DevBuf<double> lo, hi;
+    gfx::DevBuf<double> lo, hi, scale;
     gfx::DevBuf<float> inv_scale;
     std::vector<double> h_scale;
     // output envelope (knots on the host and the device)
@@ -441,11 +717,24 @@ struct gfx_mlp {
         return gfx::sur::Envelope{device ? env.p : h_env.data(), int(h_env.size()), env_cx, env_cy, env_rmax,
                                   slowness};
     }
-    // activations for up to cap rows
+    // BF16 copies of the weights, both ways, for every layer
+    gfx::sur::Layers layers{};
+    gfx::DevBuf<uint16_t> copies;
+    // inputs and outputs of a call, and the activations on the way (grown to the
+    // largest chunk or batch used, freed with the network)
     int cap = 0;
-    gfx::DevBuf<float> X, H0, Y, work, part, lossp;
-    std::vector<gfx::DevBuf<float>> Z, H;    // per hidden layer
-    gfx::DevBuf<float> out, dA, dB;
+    gfx::DevBuf<float> X, out;
+    gfx::DevBuf<uint16_t> ha, hb;      // activations of two consecutive layers
+    gfx::DevBuf<double> raw;
+    gfx::DevBuf<int32_t> tix;
+    gfx::DevBuf<float> y;
+    gfx::DevBuf<uint8_t> policy;       // a query's answer per region
+    gfx::DevBuf<int> count;            // points the judge answered
+    // training: per layer pre-activations, transposed activations and gradients
+    int train_cap = 0;
+    gfx::DevBuf<float> Y, Z, w_part, b_part, lossp;
+    gfx::DevBuf<uint16_t> H, Ht, D, Dt, dout;
+    gfx::DevBuf<double> losses;
     int64_t adam_t = 0;
     hipStream_t stream = nullptr;
     ~gfx_mlp() {
@@ -457,112 +746,224 @@ namespace gfx {
 namespace sur {
 namespace {
 
+constexpr int CHUNK = 131072;  // rows per pass of a forward call
+
+// Widest padded layer input / output.
+int wide(const gfx_mlp& M) { return std::max(pad64(M.n_feat), pad64(M.cfg.width)); }
+
 void ensure_rows(gfx_mlp& M, int rows) {
     if (rows <= M.cap) return;
-    const int cap = ((rows + 255) / 256) * 256;
+    const int cap = (rows + 255) / 256 * 256;
+    GFX_HIP(hipStreamSynchronize(M.stream));  // the old buffers may still be in use
+    M.cap = 0;
     M.X.alloc(size_t(cap) * 4);
-    M.H0.alloc(size_t(cap) * M.n_feat);
-    M.Y.alloc(size_t(cap) * M.cfg.n_out);
-    const int d = M.cfg.depth, wdt = M.cfg.width;
-    M.Z.clear();
-    M.H.clear();
-    M.Z.resize(d);
-    M.H.resize(d);
-    for (int l = 0; l < d; ++l) {
-        M.Z[l].alloc(size_t(cap) * wdt);
-        M.H[l].alloc(size_t(cap) * wdt);
-    }
-    M.out.alloc(size_t(cap) * M.cfg.n_out);
-    M.dA.alloc(size_t(cap) * std::max(wdt, M.n_feat));
-    M.dB.alloc(size_t(cap) * std::max(wdt, M.n_feat));
-    M.part.alloc(size_t(cap / sur::COLSUM_ROWS + 1) * std::max(wdt, 64));
-    M.lossp.alloc(size_t(cap) * M.cfg.n_out / 256 + 1);
+    M.out.alloc(size_t(cap) * NO);
+    M.y.alloc(size_t(cap) * NO);
+    M.raw.alloc(size_t(cap) * 4);
+    M.tix.alloc(size_t(cap));
+    M.ha.alloc(size_t(cap) * wide(M));
+    M.hb.alloc(size_t(cap) * wide(M));
+    M.ha.zero(M.stream);  // features past 2 n_freq stay zero
+    M.hb.zero(M.stream);
     M.cap = cap;
 }
 
-// C[M][N] = op(A) op(B), split over K when the output grid is small
-template <bool TA, bool TB>
-void gemm(gfx_mlp& Mm, const float* A, int lda, const float* B, int ldb, float* C, int ldc, int M, int N, int K) {
-    const int gx = (N + sur::GT - 1) / sur::GT, gy = (M + sur::GT - 1) / sur::GT;
-    int splits = 1;
-    while (gx * gy * splits < 256 && K / (splits * 2) >= 256) splits *= 2;
-    if (splits == 1) {
-        sur::k_gemm_lds<TA, TB><<<dim3(gx, gy, 1), 256, 0, Mm.stream>>>(A, lda, B, ldb, C, ldc, M, N, K, K);
-        return;
-    }
-    const int kc = ((K + splits - 1) / splits + sur::GK - 1) / sur::GK * sur::GK;
-    const size_t need = size_t(splits) * M * ldc;
-    if (Mm.work.n < need) {
-        GFX_HIP(hipStreamSynchronize(Mm.stream));  // the old buffer may still be read
-        Mm.work.alloc(need);
-    }
-    sur::k_gemm_lds<TA, TB><<<dim3(gx, gy, splits), 256, 0, Mm.stream>>>(A, lda, B, ldb, Mm.work.p, ldc, M, N, K,
-                                                                         kc);
-    const int64_t n = int64_t(M) * ldc;
-    sur::k_sum_splits<<<int((n + 255) / 256), 256, 0, Mm.stream>>>(Mm.work.p, splits, n, C);
+// Row splits of the weight gradients: about a thousand workgroups, at least 256 rows each.
+int grad_splits(const gfx_mlp& M, int rows) {
+    int tiles = 0;
+    for (size_t l = 0; l < M.lin_in.size(); ++l) tiles += ((M.lin_in[l] + 63) / 64) * ((M.lin_out[l] + 63) / 64);
+    return std::max(1, std::min((1024 + tiles - 1) / tiles, rows / 256));
 }
 
-void colsum(gfx_mlp& M, const float* X, int rows, int cols, float* dst) {
-    const int chunks = (rows + sur::COLSUM_ROWS - 1) / sur::COLSUM_ROWS;
-    sur::k_colsum_part<<<dim3((cols + 63) / 64, chunks), 64, 0, M.stream>>>(X, rows, cols, M.part.p);
-    sur::k_sum_splits<<<(cols + 255) / 256, 256, 0, M.stream>>>(M.part.p, chunks, cols, dst);
+// Buffers of forward and backward over one batch of rows.
+struct Train {
+    int ldt;                        // padded rows
+    std::vector<int64_t> z, h, ht;  // per layer input l: offsets of Z (l >= 1), H, Ht
+    std::vector<int64_t> dt;        // per layer output: offset of Dt
+};
+Train train_layout(const gfx_mlp& M, int rows) {
+    Train T;
+    T.ldt = pad64(rows);
+    int64_t z = 0, h = 0, ht = 0, dt = 0;
+    for (size_t l = 0; l < M.lin_in.size(); ++l) {
+        T.z.push_back(z);
+        T.h.push_back(h);
+        T.ht.push_back(ht);
+        T.dt.push_back(dt);
+        z += int64_t(T.ldt) * pad64(M.lin_in[l]);
+        h += int64_t(T.ldt) * pad64(M.lin_in[l]);
+        ht += int64_t(T.ldt) * M.lin_in[l];
+        dt += int64_t(T.ldt) * M.lin_out[l];
+    }
+    T.z.push_back(z);
+    T.h.push_back(h);
+    T.ht.push_back(ht);
+    T.dt.push_back(dt);
+    return T;
+}
+
+void ensure_train(gfx_mlp& M, int rows) {
+    ensure_rows(M, rows);
+    if (rows == M.train_cap) return;  // leading dimensions belong to the batch size
+    GFX_HIP(hipStreamSynchronize(M.stream));
+    M.train_cap = 0;
+    const Train T = train_layout(M, rows);
+    M.Y.alloc(size_t(rows) * NO);
+    M.Z.alloc(T.z.back());
+    M.H.alloc(T.h.back());
+    M.Ht.alloc(T.ht.back());
+    M.D.alloc(size_t(2) * T.ldt * pad64(M.cfg.width));
+    M.Dt.alloc(T.dt.back());
+    M.H.zero(M.stream);  // padding columns stay zero
+    M.D.zero(M.stream);
+    M.w_part.alloc(size_t(grad_splits(M, rows)) * M.n_params);
+    M.b_part.alloc(size_t(T.ldt / 64) * (size_t(M.cfg.width) * M.cfg.depth + NO));
+    M.dout.alloc(size_t(T.ldt) * pad64(NO));
+    M.dout.zero(M.stream);
+    M.lossp.alloc((rows + MSE_ROWS - 1) / MSE_ROWS);
+    M.train_cap = rows;
+}
+
+// One product, 128 x 128 tiles where they give every CU two workgroups, else 64 x 64.
+template <int EPI>
+int gemm(gfx_mlp& M, const GemmArgs& G) {
+    const int big = ((G.M + 127) / 128) * ((G.N + 127) / 128);
+    if (big >= 512) {
+        k_gemm<EPI, 128><<<dim3((G.N + 127) / 128, (G.M + 127) / 128), 256, 0, M.stream>>>(G);
+        return 128;
+    }
+    k_gemm<EPI, 64><<<dim3((G.N + 63) / 64, (G.M + 63) / 64), 256, 0, M.stream>>>(G);
+    return 64;
+}
+
+void features(gfx_mlp& M, int rows, uint16_t* H, uint16_t* Ht, int ldt) {
+    const int nf = M.cfg.n_freq;
+    const int n = Ht ? ldt : rows;
+    k_fourier<<<dim3((n + 63) / 64, (nf + 31) / 32), 256, 0, M.stream>>>(M.X.p, rows, M.Bf.p, nf, H,
+                                                                                     pad64(M.n_feat), Ht, ldt);
 }
 
 // forward of rows scaled inputs in M.X; output (scaled) in M.out
 void forward(gfx_mlp& M, int rows) {
-    const int nf = M.cfg.n_freq;
-    sur::k_fourier<<<int((int64_t(rows) * nf + 255) / 256), 256, 0, M.stream>>>(M.X.p, rows, 4, M.Bf.p, nf, M.H0.p);
-    const float* in = M.H0.p;
-    int in_w = M.n_feat;
+    uint16_t *in = M.ha.p, *next = M.hb.p;
+    features(M, rows, in, nullptr, 0);
     const int d = M.cfg.depth;
-    for (int l = 0; l < d; ++l) {
-        const int ow = M.lin_out[l];
-        gemm<false, false>(M, in, in_w, M.w.p + M.w_off[l], ow, M.Z[l].p, ow, rows, ow, in_w);
-        sur::k_bias_act<<<int((int64_t(rows) * ow + 255) / 256), 256, 0, M.stream>>>(
-            M.Z[l].p, M.w.p + M.b_off[l], M.H[l].p, rows, ow);
-        in = M.H[l].p;
-        in_w = ow;
-    }
-    const int no = M.cfg.n_out;
-    gemm<false, false>(M, in, in_w, M.w.p + M.w_off[d], no, M.out.p, no, rows, no, in_w);
-    sur::k_bias_act<<<int((int64_t(rows) * no + 255) / 256), 256, 0, M.stream>>>(M.out.p, M.w.p + M.b_off[d],
-                                                                                   nullptr, rows, no);
-}
-
-// loss (mean over rows x n_out of squared scaled error) and gradient into M.g
-double backward(gfx_mlp& M, int rows) {
-    const int no = M.cfg.n_out, d = M.cfg.depth;
-    const int64_t n = int64_t(rows) * no;
-    const int nb = int((n + 255) / 256);
-    sur::k_mse<<<nb, 256, 0, M.stream>>>(M.out.p, M.Y.p, n, 1.f / float(n), M.lossp.p);
-    std::vector<float> hp(nb);
-    GFX_HIP(hipMemcpyAsync(hp.data(), M.lossp.p, nb * 4, hipMemcpyDeviceToHost, M.stream));
-    // output layer
-    const float* dOut = M.out.p;
-    const float* Hl = M.H[d - 1].p;
-    const int wl = M.lin_in[d];
-    gemm<true, false>(M, Hl, wl, dOut, no, M.g.p + M.w_off[d], no, wl, no, rows);
-    colsum(M, dOut, rows, no, M.g.p + M.b_off[d]);
-    // dH_{d-1} = dOut W_d^T
-    float* dH = M.dA.p;
-    float* spare = M.dB.p;
-    gemm<false, true>(M, dOut, no, M.w.p + M.w_off[d], no, dH, wl, rows, wl, no);
-    for (int l = d - 1; l >= 0; --l) {
-        const int ow = M.lin_out[l], iw = M.lin_in[l];
-        sur::k_gelu_back<<<int((int64_t(rows) * ow + 255) / 256), 256, 0, M.stream>>>(dH, M.Z[l].p,
-                                                                                        int64_t(rows) * ow);
-        const float* Hin = (l == 0) ? M.H0.p : M.H[l - 1].p;
-        gemm<true, false>(M, Hin, iw, dH, ow, M.g.p + M.w_off[l], ow, iw, ow, rows);
-        colsum(M, dH, rows, ow, M.g.p + M.b_off[l]);
-        if (l > 0) {
-            gemm<false, true>(M, dH, ow, M.w.p + M.w_off[l], ow, spare, iw, rows, iw, ow);
-            std::swap(dH, spare);
+    for (int l = 0; l <= d; ++l) {
+        GemmArgs G{};
+        G.A = in;
+        G.lda = G.ldb = G.K = pad64(M.lin_in[l]);
+        G.B = M.copies.p + M.layers.wt[l];
+        G.M = rows;
+        G.N = M.lin_out[l];
+        G.bias = M.w.p + M.b_off[l];
+        if (l == d) {
+            G.out = M.out.p;
+            gemm<EPI_OUT>(M, G);
+        } else {
+            G.H = next;
+            G.ldh = pad64(M.lin_out[l]);
+            gemm<EPI_HIDDEN>(M, G);
+            std::swap(in, next);
         }
     }
-    GFX_HIP(hipStreamSynchronize(M.stream));
-    double loss = 0.0;
-    for (float v : hp) loss += v;
-    return loss / double(n);
+    GFX_HIP(hipGetLastError());
+}
+
+// Forward and backward of the batch in M.X, M.Y: gradient into M.g, loss (mean
+// over rows x n_out of the squared scaled error) into *loss on the device.
+void gradient(gfx_mlp& M, int rows, double* loss) {
+    const Train T = train_layout(M, rows);
+    const int d = M.cfg.depth;
+    features(M, rows, M.H.p, M.Ht.p, T.ldt);
+    for (int l = 0; l <= d; ++l) {
+        GemmArgs G{};
+        G.A = M.H.p + T.h[l];
+        G.lda = G.ldb = G.K = pad64(M.lin_in[l]);
+        G.B = M.copies.p + M.layers.wt[l];
+        G.M = rows;
+        G.N = M.lin_out[l];
+        G.bias = M.w.p + M.b_off[l];
+        if (l == d) {
+            G.out = M.out.p;
+            gemm<EPI_OUT>(M, G);
+        } else {
+            G.Z = M.Z.p + T.z[l + 1];
+            G.ldz = pad64(M.lin_out[l]);
+            G.H = M.H.p + T.h[l + 1];
+            G.ldh = pad64(M.lin_out[l]);
+            G.Ht = M.Ht.p + T.ht[l + 1];
+            G.ldt = T.ldt;
+            gemm<EPI_HIDDEN>(M, G);
+        }
+    }
+    // bias sums: one row per row tile, layer after layer
+    ReduceArgs R{};
+    R.n = d + 1;
+    R.splits = grad_splits(M, rows);
+    int64_t bp = 0, wp = 0;
+    uint16_t *dcur = M.D.p, *dnext = M.D.p + int64_t(T.ldt) * pad64(M.cfg.width);
+    const int64_t n = int64_t(rows) * NO;
+    const int mb = (rows + MSE_ROWS - 1) / MSE_ROWS;
+    k_mse<<<mb, MSE_ROWS, 0, M.stream>>>(M.out.p, M.Y.p, rows, 1.f / float(n), M.dout.p, pad64(NO), M.Dt.p + T.dt[d],
+                                         T.ldt, M.b_part.p, M.lossp.p);
+    k_loss<<<1, 64, 0, M.stream>>>(M.lossp.p, mb, 1.0 / double(n), loss);
+    R.b_part[d] = 0;
+    R.tiles[d] = mb;
+    bp = int64_t(mb) * NO;
+    const uint16_t* grad = M.dout.p;
+    for (int l = d; l >= 1; --l) {  // dZ_{l-1} = (dZ_l W_l^T) gelu'(Z_{l-1})
+        GemmArgs G{};
+        G.A = grad;
+        G.lda = G.ldb = G.K = pad64(M.lin_out[l]);
+        G.B = M.copies.p + M.layers.wn[l];
+        G.M = rows;
+        G.N = M.lin_in[l];
+        G.Z = M.Z.p + T.z[l];
+        G.ldz = pad64(M.lin_in[l]);
+        G.H = l > 1 ? dcur : nullptr;
+        G.ldh = pad64(M.lin_in[l]);
+        G.Ht = M.Dt.p + T.dt[l - 1];
+        G.ldt = T.ldt;
+        G.out = M.b_part.p + bp;
+        const int tile = gemm<EPI_BACK>(M, G);
+        R.b_part[l - 1] = bp;
+        R.tiles[l - 1] = (rows + tile - 1) / tile;
+        bp += int64_t(R.tiles[l - 1]) * M.lin_in[l];
+        grad = dcur;
+        std::swap(dcur, dnext);
+    }
+    GradArgs W{};
+    W.n = d + 1;
+    W.kc = (T.ldt / 64 + R.splits - 1) / R.splits * 64;
+    R.splits = (T.ldt + W.kc - 1) / W.kc;
+    int tiles = 0;
+    for (int l = 0; l <= d; ++l) {
+        GemmArgs& G = W.g[l];
+        G.A = M.Ht.p + T.ht[l];
+        G.B = M.Dt.p + T.dt[l];
+        G.lda = G.ldb = G.K = T.ldt;
+        G.M = M.lin_in[l];
+        G.N = M.lin_out[l];
+        G.out = M.w_part.p + wp;
+        W.tile0[l] = tiles;
+        tiles += ((G.M + 63) / 64) * ((G.N + 63) / 64);
+        R.w_off[l] = M.w_off[l];
+        R.b_off[l] = M.b_off[l];
+        R.w_part[l] = wp;
+        R.size[l] = G.M * G.N;
+        R.cols[l] = G.N;
+        wp += int64_t(R.splits) * R.size[l];
+    }
+    W.tile0[d + 1] = tiles;
+    k_gemm_grads<<<dim3(tiles, R.splits), 256, 0, M.stream>>>(W);
+    k_reduce_grads<<<int((M.n_params + 63) / 64), 256, 0, M.stream>>>(R, M.w_part.p, M.b_part.p, M.g.p, M.n_params);
+    GFX_HIP(hipGetLastError());
+}
+
+// BF16 copies of the weights after they changed outside Adam.
+void round_weights(gfx_mlp& M) {
+    k_round_weights<<<int((M.n_params + 255) / 256), 256, 0, M.stream>>>(M.w.p, M.n_params, M.layers, M.copies.p);
+    GFX_HIP(hipGetLastError());
 }
 
 void adam(gfx_mlp& M, float lr) {
@@ -570,7 +971,8 @@ void adam(gfx_mlp& M, float lr) {
     const float b1 = M.cfg.beta1, b2 = M.cfg.beta2;
     const float c1 = 1.f - std::pow(b1, float(M.adam_t)), c2 = 1.f - std::pow(b2, float(M.adam_t));
     sur::k_adam<<<int((M.n_params + 255) / 256), 256, 0, M.stream>>>(M.w.p, M.g.p, M.m.p, M.v.p, M.n_params,
-                                                                      lr, b1, b2, M.cfg.eps, c1, c2);
+                                                                      lr, b1, b2, M.cfg.eps, c1, c2, M.layers,
+                                                                      M.copies.p);
 }
 
 }  // namespace
@@ -685,21 +1087,18 @@ extern "C" gfx_status gfx_green_interpolate(const gfx_green* g, int n, const dou
     return guarded([&] {
         require(g && xyz && tix && out && n >= 0, "null argument");
         if (n == 0) return;
-        DevBuf<double> q;
-        DevBuf<int32_t> t, c;
-        DevBuf<float> o;
-        q.alloc(size_t(n) * 3);
-        t.alloc(n);
-        o.alloc(size_t(n) * 18);
-        if (cell) c.alloc(n);
-        GFX_HIP(hipMemcpy(q.p, xyz, size_t(n) * 24, hipMemcpyHostToDevice));
-        GFX_HIP(hipMemcpy(t.p, tix, size_t(n) * 4, hipMemcpyHostToDevice));
-        sur::k_judge<<<(n + 127) / 128, 128, 0, g->stream>>>(sur::judge_args(*g), n, q.p, t.p, nullptr, 1, o.p,
-                                                              cell ? c.p : nullptr);
+        std::lock_guard<std::mutex> lock(g->work_mu);
+        gfx_green::Work& w = g->work;
+        w.fit(n);
+        GFX_HIP(hipMemcpyAsync(w.q.p, xyz, size_t(n) * 24, hipMemcpyHostToDevice, g->stream));
+        GFX_HIP(hipMemcpyAsync(w.t.p, tix, size_t(n) * 4, hipMemcpyHostToDevice, g->stream));
+        sur::k_judge<<<sur::judge_blocks(n), 64 * sur::JQ, 0, g->stream>>>(
+            sur::judge_args(*g), n, sur::judge_q(n), w.q.p, w.t.p, nullptr, 1, w.o.p, cell ? w.c.p : nullptr, nullptr);
         GFX_HIP(hipGetLastError());
+        GFX_HIP(hipMemcpyAsync(out, w.o.p, size_t(n) * 18 * 4, hipMemcpyDeviceToHost, g->stream));
+        if (cell) GFX_HIP(hipMemcpyAsync(cell, w.c.p, size_t(n) * 4, hipMemcpyDeviceToHost, g->stream));
         GFX_HIP(hipStreamSynchronize(g->stream));
-        GFX_HIP(hipMemcpy(out, o.p, size_t(n) * 18 * 4, hipMemcpyDeviceToHost));
-        if (cell) GFX_HIP(hipMemcpy(cell, c.p, size_t(n) * 4, hipMemcpyDeviceToHost));
+        w.trim();
     });
 }
 
@@ -836,9 +1235,28 @@ extern "C" gfx_status gfx_mlp_create(const gfx_mlp_config* cfg, const double* in
         M->m.zero(M->stream);
         M->v.zero(M->stream);
         M->Bf.upload(hb);
+        {
+            int64_t at = 0;
+            M->layers.n = int(M->lin_in.size());
+            for (int l = 0; l < M->layers.n; ++l) {
+                sur::Layers& Y = M->layers;
+                Y.w_off[l] = M->w_off[l];
+                Y.b_off[l] = M->b_off[l];
+                Y.in[l] = M->lin_in[l];
+                Y.out[l] = M->lin_out[l];
+                Y.wt[l] = at;
+                at += int64_t(Y.out[l]) * sur::pad64(Y.in[l]);
+                Y.wn[l] = at;
+                at += int64_t(Y.in[l]) * sur::pad64(Y.out[l]);
+            }
+            M->copies.alloc(at);
+            M->copies.zero(M->stream);  // padding stays zero
+            sur::round_weights(*M);
+        }
         M->lo.upload(std::vector<double>(in_lo, in_lo + 4));
         M->hi.upload(std::vector<double>(in_hi, in_hi + 4));
         M->h_scale.assign(out_scale, out_scale + 18);
+        M->scale.upload(M->h_scale);
         std::vector<float> inv(18);
         for (int k = 0; k < 18; ++k) {
             require(out_scale[k] > 0, "output scales must be > 0");
@@ -875,6 +1293,7 @@ extern "C" gfx_status gfx_mlp_set_params(gfx_mlp* m, const float* w, size_t n) {
         require(m && w && n == size_t(m->n_params), "parameter buffer must hold n_params floats");
         GFX_HIP(hipStreamSynchronize(m->stream));
         GFX_HIP(hipMemcpy(m->w.p, w, n * 4, hipMemcpyHostToDevice));
+        sur::round_weights(*m);
     });
 }
 
@@ -901,47 +1320,24 @@ extern "C" gfx_status gfx_mlp_set_envelope(gfx_mlp* m, double cx, double cy, dou
     });
 }
 
-namespace gfx {
-namespace sur {
-namespace {
-// raw (x, y, z, t) rows with t replaced by the network's time input
-std::vector<double> network_inputs(const gfx_mlp& m, const double* x, int rows) {
-    std::vector<double> v(x, x + size_t(rows) * 4);
-    const Envelope E = m.envelope(false);
-    if (E.slowness != 0.0)
-        for (int r = 0; r < rows; ++r) v[size_t(r) * 4 + 3] = retarded_time(E, v[size_t(r) * 4], v[size_t(r) * 4 + 1], v[size_t(r) * 4 + 3]);
-    return v;
-}
-}  // namespace
-}  // namespace sur
-}  // namespace gfx
-
 // inputs raw (x, y, z, t) [n][4] FP64; outputs unscaled [n][18]
 extern "C" gfx_status gfx_mlp_forward(gfx_mlp* m, int n, const double* x, float* y) {
     return guarded([&] {
         require(m && x && y && n >= 0, "null argument");
-        const int chunk = 65536;
-        DevBuf<double> raw;
-        raw.alloc(size_t(std::min(n, chunk)) * 4 + 4);
-        std::vector<float> ho;
-        const sur::Envelope E = m->envelope(false);
-        for (int b = 0; b < n; b += chunk) {
-            const int rows = std::min(chunk, n - b);
+        const sur::Envelope E = m->envelope(true);
+        for (int b = 0; b < n; b += sur::CHUNK) {
+            const int rows = std::min(sur::CHUNK, n - b);
             sur::ensure_rows(*m, rows);
-            const std::vector<double> xin = sur::network_inputs(*m, x + size_t(b) * 4, rows);  // lives past the sync
-            GFX_HIP(hipMemcpyAsync(raw.p, xin.data(), size_t(rows) * 32, hipMemcpyHostToDevice, m->stream));
-            sur::k_scale_in<<<(rows + 255) / 256, 256, 0, m->stream>>>(raw.p, rows, m->lo.p, m->hi.p, m->X.p);
+            GFX_HIP(hipMemcpyAsync(m->raw.p, x + size_t(b) * 4, size_t(rows) * 32, hipMemcpyHostToDevice, m->stream));
+            sur::k_inputs<<<(rows + 255) / 256, 256, 0, m->stream>>>(m->raw.p, nullptr, 0.0, 0.0, rows, m->lo.p, m->hi.p,
+                                                                     E, m->X.p);
             sur::forward(*m, rows);
-            ho.resize(size_t(rows) * 18);
-            GFX_HIP(hipMemcpyAsync(ho.data(), m->out.p, ho.size() * 4, hipMemcpyDeviceToHost, m->stream));
-            GFX_HIP(hipStreamSynchronize(m->stream));
-            for (int r = 0; r < rows; ++r) {
-                const double* xr = x + (size_t(b) + r) * 4;
-                const double e = sur::envelope_at(E, xr[0], xr[1]);
-                for (int k = 0; k < 18; ++k)
-                    y[(size_t(b) + r) * 18 + k] = float(ho[size_t(r) * 18 + k] * m->h_scale[k] * e);
-            }
+            sur::k_outputs<<<(rows * sur::NO + 255) / 256, 256, 0, m->stream>>>(m->out.p, m->raw.p, 4, rows, m->scale.p,
+                                                                               E, m->y.p);
+            GFX_HIP(hipGetLastError());
+            GFX_HIP(hipMemcpyAsync(y + size_t(b) * 18, m->y.p, size_t(rows) * 72, hipMemcpyDeviceToHost, m->stream));
         }
+        GFX_HIP(hipStreamSynchronize(m->stream));
     });
 }
 
@@ -951,11 +1347,9 @@ extern "C" gfx_status gfx_mlp_gradient(gfx_mlp* m, int n, const double* x, const
                                        double* loss) {
     return guarded([&] {
         require(m && x && y && grad && loss && n >= 1, "null argument");
-        sur::ensure_rows(*m, n);
-        DevBuf<double> raw;
-        raw.alloc(size_t(n) * 4);
-        const std::vector<double> xin = sur::network_inputs(*m, x, n);
-        GFX_HIP(hipMemcpy(raw.p, xin.data(), size_t(n) * 32, hipMemcpyHostToDevice));
+        sur::ensure_train(*m, n);
+        GFX_HIP(hipStreamSynchronize(m->stream));
+        GFX_HIP(hipMemcpy(m->raw.p, x, size_t(n) * 32, hipMemcpyHostToDevice));
         std::vector<float> ys(size_t(n) * 18);
         const sur::Envelope E = m->envelope(false);
         for (int r = 0; r < n; ++r) {
@@ -963,9 +1357,12 @@ extern "C" gfx_status gfx_mlp_gradient(gfx_mlp* m, int n, const double* x, const
             for (int k = 0; k < 18; ++k) ys[size_t(r) * 18 + k] = float(y[size_t(r) * 18 + k] / (m->h_scale[k] * e));
         }
         GFX_HIP(hipMemcpy(m->Y.p, ys.data(), ys.size() * 4, hipMemcpyHostToDevice));
-        sur::k_scale_in<<<(n + 255) / 256, 256, 0, m->stream>>>(raw.p, n, m->lo.p, m->hi.p, m->X.p);
-        sur::forward(*m, n);
-        *loss = sur::backward(*m, n);
+        if (m->losses.n < 1) m->losses.alloc(1);
+        sur::k_inputs<<<(n + 255) / 256, 256, 0, m->stream>>>(m->raw.p, nullptr, 0.0, 0.0, n, m->lo.p, m->hi.p,
+                                                              m->envelope(true), m->X.p);
+        sur::gradient(*m, n, m->losses.p);
+        GFX_HIP(hipStreamSynchronize(m->stream));
+        GFX_HIP(hipMemcpy(loss, m->losses.p, sizeof(double), hipMemcpyDeviceToHost));
         GFX_HIP(hipMemcpy(grad, m->g.p, size_t(m->n_params) * 4, hipMemcpyDeviceToHost));
     });
 }
@@ -979,28 +1376,31 @@ extern "C" gfx_status gfx_mlp_train(gfx_mlp* m, const gfx_green* g, double t0, d
         require(m && g && loss && iters >= 0, "null argument");
         const int rows = m->cfg.batch;
         require(rows >= 64, "batch must be >= 64");
-        sur::ensure_rows(*m, rows);
+        sur::ensure_train(*m, rows);
         GFX_HIP(hipStreamSynchronize(g->stream));
-        double tail = 0.0;
-        int nt = 0;
+        if (m->losses.n < size_t(std::max(iters, 1))) {
+            GFX_HIP(hipStreamSynchronize(m->stream));
+            m->losses.alloc(std::max(iters, 1));
+        }
         const sur::Envelope E = m->envelope(true);
         const double lr0 = m->cfg.lr, lr1 = m->cfg.lr_final;
         for (int it = 0; it < iters; ++it) {
             sur::k_sample_tile<<<(rows + 255) / 256, 256, 0, m->stream>>>(
                 g->val.p, g->xyz.p, g->n_node, g->n_time, t0, dt, m->lo.p, m->hi.p, m->inv_scale.p, E,
                 seed * 0x9E3779B97F4A7C15ULL + uint64_t(it), rows, m->X.p, m->Y.p);
-            sur::forward(*m, rows);
-            const double l = sur::backward(*m, rows);
+            sur::gradient(*m, rows, m->losses.p + it);
             // cosine decay from lr to lr_final over this call
             const double ph = iters > 1 ? double(it) / double(iters - 1) : 1.0;
             sur::adam(*m, float(lr1 + 0.5 * (lr0 - lr1) * (1.0 + std::cos(3.14159265358979323846 * ph))));
-            if (it >= iters - std::max(1, iters / 10)) {
-                tail += l;
-                ++nt;
-            }
         }
         GFX_HIP(hipStreamSynchronize(m->stream));
-        *loss = nt ? tail / nt : 0.0;
+        const int nt = iters > 0 ? std::max(1, iters / 10) : 0;
+        std::vector<double> tail(nt);
+        if (nt)
+            GFX_HIP(hipMemcpy(tail.data(), m->losses.p + (iters - nt), nt * sizeof(double), hipMemcpyDeviceToHost));
+        double sum = 0.0;
+        for (double l : tail) sum += l;
+        *loss = nt ? sum / nt : 0.0;
     });
 }
 
@@ -1017,51 +1417,33 @@ extern "C" gfx_status gfx_surrogate_query(gfx_mlp* m, const gfx_green* g, const 
             *n_fallback = 0;
             return;
         }
-        std::vector<double> x4(size_t(n) * 4);
-        for (int i = 0; i < n; ++i) {
-            for (int d = 0; d < 3; ++d) x4[size_t(i) * 4 + d] = xyz[size_t(i) * 3 + d];
-            x4[size_t(i) * 4 + 3] = t0 + tix[i] * dt;
+        const size_t nreg = size_t(g->n_cell) * n_window;
+        GFX_HIP(hipStreamSynchronize(g->stream));  // the tile's values are in place
+        if (m->policy.n < nreg) {
+            GFX_HIP(hipStreamSynchronize(m->stream));
+            m->policy.alloc(nreg);
         }
-        std::vector<float> mo(size_t(n) * 18);
-        {
-            const gfx_status st = gfx_mlp_forward(m, n, x4.data(), mo.data());
-            if (st != GFX_OK) throw Error(st, gfx_last_error());
+        if (m->count.n < 1) m->count.alloc(1);
+        GFX_HIP(hipMemcpyAsync(m->policy.p, fallback, nreg, hipMemcpyHostToDevice, m->stream));
+        m->count.zero(m->stream);
+        const sur::Envelope E = m->envelope(true);
+        for (int b = 0; b < n; b += sur::CHUNK) {
+            const int rows = std::min(sur::CHUNK, n - b);
+            sur::ensure_rows(*m, rows);
+            GFX_HIP(hipMemcpyAsync(m->raw.p, xyz + size_t(b) * 3, size_t(rows) * 24, hipMemcpyHostToDevice, m->stream));
+            GFX_HIP(hipMemcpyAsync(m->tix.p, tix + b, size_t(rows) * 4, hipMemcpyHostToDevice, m->stream));
+            sur::k_inputs<<<(rows + 255) / 256, 256, 0, m->stream>>>(m->raw.p, m->tix.p, t0, dt, rows, m->lo.p, m->hi.p, E,
+                                                                     m->X.p);
+            sur::forward(*m, rows);
+            sur::k_outputs<<<(rows * sur::NO + 255) / 256, 256, 0, m->stream>>>(m->out.p, m->raw.p, 3, rows, m->scale.p,
+                                                                               E, m->y.p);
+            // the judge's answers, and zeros, over the network's
+            sur::k_judge<<<sur::judge_blocks(rows), 64 * sur::JQ, 0, m->stream>>>(
+                sur::judge_args(*g), rows, sur::judge_q(rows), m->raw.p, m->tix.p, m->policy.p, n_window, m->y.p, nullptr, m->count.p);
+            GFX_HIP(hipGetLastError());
+            GFX_HIP(hipMemcpyAsync(out + size_t(b) * 18, m->y.p, size_t(rows) * 72, hipMemcpyDeviceToHost, m->stream));
         }
-        std::vector<int32_t> cell(n);
-        std::vector<float> jo(size_t(n) * 18);
-        DevBuf<double> q;
-        DevBuf<int32_t> t, c;
-        DevBuf<float> o;
-        DevBuf<uint8_t> fb;
-        q.alloc(size_t(n) * 3);
-        t.alloc(n);
-        c.alloc(n);
-        o.alloc(size_t(n) * 18);
-        std::vector<uint8_t> judge_only(size_t(g->n_cell) * n_window);
-        for (size_t r = 0; r < judge_only.size(); ++r) judge_only[r] = fallback[r] == 1 ? 1 : 0;
-        fb.upload(judge_only);
-        GFX_HIP(hipMemcpy(q.p, xyz, size_t(n) * 24, hipMemcpyHostToDevice));
-        GFX_HIP(hipMemcpy(t.p, tix, size_t(n) * 4, hipMemcpyHostToDevice));
-        GFX_HIP(hipMemsetAsync(o.p, 0, size_t(n) * 72, g->stream));
-        sur::k_judge<<<(n + 127) / 128, 128, 0, g->stream>>>(sur::judge_args(*g), n, q.p, t.p, fb.p, n_window, o.p,
-                                                              c.p);
-        GFX_HIP(hipGetLastError());
-        GFX_HIP(hipStreamSynchronize(g->stream));
-        GFX_HIP(hipMemcpy(jo.data(), o.p, jo.size() * 4, hipMemcpyDeviceToHost));
-        GFX_HIP(hipMemcpy(cell.data(), c.p, size_t(n) * 4, hipMemcpyDeviceToHost));
-        int nf = 0;
-        const float zero[18] = {};
-        for (int i = 0; i < n; ++i) {
-            const uint8_t how = cell[i] < 0 ? 1 : fallback[sur::region_of(cell[i], tix[i], g->n_time, n_window)];
-            const bool use_judge = how == 1;
-            const float* src = use_judge ? &jo[size_t(i) * 18] : how == 2 ? zero : &mo[size_t(i) * 18];
-            if (use_judge) {
-                ++nf;
-                if (cell[i] < 0)
-                    for (int k = 0; k < 18; ++k) jo[size_t(i) * 18 + k] = __builtin_nanf("");
-            }
-            std::memcpy(out + size_t(i) * 18, src, 72);
-        }
-        *n_fallback = nf;
+        GFX_HIP(hipMemcpyAsync(n_fallback, m->count.p, sizeof(int), hipMemcpyDeviceToHost, m->stream));
+        GFX_HIP(hipStreamSynchronize(m->stream));
     });
 }

@@ -275,3 +275,61 @@ def test_network_serves_regions_the_zero_predictor_cannot():
     assert res["combined_tile_bytes"] < res["zero_gate_tile_bytes"] <= res["tile_bytes"]
     assert res["combined_judge_fraction"] < 1.0 - res["combined_zero_fraction"]
     assert res["combined_rel_l2"] <= 0.02
+
+
+@pytest.mark.parametrize("width,depth,n_freq,rows", [(16, 1, 1, 1), (48, 2, 10, 63), (100, 3, 13, 65), (64, 2, 32, 257),
+                                                     (200, 2, 8, 1000), (320, 1, 70, 130)])
+def test_mlp_products_at_tile_edges(width, depth, n_freq, rows):
+    """Widths, feature counts and rows off the products' tiles (64, 128) and
+    padding (64): forward and every gradient block against the CPU model, with
+    the bars of the default shape (BF16 operands on both sides; only the order
+    of the FP32 sums differs)."""
+    net, ref, lo, hi = _model_pair(width=width, depth=depth, n_freq=n_freq)
+    rng = np.random.default_rng(rows)
+    x = lo + rng.random((rows, 4)) * (hi - lo)
+    y = rng.standard_normal((rows, 18)).astype(np.float32)
+    want = ref.predict(x)
+    for _ in range(2):  # the second call finds the first one's activations in the buffers
+        assert np.linalg.norm(net.forward(x) - want) < 1e-3 * np.linalg.norm(want)
+    lref, gref = ref.loss_grad(x, y)
+    for _ in range(2):
+        g, loss = net.gradient(x, y)
+        assert abs(loss - lref) <= 1e-4 * abs(lref)
+        for off, iw, ow in ref.shapes:
+            for b in (slice(off, off + iw * ow), slice(off + iw * ow, off + iw * ow + ow)):
+                assert np.linalg.norm(g[b] - gref[b]) <= 5e-3 * np.linalg.norm(gref[b]) + 1e-12
+
+
+def test_mlp_large_tiles_equal_small_tiles():
+    """Enough rows for the 128 x 128 tiles: each output equals, bit for bit, the
+    one a small call computes on 64 x 64 tiles (one output, the same products in
+    the same order)."""
+    net, _, lo, hi = _model_pair(width=256, depth=2, n_freq=16)
+    rng = np.random.default_rng(2)
+    x = lo + rng.random((33000, 4)) * (hi - lo)
+    big = net.forward(x)
+    for b in (0, 16384, 32900):
+        assert np.array_equal(net.forward(x[b:b + 100]), big[b:b + 100])
+
+
+def test_judge_groups_of_queries_equal_single_queries():
+    """More than 8,192 queries run several to a wavefront; each answer is the one
+    a small call gives, inside the tile, at its nodes and outside."""
+    rng = np.random.default_rng(4)
+    mesh = mc.small_halfspace(nx=4, ny=4, nz=3, pml=1)
+    ib = mesh.ibool.reshape(-1, 125)
+    nodes, inv = np.unique(ib.ravel(), return_inverse=True)
+    xyz = mesh.node_xyz.reshape(-1, 3)[nodes]
+    tile = pygfx.GreenTile(3, xyz, inv.reshape(-1, 125).astype(np.int32))
+    for t in range(3):
+        tile.set_values(t, rng.normal(size=(len(nodes), 18)).astype(np.float32))
+    lo, hi = xyz.min(axis=0), xyz.max(axis=0)
+    q = lo - 50.0 + rng.random((20001, 3)) * (hi - lo + 100.0)
+    q[::37] = xyz[rng.integers(0, len(nodes), len(q[::37]))]
+    tix = rng.integers(-1, 4, len(q)).astype(np.int32)
+    out, cell = tile.interpolate(q, tix)
+    assert (cell < 0).any() and (cell >= 0).any()
+    for b in (0, 7777, 19990):
+        o, c = tile.interpolate(q[b:b + 300], tix[b:b + 300])
+        assert np.array_equal(c, cell[b:b + 300])
+        assert np.array_equal(o, out[b:b + 300], equal_nan=True)
