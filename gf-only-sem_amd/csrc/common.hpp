@@ -56,13 +56,15 @@ struct GLL {
     void lagrange(double xi, double* ell) const;
 };
 
-// Static-partitioned parallel loop over [0, n) with up to `threads` workers.
+// Static-partitioned parallel loop over [0, n) with up to `threads` workers of at
+// least `grain` items each (starting a worker costs tens of microseconds).
 template <typename Fn>
-void parallel_for(int64_t n, Fn&& fn, int threads = 0) {
+void parallel_for(int64_t n, Fn&& fn, int threads = 0, int64_t grain = 1) {
     if (threads <= 0) {
         unsigned hc = std::thread::hardware_concurrency();
         threads = (int)std::min<unsigned>(hc ? hc : 1, 16);
     }
+    threads = int(std::min<int64_t>(threads, std::max<int64_t>(1, n / grain)));
     if (n < 4096 || threads == 1) {
         for (int64_t i = 0; i < n; ++i) fn(i);
         return;
