@@ -735,19 +735,22 @@ __device__ __forceinline__ float conv_step(const float* abc, float& q, float g) 
 // the 45).  The arithmetic is the same for every AX: the terms of an axis
 // with d = 0 are exact zeros either way, so the residuals do not depend on
 // how elements are grouped.
+struct CpmlShared {
+    float sD[25];
+    float su[3][NP];
+    float sf[9][NP];
+    float scf[CPML_NC][128];  // each lane's own coefficients
+};
 template <int MODE, int AX>
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(3, 3)))
-k_element_cpml(ElemArgs A, int e0, int ne) {
-    __shared__ float sD[25];
-    __shared__ float su[3][NP];
-    __shared__ float sf[9][NP];
-    __shared__ float scf[CPML_NC][128];  // each lane's own coefficients
+__device__ __forceinline__ void cpml_body(const ElemArgs& A, CpmlShared& S, int e, int f0, int f1) {
+    auto& sD = S.sD;
+    auto& su = S.su;
+    auto& sf = S.sf;
+    auto& scf = S.scf;
     const int tid = threadIdx.x;
     if (tid < 25) sD[tid] = A.D[tid];
-    const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int p = tid;
-    const bool valid = p < NP && blk < ne;
-    const int e = e0 + (valid ? blk : 0);
+    const bool valid = p < NP;
     const int pc = valid ? p : 0;
     const int i = pc / 25, j = (pc / 5) % 5, k = pc % 5;
     float g[9];
@@ -787,7 +790,7 @@ k_element_cpml(ElemArgs A, int e0, int ne) {
     const float* Di = &sD[i * 5];
     const float* Dj = &sD[j * 5];
     const float* Dk = &sD[k * 5];
-    for (int f = 0; f < A.nf; ++f) {
+    for (int f = f0; f < f1; ++f) {
         const int64_t fo = int64_t(f) * A.fstride;
         if (valid) {
             const float* ut = A.U + fo + node * 3;
@@ -896,6 +899,37 @@ k_element_cpml(ElemArgs A, int e0, int ne) {
             emit_residual<MODE>(A, f, node, rslot, rold, rv);
         }
         __syncthreads();  // su and sf are rewritten by the next field
+    }
+}
+
+// The PML elements of up to eight ranges, one per set of damped axes, in one
+// launch: the ranges are small (a corner's has tens of elements) and one after
+// the other each left most of the device idle.  All forms hold at most the
+// registers of three waves per SIMD, so sharing a launch costs none of them any.
+// blockIdx.y: fields [y * chunk, (y + 1) * chunk).
+struct CpmlRanges {
+    int n;
+    int first[9];  // first workgroup of each range, then the total
+    int e0[8], ax[8];
+};
+template <int MODE>
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(3, 3)))
+k_element_cpml(ElemArgs A, CpmlRanges R, int chunk) {
+    __shared__ CpmlShared S;
+    const int blk = xcd_block(blockIdx.x, gridDim.x);
+    int r = 0;
+    while (r + 1 < R.n && blk >= R.first[r + 1]) ++r;
+    const int e = R.e0[r] + blk - R.first[r];
+    const int f0 = blockIdx.y * chunk, f1 = min(A.nf, f0 + chunk);
+    switch (R.ax[r]) {
+        case 0: cpml_body<MODE, 0>(A, S, e, f0, f1); break;
+        case 1: cpml_body<MODE, 1>(A, S, e, f0, f1); break;
+        case 2: cpml_body<MODE, 2>(A, S, e, f0, f1); break;
+        case 3: cpml_body<MODE, 3>(A, S, e, f0, f1); break;
+        case 4: cpml_body<MODE, 4>(A, S, e, f0, f1); break;
+        case 5: cpml_body<MODE, 5>(A, S, e, f0, f1); break;
+        case 6: cpml_body<MODE, 6>(A, S, e, f0, f1); break;
+        default: cpml_body<MODE, 7>(A, S, e, f0, f1); break;
     }
 }
 

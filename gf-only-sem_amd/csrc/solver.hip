@@ -36,6 +36,7 @@ struct ElemRange {
     bool pml;
     int ax;  // complete C-PML: the axes (bit 0 x, 1 y, 2 z) with d != 0 at some point of the range's elements
     int cb, ce;  // GATHER: the range's clusters
+    int color;
 };
 
 // Where GATHER assembly leaves residuals: node n sums the entries
@@ -468,17 +469,28 @@ void launch_att(gfx_solver& S, const dev::ElemArgs& a, int b, int n) {
     }
 }
 
-template <int MODE>
-void launch_cpml(gfx_solver& S, const dev::ElemArgs& a, int ax, int b, int n) {
-    switch (ax) {
-        case 0: dev::k_element_cpml<MODE, 0><<<n, 128, 0, S.stream>>>(a, b, n); break;
-        case 1: dev::k_element_cpml<MODE, 1><<<n, 128, 0, S.stream>>>(a, b, n); break;
-        case 2: dev::k_element_cpml<MODE, 2><<<n, 128, 0, S.stream>>>(a, b, n); break;
-        case 3: dev::k_element_cpml<MODE, 3><<<n, 128, 0, S.stream>>>(a, b, n); break;
-        case 4: dev::k_element_cpml<MODE, 4><<<n, 128, 0, S.stream>>>(a, b, n); break;
-        case 5: dev::k_element_cpml<MODE, 5><<<n, 128, 0, S.stream>>>(a, b, n); break;
-        case 6: dev::k_element_cpml<MODE, 6><<<n, 128, 0, S.stream>>>(a, b, n); break;
-        default: dev::k_element_cpml<MODE, 7><<<n, 128, 0, S.stream>>>(a, b, n); break;
+// The complete C-PML's elements of ranges [r0, r1) in one launch.  With few
+// elements the fields are spread over workgroups too, until the launch has some
+// eight rounds of the device's workgroup places.
+void launch_cpml(gfx_solver& S, const dev::ElemArgs& a, int r0, int r1) {
+    dev::CpmlRanges R{};
+    int blocks = 0;
+    for (int i = r0; i < r1; ++i) {
+        R.first[R.n] = blocks;
+        R.e0[R.n] = S.ranges[i].b;
+        R.ax[R.n] = S.ranges[i].ax;
+        ++R.n;
+        blocks += S.ranges[i].e - S.ranges[i].b;
+    }
+    if (blocks == 0) return;
+    R.first[R.n] = blocks;
+    const int want = std::max(1, 12288 / blocks);
+    const int chunk = (S.nf + want - 1) / want;
+    const dim3 grid(unsigned(blocks), unsigned((S.nf + chunk - 1) / chunk));
+    switch (S.assembly) {
+        case GFX_ASSEMBLY_GATHER: dev::k_element_cpml<dev::ASM_GATHER><<<grid, 128, 0, S.stream>>>(a, R, chunk); break;
+        case GFX_ASSEMBLY_ATOMIC: dev::k_element_cpml<dev::ASM_ATOMIC><<<grid, 128, 0, S.stream>>>(a, R, chunk); break;
+        default: dev::k_element_cpml<dev::ASM_COLORED><<<grid, 128, 0, S.stream>>>(a, R, chunk); break;
     }
 }
 
@@ -492,9 +504,10 @@ void launch_clusters(gfx_solver& S, const dev::ElemArgs& a, const ElemRange& rg)
         dev::k_cluster<false, OUT><<<grid, dev::CLUSTER_THREADS, 0, S.stream>>>(a, rg.cb);
 }
 
-void launch_element(gfx_solver& S, const dev::ElemArgs& a, const ElemRange& rg) {
+// One range of elements that are not the complete C-PML's.
+void launch_range(gfx_solver& S, const dev::ElemArgs& a, const ElemRange& rg) {
     const int b = rg.b, n = rg.e - rg.b;
-    if (S.n_sls > 0 && !rg.pml) {  // shear attenuation: one kernel form for every range
+    if (S.n_sls > 0) {  // shear attenuation: one kernel form for every range
         if (n > 0) {
             switch (S.assembly) {
                 case GFX_ASSEMBLY_GATHER: launch_att<dev::ASM_GATHER>(S, a, b, n); break;
@@ -504,15 +517,7 @@ void launch_element(gfx_solver& S, const dev::ElemArgs& a, const ElemRange& rg) 
         }
         return;
     }
-    if (rg.pml) {  // complete C-PML: one element per workgroup, general form (elastic)
-        if (n > 0) {
-            switch (S.assembly) {
-                case GFX_ASSEMBLY_GATHER: launch_cpml<dev::ASM_GATHER>(S, a, rg.ax, b, n); break;
-                case GFX_ASSEMBLY_ATOMIC: launch_cpml<dev::ASM_ATOMIC>(S, a, rg.ax, b, n); break;
-                default: launch_cpml<dev::ASM_COLORED>(S, a, rg.ax, b, n); break;
-            }
-        }
-    } else if (ref_elem_pml(S)) {
+    if (ref_elem_pml(S)) {
         launch_element_p<true, false>(S, a, b, n);  // element-local C-PML: block kernel, general form
     } else if (uses_clusters(S)) {
         launch_clusters<dev::CL_FUSED>(S, a, rg);
@@ -521,6 +526,20 @@ void launch_element(gfx_solver& S, const dev::ElemArgs& a, const ElemRange& rg) 
     } else {
         launch_element_d<false>(S, a, b, n);
     }
+}
+
+// Ranges from i on: one, or all of the complete C-PML's that follow each other
+// (they share a launch; one colour's under COLORED assembly).  Returns the next.
+int launch_element(gfx_solver& S, const dev::ElemArgs& a, int i) {
+    const int n = int(S.ranges.size());
+    if (!S.ranges[i].pml) {
+        launch_range(S, a, S.ranges[i]);
+        return i + 1;
+    }
+    int j = i + 1;
+    while (j < n && S.ranges[j].pml && S.ranges[j].color == S.ranges[i].color && j - i < 8) ++j;
+    launch_cpml(S, a, i, j);
+    return j;
 }
 
 void launch_node_special(gfx_solver& S, const dev::NodeArgs& na, int grid) {
@@ -707,9 +726,9 @@ void enqueue_step(gfx_solver& S, const StepArgs& a, bool record, hipEvent_t* ev)
         dev::k_zero<<<a.zero_grid, 256, 0, S.stream>>>(reinterpret_cast<float4*>(S.R.p), a.r4);
     const int nr = int(S.ranges.size());
     const int pml_tail = S.pml_tail >= 0 ? S.pml_tail : nr;
-    for (int i = 0; i < nr; ++i) {
+    for (int i = 0; i < nr;) {
         if (ev && i == pml_tail) GFX_HIP(hipEventRecord(ev[0], S.stream));
-        launch_element(S, a.ea, S.ranges[i]);
+        i = launch_element(S, a.ea, i);
     }
     if (ev && pml_tail == nr) GFX_HIP(hipEventRecord(ev[0], S.stream));
     GFX_HIP(hipGetLastError());
@@ -1214,7 +1233,7 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
             if (i == E || col[elem_of_int[i]] != col[e0] || pml_el[elem_of_int[i]] != pml_el[e0] ||
                 pml_ax[elem_of_int[i]] != pml_ax[e0] || diag_el[elem_of_int[i]] != diag_el[e0]) {
                 const bool pml = pml_el[e0] != 0;
-                S.ranges.push_back({b, i, diag_el[e0] != 0 && !pml, pml, int(pml_ax[e0]), 0, 0});
+                S.ranges.push_back({b, i, diag_el[e0] != 0 && !pml, pml, int(pml_ax[e0]), 0, 0, col[e0]});
                 if (by_cluster) {
                     S.ranges.back().cb = int(S.cl_begin.size());
                     cluster_range(key, elem_of_int, b, i, d.elem_centroid != nullptr, S.cl_begin);
@@ -1979,11 +1998,11 @@ extern "C" gfx_status gfx_step_element_residual(gfx_solver* s, int ngll, int n_e
                 "ATOMIC assembly adds into the residual: call gfx_step_zero_residual first");
         StepArgs a = make_step_args(*s, true);
         a.ea.nstf = 0;  // sources come from gfx_step_source_injection
-        for (const auto& rg : s->ranges) {
+        for (int i = 0; i < int(s->ranges.size());) {
             if (uses_clusters(*s))
-                launch_clusters<dev::CL_POINTS>(*s, a.ea, rg);
+                launch_clusters<dev::CL_POINTS>(*s, a.ea, s->ranges[i++]);
             else
-                launch_element(*s, a.ea, rg);
+                i = launch_element(*s, a.ea, i);
         }
         GFX_HIP(hipGetLastError());
         s->stage = STAGE_ELEMENT;
