@@ -581,7 +581,7 @@ int node_chunk(int blocks, int nf) {
 }
 
 struct StepArgs {
-    bool clusters = false;  // cluster form: one launch for all nodes
+    bool direct = false;  // one launch for all nodes, each lane summing its node's entries
     dev::ElemArgs ea{};
     dev::NodeArgs na{};
     dev::RecArgs ra{};
@@ -598,7 +598,11 @@ void require_plan(gfx_solver& S, int which);
 StepArgs make_step_args(gfx_solver& S, bool points = false) {
     StepArgs a;
     const bool clusters = !points && uses_clusters(S);
-    a.clusters = clusters;
+    // entries per element point: with few fields the one launch without LDS staging
+    // is faster (28 x 26 x 15 elements, 3 fields: 67 us against 77 in two launches;
+    // 4,000 elements, 1 field: 21 us a step against 28), with many the staged sums
+    // are (36 x 36 x 18, 24 fields: 793 us against 847)
+    a.direct = clusters || (S.assembly == GFX_ASSEMBLY_GATHER && !points && S.node_fg == 1 && S.nf <= 4);
     require_plan(S, S.assembly != GFX_ASSEMBLY_GATHER ? R_ASSEMBLED : clusters ? R_CLUSTERS : R_POINTS);
     const GatherPlan& gp = clusters ? S.by_cluster : S.by_point;
     const double theta = 1.0 / 8.0;  // pml.cpp:35, coefficients pml.cpp:63-64
@@ -681,7 +685,7 @@ StepArgs make_step_args(gfx_solver& S, bool points = false) {
     na.c2 = c2;
     na.dt = float(S.dt);
     const int fg = S.node_fg;
-    if (clusters) {  // one node per lane
+    if (a.direct) {  // one node per lane
         a.spec_grid = int((S.Ga + 255) / 256);
         a.reg_grid = int((na.G4 - S.Ga + 255) / 256);
     } else {
@@ -735,10 +739,10 @@ void enqueue_step(gfx_solver& S, const StepArgs& a, bool record, hipEvent_t* ev)
     if (ev) GFX_HIP(hipEventRecord(ev[1], S.stream));
     const bool rec = record && a.recording && a.rec_grid > 0;
     const bool split = ev != nullptr;  // per-kernel timing: special and regular nodes apart
-    int* const close = a.clusters && !rec ? S.ctr.p : nullptr;  // the node launch closes the step
+    int* const close = a.direct && !rec ? S.ctr.p : nullptr;  // the node launch closes the step
     bool closed = false;
     auto nodes = [&](bool special, bool regular) {
-        if (!a.clusters) {
+        if (!a.direct) {
             if (special && a.spec_grid > 0) launch_node_special(S, a.na, a.spec_grid);
             if (regular && a.reg_grid > 0) launch_node_regular(S, a.na, a.reg_grid);
             return;
@@ -2543,6 +2547,7 @@ struct gfx_batch {
         // launch shape: workgroups per launch, kernel form
         int bg = 0, bd = 0, bs = 0, br = 0, n_ctr = 0;
         int fg = 1, kernel = 0, epb = 1;
+        bool direct = false;  // one launch for all nodes
     };
     struct Cached {
         std::vector<char> active;
@@ -2638,7 +2643,7 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
             }
             for (int w = 0; w < (n + S.epb - 1) / S.epb; ++w) m.push_back(make_int4(t, rg.b, n, w));
         }
-        if (args[i].clusters) {  // all nodes in the one launch of c.map_spec
+        if (args[i].direct) {  // all nodes in the one launch of c.map_spec
             for (int f = 0; f < S.nf; f += GROUP_CHUNK)
                 for (int w = 0; w < args[i].spec_grid + args[i].reg_grid; ++w)
                     es.push_back(make_int4(t, args[i].spec_grid, f, w));
@@ -2668,6 +2673,7 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
     c.n_ctr = int(ctr.size());
     c.fg = fg;
     c.kernel = kernel;
+    c.direct = args[c.members.front()].direct;
     c.epb = epb;
 }
 
@@ -2677,7 +2683,7 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
 void enqueue_group(gfx_batch::Group& c, const std::vector<StepArgs>& args, hipStream_t st) {
     if (c.bg > 0) launch_element_grp<false>(c.kernel, c.epb, c, c.map_gen, c.bg, st);
     if (c.bd > 0) launch_element_grp<true>(c.kernel, c.epb, c, c.map_diag, c.bd, st);
-    if (c.kernel == GFX_ELEMENT_WAVE && c.bs > 0)
+    if (c.direct && c.bs > 0)
         dev::k_cluster_nodes_grp<<<c.bs, 256, 0, st>>>(c.ntab.p, c.map_spec.p, GROUP_CHUNK);
     else switch (c.fg) {
         case 2: launch_nodes_grp<2>(c, st); break;
