@@ -9,7 +9,7 @@
 // through LDS (54 dwords per point and field; one lane per point needs 102).
 // The residuals of the cluster's elements are then summed per node in LDS:
 //   - interior nodes (regular, in no other cluster) take their Newmark update
-//     here, with no trip through memory for their residual but the copy kept
+//     here; their residual goes to memory only in a run's last step (keep_r),
 //     for gfx_solver_get_state;
 //   - the others leave one entry per cluster and node in Rl, which the node
 //     kernel sums in cluster order.
@@ -321,7 +321,7 @@ __device__ __forceinline__ void cluster_body(const ElemArgs& A, const ClusterHea
                     if (i < count(4)) more(integral_constant<int, 4>{}, integral_constant<int, 4>{});
                 }
             }
-            at_node(A.Rl + int64_t(f) * A.PR * 3, dst[q]) = F3{r[q][0], r[q][1], r[q][2]};
+            if (!in || A.keep_r) at_node(A.Rl + int64_t(f) * A.PR * 3, dst[q]) = F3{r[q][0], r[q][1], r[q][2]};
             if (in) {  // the regular nodes' update
                 F3 u, w;
                 float m1;

@@ -94,6 +94,7 @@ struct ElemArgs {
     const float* __restrict__ minv;
     float* Uw;
     float* Ww;
+    int keep_r;  // the interior nodes' residuals are wanted too (the run's last step)
     float D[25];
 };
 
@@ -1664,7 +1665,7 @@ __global__ void __launch_bounds__(256) k_zero(float4* __restrict__ p, int64_t n4
 // Strain of the recording cells (forward/share/src/solver.cpp:282-335) from
 // u_{n+1} = U - dt W, and copies of u, v, a at their points (solver.cpp:656-674).
 template <int EPB>
-__global__ void __launch_bounds__(((EPB * NP + 63) / 64) * 64) k_record(RecArgs A) {
+__device__ __forceinline__ void record_body(const RecArgs& A, int blk) {
     __shared__ float sD[25];
     __shared__ float su[EPB][3][NP];
     // snapshot steps only (step % stride == 0), into ring slot n_snap % cap;
@@ -1679,7 +1680,7 @@ __global__ void __launch_bounds__(((EPB * NP + 63) / 64) * 64) k_record(RecArgs 
     if (tid < 25) sD[tid] = A.D[tid];
     const int le = tid / NP;
     const int p = tid - le * NP;
-    const int cell = blockIdx.x * EPB + le;
+    const int cell = blk * EPB + le;
     const bool valid = (le < EPB) && (cell < A.n_rec);
     const int lel = valid ? le : 0;
     const int i = p / 25, j = (p / 5) % 5, k = p % 5;
@@ -1744,6 +1745,19 @@ __global__ void __launch_bounds__(((EPB * NP + 63) / 64) * 64) k_record(RecArgs 
         }
         if (f + 1 < A.nf) __syncthreads();
     }
+}
+
+template <int EPB>
+__global__ void __launch_bounds__(((EPB * NP + 63) / 64) * 64) k_record(RecArgs A) {
+    record_body<EPB>(A, blockIdx.x);
+}
+
+// One launch for the recording cells of several solvers: map entry (solver, workgroup).
+template <int EPB>
+__global__ void __launch_bounds__(((EPB * NP + 63) / 64) * 64)
+    k_record_grp(const RecArgs* __restrict__ tab, const int4* __restrict__ map) {
+    const int4 E = map[blockIdx.x];
+    record_body<EPB>(const_row(tab, E.x), E.w);
 }
 
 // ---------------------------------------------------------------------------

@@ -628,6 +628,7 @@ StepArgs make_step_args(gfx_solver& S, bool points = false) {
     ea.minv = S.minv.p;
     ea.Uw = S.U.p;
     ea.Ww = S.W.p;
+    ea.keep_r = 1;
     ea.W = S.W.p;
     ea.Aacc = S.Aacc.p;
     ea.astride = S.astride;
@@ -803,7 +804,7 @@ void run_steps(gfx_solver& S, int nsteps) {
         GFX_HIP(hipStreamSynchronize(S.stream));
         return;
     }
-    const StepArgs a = make_step_args(S);
+    StepArgs a = make_step_args(S);
     std::vector<hipEvent_t> ev;
     constexpr size_t EV = 5;
     if (S.timing) {
@@ -818,6 +819,7 @@ void run_steps(gfx_solver& S, int nsteps) {
     std::vector<char> did_rec(nsteps, 0);
     for (int t = 0; t < nsteps; ++t) {
         const bool snap = a.recording && S.step % S.stride == 0;
+        a.ea.keep_r = t + 1 == nsteps;  // only the last step's residual can be asked for
         enqueue_step(S, a, snap, S.timing ? &ev[size_t(t) * EV + 1] : nullptr);
         did_rec[t] = snap ? 1 : 0;
         advance_host(S);
@@ -2539,13 +2541,14 @@ struct gfx_batch {
         std::vector<int> members;  // solver indices
         gfx::DevBuf<gfx::dev::ElemArgs> etab;
         gfx::DevBuf<gfx::dev::NodeArgs> ntab;
+        gfx::DevBuf<gfx::dev::RecArgs> rtab;
         // per-workgroup work of each launch (general and diagonal element
         // forms, special and regular nodes)
-        gfx::DevBuf<int4> map_gen, map_diag, map_spec, map_reg;
+        gfx::DevBuf<int4> map_gen, map_diag, map_spec, map_reg, map_rec;
         gfx::DevBuf<int*> ctrs;
         gfx::DevBuf<int> strides;
         // launch shape: workgroups per launch, kernel form
-        int bg = 0, bd = 0, bs = 0, br = 0, n_ctr = 0;
+        int bg = 0, bd = 0, bs = 0, br = 0, bc = 0, n_ctr = 0;
         int fg = 1, kernel = 0, epb = 1;
         bool direct = false;  // one launch for all nodes
     };
@@ -2622,7 +2625,8 @@ constexpr int GROUP_CHUNK = 4;  // fields per workgroup of a group's node launch
 void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>& args) {
     std::vector<dev::ElemArgs> et;
     std::vector<dev::NodeArgs> nt;
-    std::vector<int4> eg, ed, es, er;  // one entry per workgroup
+    std::vector<dev::RecArgs> rt;
+    std::vector<int4> eg, ed, es, er, ec;  // one entry per workgroup
     std::vector<int*> ctr;
     std::vector<int> strides;
     int fg = 1, kernel = GFX_ELEMENT_BLOCK, epb = 1;
@@ -2651,6 +2655,9 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
             for (int w = 0; w < args[i].spec_grid; ++w) es.push_back(make_int4(t, 0, 0, w));
             for (int w = 0; w < args[i].reg_grid; ++w) er.push_back(make_int4(t, 0, 0, w));
         }
+        rt.push_back(args[i].ra);
+        if (args[i].recording)
+            for (int w = 0; w < args[i].rec_grid; ++w) ec.push_back(make_int4(t, 0, 0, w));
         ctr.push_back(S.ctr.p);
         strides.push_back(S.stride);
     }
@@ -2664,12 +2671,15 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
     put(c.map_diag, ed);
     put(c.map_spec, es);
     put(c.map_reg, er);
+    put(c.rtab, rt);
+    put(c.map_rec, ec);
     put(c.ctrs, ctr);
     put(c.strides, strides);
     c.bg = int(eg.size());
     c.bd = int(ed.size());
     c.bs = int(es.size());
     c.br = int(er.size());
+    c.bc = int(ec.size());
     c.n_ctr = int(ctr.size());
     c.fg = fg;
     c.kernel = kernel;
@@ -2679,7 +2689,7 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
 
 // One step of a group of solvers as shared launches on stream st: the element
 // ranges of every member (general form, then diagonal form), all special nodes,
-// all regular nodes, then each member's recording and one counter update for all.
+// all regular nodes, all recording cells and one counter update for all.
 void enqueue_group(gfx_batch::Group& c, const std::vector<StepArgs>& args, hipStream_t st) {
     if (c.bg > 0) launch_element_grp<false>(c.kernel, c.epb, c, c.map_gen, c.bg, st);
     if (c.bd > 0) launch_element_grp<true>(c.kernel, c.epb, c, c.map_diag, c.bd, st);
@@ -2691,9 +2701,7 @@ void enqueue_group(gfx_batch::Group& c, const std::vector<StepArgs>& args, hipSt
         case 8: launch_nodes_grp<8>(c, st); break;
         default: launch_nodes_grp<1>(c, st); break;
     }
-    for (const int i : c.members)
-        if (args[i].recording && args[i].rec_grid > 0)
-            dev::k_record<REPB><<<args[i].rec_grid, args[i].rec_threads, 0, st>>>(args[i].ra);
+    if (c.bc > 0) dev::k_record_grp<REPB><<<c.bc, args[c.members.front()].rec_threads, 0, st>>>(c.rtab.p, c.map_rec.p);
     dev::k_advance_grp<<<(c.n_ctr + 63) / 64, 64, 0, st>>>(c.ctrs.p, c.strides.p, c.n_ctr);
     GFX_HIP(hipGetLastError());
 }
