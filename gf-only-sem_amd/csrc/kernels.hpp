@@ -78,14 +78,13 @@ struct ElemArgs {
     const int* __restrict__ ctr;          // device counters: [0] step index, [1] snapshots taken
     // shear attenuation (n_sls > 0): lam / mu hold the unrelaxed moduli; per
     // mechanism l and point: att_a = exp(-dt/tau_sigma), att_b = Y b, att_c = Y c
-    // ([n_sls][P]); memory zeta [nf][n_sls*5][P] and previous deviatoric
-    // strain devp [nf][5][P], both in the scaled strain units of the kernels
+    // ([n_sls][P]); carry zeta [nf][n_sls*5][P] = att_a z + att_b dev of the last
+    // step, in the scaled strain units of the kernels
     int n_sls;
     const float* __restrict__ att_a;
     const float* __restrict__ att_b;
     const float* __restrict__ att_c;
     float* __restrict__ zeta;
-    float* __restrict__ devp;
     // clusters (GATHER, wavefront form): heads, point lists, entries of the
     // nodes shared with other clusters, and what the interior update needs
     const ClusterHead* __restrict__ cl_head;
@@ -508,7 +507,10 @@ __global__ void __launch_bounds__(((EPB * NP + 63) / 64) * 64)
 // Stress with shear attenuation at one point of field f (general geometry):
 // strain from the gradient, the memory update of every mechanism
 // z <- a z + (Y b) dev_old + (Y c) dev_new, sigma = lam_U tr I + 2 mu_U eps -
-// sum z, and the fluxes F = sigma . g.  L > 0: L solids whose coefficients
+// sum z, and the fluxes F = sigma . g.  Kept between steps is the carry
+// a z + (Y b) dev, known when its step ends: the next z is carry + (Y c) dev_new
+// and no strain has to be kept beside it (three solids: 120 bytes per point and
+// field and step instead of 160; the kernel moves them at 5 TB/s).  L > 0: L solids whose coefficients
 // the caller holds in ca, cb, cc; L = 0: A.n_sls solids read from memory.
 template <int L>
 __device__ __forceinline__ void flux_att(const float (&ui)[3][5], const float (&uj)[3][5], const float (&uk)[3][5],
@@ -537,10 +539,6 @@ __device__ __forceinline__ void flux_att(const float (&ui)[3][5], const float (&
     const float tr = gr[0][0] + gr[1][1] + gr[2][2];
     const float dev[5] = {gr[0][0] - tr * (1.f / 3.f), gr[1][1] - tr * (1.f / 3.f), 0.5f * (gr[0][1] + gr[1][0]),
                           0.5f * (gr[0][2] + gr[2][0]), 0.5f * (gr[1][2] + gr[2][1])};
-    float* dp = A.devp + int64_t(f) * 5 * A.P + pt;
-    float old[5];
-#pragma unroll
-    for (int q = 0; q < 5; ++q) old[q] = dp[int64_t(q) * A.P];
     float zs[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
     const int nl = L > 0 ? L : A.n_sls;
     float* zf = A.zeta + int64_t(f) * nl * 5 * A.P + pt;
@@ -552,8 +550,8 @@ __device__ __forceinline__ void flux_att(const float (&ui)[3][5], const float (&
         for (int l = 0; l < L; ++l)
 #pragma unroll
             for (int q = 0; q < 5; ++q) {
-                const float z = ca[l] * zo[l * 5 + q] + cb[l] * old[q] + cc[l] * dev[q];
-                zf[int64_t(l * 5 + q) * A.P] = z;
+                const float z = zo[l * 5 + q] + cc[l] * dev[q];
+                zf[int64_t(l * 5 + q) * A.P] = ca[l] * z + cb[l] * dev[q];
                 zs[q] += z;
             }
     } else {
@@ -563,14 +561,12 @@ __device__ __forceinline__ void flux_att(const float (&ui)[3][5], const float (&
 #pragma unroll
             for (int q = 0; q < 5; ++q) {
                 float* zq = zf + int64_t(l * 5 + q) * A.P;
-                const float z = a * zq[0] + b * old[q] + c * dev[q];
-                zq[0] = z;
+                const float z = zq[0] + c * dev[q];
+                zq[0] = a * z + b * dev[q];
                 zs[q] += z;
             }
         }
     }
-#pragma unroll
-    for (int q = 0; q < 5; ++q) dp[int64_t(q) * A.P] = dev[q];
     const float mu2 = 2.f * mu;
     float sig[3][3];
     sig[0][0] = mu2 * gr[0][0] + lam * tr - zs[0];

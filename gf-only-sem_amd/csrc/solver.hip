@@ -95,7 +95,7 @@ struct gfx_solver {
     int64_t n_diag = 0;                       // elements on the axis-aligned (diagonal) path
     gfx::DevBuf<float> G9, lam, mu, minv, damp;
     int n_sls = 0;                                     // shear attenuation mechanisms
-    gfx::DevBuf<float> att_a, att_b, att_c, zeta, devp;
+    gfx::DevBuf<float> att_a, att_b, att_c, zeta;
     gfx::DevBuf<uint32_t> ibool;
     // C-PML: nodal (pc, palpha, pmem, pnew over [0,Gpml)) or element-local (Ppml points)
     gfx::DevBuf<float> pc, palpha, pabar, pmem, pnew;
@@ -322,7 +322,6 @@ void init_state(gfx_solver& S) {
     S.pmem.zero(S.stream);
     S.pnew.zero(S.stream);
     S.zeta.zero(S.stream);
-    S.devp.zero(S.stream);
     S.ctr.zero(S.stream);
     GFX_HIP(hipStreamSynchronize(S.stream));
     S.step = 0;
@@ -653,7 +652,6 @@ StepArgs make_step_args(gfx_solver& S, bool points = false) {
     ea.att_b = S.att_b.p;
     ea.att_c = S.att_c.p;
     ea.zeta = S.zeta.p;
-    ea.devp = S.devp.p;
     std::memcpy(ea.D, S.D, sizeof(S.D));
 
     dev::NodeArgs& na = a.na;
@@ -1325,60 +1323,78 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
             }
         }
     }
-    // regular nodes of one cluster only form a class of their own (-1) behind the
-    // other regular nodes
+    // Each cluster's nodes, once, with the number of its elements that hold them,
+    // those of most elements first: the order of the cluster kernel's lists.
+    // Regular nodes of one cluster only form a class of their own (-1) behind the
+    // other regular nodes.
+    std::vector<int32_t> cl_node;
+    std::vector<int64_t> cl_first;
     if (by_cluster) {
-        std::vector<int32_t> seen(G, -1), in_elem(G, -1);
-        std::vector<char> shared(G, 0);
-        S.cl_ok = true;
-        for (int c = 0; c + 1 < int(S.cl_begin.size()); ++c)
-            for (int i = S.cl_begin[c]; i < S.cl_begin[c + 1]; ++i)
-                for (int p = 0; p < NP; ++p) {
-                    const int g = d.ibool[int64_t(elem_of_int[i]) * NP + p];
-                    if (in_elem[g] == i) S.cl_ok = false;  // a node twice in one element: one entry per point only
-                    in_elem[g] = i;
-                    if (seen[g] >= 0 && seen[g] != c) shared[g] = 1;
-                    seen[g] = c;
+        const int nc = int(S.cl_begin.size()) - 1;
+        std::vector<std::vector<int32_t>> lists(nc);
+        std::atomic<bool> repeated{false};
+        parallel_for(nc, [&](int64_t c) {
+            std::vector<int32_t> ids;
+            ids.reserve(dev::CE * NP);
+            for (int i = S.cl_begin[c]; i < S.cl_begin[c + 1]; ++i) {
+                const int32_t* ib = d.ibool + int64_t(elem_of_int[i]) * NP;
+                ids.insert(ids.end(), ib, ib + NP);
+            }
+            std::vector<uint64_t> at(ids.size());  // (node, position), sorted: equal nodes meet
+            for (size_t q = 0; q < ids.size(); ++q) at[q] = (uint64_t(uint32_t(ids[q])) << 32) | q;
+            std::sort(at.begin(), at.end());
+            std::vector<uint64_t> uniq;  // (elements short of CE, first position)
+            uniq.reserve(at.size());
+            for (size_t q = 0; q < at.size();) {
+                size_t e = q + 1;
+                while (e < at.size() && (at[e] >> 32) == (at[q] >> 32)) {
+                    // a node twice in one element: one entry per point only
+                    if ((at[e] & 0xffff) / NP == (at[e - 1] & 0xffff) / NP) repeated = true;
+                    ++e;
                 }
+                uniq.push_back((uint64_t(dev::CE * NP - (e - q)) << 32) | (at[q] & 0xffff));
+                q = e;
+            }
+            std::sort(uniq.begin(), uniq.end());
+            for (const uint64_t u : uniq) lists[c].push_back(ids[u & 0xffff]);
+        }, 0, 64);
+        S.cl_ok = !repeated;
+        cl_first.assign(nc + 1, 0);
+        for (int c = 0; c < nc; ++c) cl_first[c + 1] = cl_first[c] + int64_t(lists[c].size());
+        cl_node.resize(cl_first[nc]);
+        std::vector<char> clusters(G, 0);  // of each node: 0, 1, 2 = more
+        for (int c = 0; c < nc; ++c) {
+            std::copy(lists[c].begin(), lists[c].end(), cl_node.begin() + cl_first[c]);
+            for (const int32_t g : lists[c])
+                if (clusters[g] < 2) ++clusters[g];
+        }
         for (int g = 0; g < G; ++g)
-            if (cls[g] == 0 && seen[g] >= 0 && !shared[g]) cls[g] = -1;
+            if (cls[g] == 0 && clusters[g] == 1) cls[g] = -1;
     }
     // numbering: C-PML nodes, other special nodes, regular nodes; first touch
     // in solver element order inside each class; C-PML nodes grouped by their
     // direction mask (first touch inside a group), so wavefronts share a mask;
-    // with clusters: cluster by cluster, the nodes of most of the cluster's elements
-    // first (the order of the cluster kernel's lists)
+    // with clusters: cluster by cluster in list order
     // (-1 = not yet seen, -2 = queued in this class, >= 0 = numbered)
     S.node_new_of_old.assign(G, -1);
     int next = 0;
     for (int pass = 2; pass >= -1; --pass) {
         std::vector<int> order;
         if (by_cluster) {
-            std::vector<uint8_t> held(G, 0);  // elements of the cluster that hold the node
-            for (int c = 0; c + 1 < int(S.cl_begin.size()); ++c) {
-                const size_t b = order.size();
-                for (int i = S.cl_begin[c]; i < S.cl_begin[c + 1]; ++i)
-                    for (int p = 0; p < NP; ++p) {
-                        const int g = d.ibool[int64_t(elem_of_int[i]) * NP + p];
-                        if (cls[g] != pass) continue;
-                        if (S.node_new_of_old[g] == -1) {
-                            S.node_new_of_old[g] = -2;
-                            held[g] = 0;
-                            order.push_back(g);
-                        }
-                        ++held[g];
-                    }
-                std::stable_sort(order.begin() + b, order.end(), [&](int x, int y) { return held[x] > held[y]; });
-            }
-        }
-        for (int i = 0; i < E; ++i) {
-            if (by_cluster) break;
-            const int64_t e = elem_of_int[i];
-            for (int p = 0; p < NP; ++p) {
-                const int g = d.ibool[e * NP + p];
+            for (const int32_t g : cl_node)
                 if (cls[g] == pass && S.node_new_of_old[g] == -1) {
                     S.node_new_of_old[g] = -2;
                     order.push_back(g);
+                }
+        } else {
+            for (int i = 0; i < E; ++i) {
+                const int64_t e = elem_of_int[i];
+                for (int p = 0; p < NP; ++p) {
+                    const int g = d.ibool[e * NP + p];
+                    if (cls[g] == pass && S.node_new_of_old[g] == -1) {
+                        S.node_new_of_old[g] = -2;
+                        order.push_back(g);
+                    }
                 }
             }
         }
@@ -1480,7 +1496,6 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
         dv.upload(S.att_b, std::move(hb));
         dv.upload(S.att_c, std::move(hc));
         dv.alloc(S.zeta, size_t(S.nf) * L * 5 * P);
-        dv.alloc(S.devp, size_t(S.nf) * 5 * P);
     }
     dv.upload(S.G9, std::move(hG));
     dv.upload(S.lam, std::move(hlam));
@@ -2195,7 +2210,7 @@ uint64_t layout_signature(const gfx_solver& S) {
 
 size_t checkpoint_bytes(const gfx_solver& S) {
     const size_t fl = size_t(S.nf) * S.fstride;
-    return CKPT_WORDS * 8 + 4 * (3 * fl + size_t(S.nf) * S.astride + S.pmem.n + S.pnew.n + S.zeta.n + S.devp.n);
+    return CKPT_WORDS * 8 + 4 * (3 * fl + size_t(S.nf) * S.astride + S.pmem.n + S.pnew.n + S.zeta.n);
 }
 
 }  // namespace
@@ -2226,7 +2241,7 @@ extern "C" gfx_status gfx_solver_checkpoint_save(const gfx_solver* s, void* host
         hdr[8] = int64_t(s->pmem.n);
         hdr[9] = int64_t(s->pnew.n);
         hdr[10] = int64_t(s->zeta.n);
-        hdr[11] = int64_t(s->devp.n);
+        hdr[11] = 0;  // (earlier images: previous deviatoric strains)
         float* p = reinterpret_cast<float*>(static_cast<char*>(host) + CKPT_WORDS * 8);
         const size_t fl = size_t(s->nf) * s->fstride, al = size_t(s->nf) * s->astride;
         auto get = [&](const float* d, size_t n) {
@@ -2239,7 +2254,6 @@ extern "C" gfx_status gfx_solver_checkpoint_save(const gfx_solver* s, void* host
         get(s->pmem.p, s->pmem.n);
         get(s->pnew.p, s->pnew.n);
         get(s->zeta.p, s->zeta.n);
-        get(s->devp.p, s->devp.n);
         // assembled residual of the last step (what get_state reads for a at
         // regular nodes): R itself, or the fixed-order slot sums
         if (s->r_src == R_ASSEMBLED) {
@@ -2264,11 +2278,14 @@ extern "C" gfx_status gfx_solver_checkpoint_load(gfx_solver* s, const void* host
         require(bytes >= size_t(CKPT_WORDS) * 8, "checkpoint image too small");
         const int64_t* hdr = static_cast<const int64_t*>(host);
         require(hdr[0] == CKPT_MAGIC, "not a solver checkpoint image");
+        // earlier images hold the solids' memories z and the previous deviatoric
+        // strain of every point instead of the carry a z + b dev
+        const int64_t n_dev = s->n_sls > 0 ? int64_t(s->nf) * 5 * s->E * NP : 0;
         require(hdr[1] == s->E && hdr[2] == s->G && hdr[3] == s->nf && hdr[4] == s->assembly &&
                     hdr[7] == int64_t(layout_signature(*s)) && hdr[8] == int64_t(s->pmem.n) &&
-                    hdr[9] == int64_t(s->pnew.n) && hdr[10] == int64_t(s->zeta.n) && hdr[11] == int64_t(s->devp.n),
+                    hdr[9] == int64_t(s->pnew.n) && hdr[10] == int64_t(s->zeta.n) && (hdr[11] == 0 || hdr[11] == n_dev),
                 "checkpoint was taken from a solver with another mesh, field count, assembly or attenuation");
-        require(bytes >= checkpoint_bytes(*s), "checkpoint image truncated");
+        require(bytes >= checkpoint_bytes(*s) + size_t(hdr[11]) * 4, "checkpoint image truncated");
         const float* p = reinterpret_cast<const float*>(static_cast<const char*>(host) + CKPT_WORDS * 8);
         const size_t fl = size_t(s->nf) * s->fstride, al = size_t(s->nf) * s->astride;
         GFX_HIP(hipStreamSynchronize(s->stream));
@@ -2281,8 +2298,23 @@ extern "C" gfx_status gfx_solver_checkpoint_load(gfx_solver* s, const void* host
         put(s->Aacc.p, al);
         put(s->pmem.p, s->pmem.n);
         put(s->pnew.p, s->pnew.n);
-        put(s->zeta.p, s->zeta.n);
-        put(s->devp.p, s->devp.n);
+        if (hdr[11] != 0) {
+            const int64_t P = int64_t(s->E) * NP, L = s->n_sls;
+            const std::vector<float> a = fetch(s, s->att_a.p, size_t(L * P)), b = fetch(s, s->att_b.p, size_t(L * P));
+            std::vector<float> q(p, p + s->zeta.n);
+            const float* dev = p + s->zeta.n;
+            for (int f = 0; f < s->nf; ++f)
+                for (int64_t l = 0; l < L; ++l)
+                    for (int64_t c = 0; c < 5; ++c)
+                        for (int64_t i = 0; i < P; ++i) {
+                            float& z = q[((f * L + l) * 5 + c) * P + i];
+                            z = a[l * P + i] * z + b[l * P + i] * dev[(f * 5 + c) * P + i];
+                        }
+            GFX_HIP(hipMemcpy(s->zeta.p, q.data(), q.size() * 4, hipMemcpyHostToDevice));
+            p += s->zeta.n + size_t(hdr[11]);
+        } else {
+            put(s->zeta.p, s->zeta.n);
+        }
         if (s->assembly != GFX_ASSEMBLY_GATHER) {
             put(s->R.p, fl);
         } else {
@@ -2501,10 +2533,10 @@ extern "C" double gfx_solver_algorithmic_bytes(const gfx_solver* s, int which) {
     if (s->cpml_complete) elem += 112.0 * Q + F * (8.0 * double(s->cpml_mem_active) + 12.0 * Q);
     // shear attenuation: the general form (48 B) at every point, 3 step
     // coefficients per solid per point, and per field the memory (5 per solid)
-    // and previous deviatoric strain (5) read and written at every point
+    // read and written at every point
     if (s->n_sls > 0) {
         const double L = s->n_sls;
-        elem = 48.0 * P + F * 24.0 * G + 12.0 * L * P + F * 8.0 * (5.0 * L + 5.0) * P;
+        elem = 48.0 * P + F * 24.0 * G + 12.0 * L * P + F * 40.0 * L * P;
     }
     // node stage: 1/m per node; per field r, u~, w read and u~, w written;
     // special nodes also read and write a; C-PML nodes read 5 + 9 coefficients

@@ -114,3 +114,34 @@ def test_forward_driver_reads_the_solids(tmp_path):
     assert mc.rel_l2(rec, mine) <= 1e-6
     ela = gpu_run(back, (cells, w, stf, 2), attenuation=False)
     assert mc.rel_l2(records(ela).reshape(rec.shape), rec) > 1e-3
+
+
+def test_images_with_memories_and_strains_load_as_carries():
+    """An image that holds the solids' memories z and the last deviatoric strain
+    (the form before the carry a z + b dev replaced both) loads as the carry.
+    One material and Q, so a and b are the same at every point."""
+    mesh = pygfx.build_box(nx=4, ny=3, nz=3, lx=2400.0, ly=1800.0, lz=1800.0, layers=[(0.0, 5000.0, 2900.0, 2500.0)],
+                           pml_xmin=0, pml_xmax=0, pml_ymin=0, pml_ymax=0, pml_zmax=0, duration=1.0,
+                           record_depth_max=0.0, n_sls=2, q_mu=[30.0], att_fmin=0.1, att_fmax=4.0)
+    P = mesh.n_elem * 125
+    s = pygfx.Solver(mesh, n_fields=1, assembly=pygfx.GFX_ASSEMBLY_GATHER, has_cpml=False, record_capacity=0)
+    image = np.frombuffer(s.checkpoint(), np.uint8).copy()
+    hdr = image[:128].view(np.int64)
+    n_z = int(hdr[10])
+    assert n_z == 2 * 5 * P and hdr[11] == 0
+    body = image[128:].view(np.float32)
+    n_r = -(-(-(-mesh.n_node // 4) * 4 * 3) // 64) * 64  # padded field of R, the last part
+    z_at = body.size - n_r - n_z
+    rng = np.random.default_rng(1)
+    z, dev = rng.normal(size=n_z).astype(np.float32), rng.normal(size=5 * P).astype(np.float32)
+    old = np.concatenate([body[:z_at], z, dev, body[z_at + n_z:]])
+    hdr[11] = 5 * P
+    s.restore(image[:128].tobytes() + old.tobytes())
+    got = np.frombuffer(s.checkpoint(), np.uint8)[128:].view(np.float32)[z_at:z_at + n_z]
+    ts, te = mesh.tau_sigma.reshape(-1, 2)[0], mesh.tau_epsilon.reshape(-1, 2)[0]
+    a = np.exp(-mesh.dt / ts)
+    q = ts * (1 - a) / mesh.dt
+    b = 2 * mesh.mu_[0] * (te / ts - 1) * (q - a)
+    want = a[:, None, None] * z.reshape(2, 5, P) + b[:, None, None] * dev.reshape(1, 5, P)
+    # FP32 coefficients and one FP32 rounding per operation: a few 1e-7
+    assert mc.rel_l2(got, want.ravel()) <= 1e-6
