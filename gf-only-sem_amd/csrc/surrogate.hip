@@ -30,6 +30,7 @@ constexpr int NP = 125;
 constexpr double EXACT_TOL = 1e-6;  // gll_interpolator.py:19
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __host__ __device__ inline uint16_t f2bf(float f) {
     uint32_t u = __builtin_bit_cast(uint32_t, f);
@@ -264,12 +265,12 @@ JudgeArgs judge_args(const gfx_green& G) {
 // network and [unit][row] for the weight gradients, weights both ways.  Sums,
 // biases, pre-activations, master weights and moments stay FP32.
 //
-// Bound: at 131,072 rows a hidden layer takes 115 us, of which erff is more than
+// Bound: at 131,072 rows a hidden layer takes 61 us, of which erff is more than
 // half (33.5 M values); its traffic would take 26 us.  At a training batch of
-// 8,192 rows the launches are latency bound (15 us a layer).  One Adam iteration
-// of the default network: 344 us, with FP32 operands rounded and transposed
-// while staging, separate bias and GELU passes and 256-term sums by single lanes
-// 1,380 us; 150,000 queries: 1.3 ms of kernels (2.9 ms).
+// 8,192 rows the launches are latency bound (9 to 11 us a layer and direction,
+// traffic 2 to 4).  One Adam iteration of the default network: 212 us, with FP32
+// operands rounded and transposed while staging, separate bias and GELU passes and
+// 256-term sums by single lanes 1,380 us; 150,000 queries: 0.8 ms of kernels (2.9 ms).
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int GK = 64;        // k per stage, and the padding of leading dimensions
@@ -331,14 +332,18 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& G, int mt, int nt, int
     const int mb = mt * T, nb = nt * T;
     const int wm = (wave >> 1) * (T / 2), wn = (wave & 1) * (T / 2);
     const int r16 = lane & 15, kq = (lane >> 4) * 8;
-    uint4 ra[L], rb[L];
+    // Built-in vectors: as an array of uint4 structs the stage went to scratch, and
+    // eight Adam iterations of 8,192 rows took 2.7 instead of 1.8 ms.  Two or four
+    // stages ahead (four are a whole layer of 256 units) were no faster: 1.70 and
+    // 1.80 ms against 1.69.
+    u32x4 ra[L], rb[L];
     auto fetch = [&](int k0) {
 #pragma unroll
         for (int q = 0; q < L; ++q) {
             const int i = t + 256 * q, row = i >> 3, kk = (i & 7) * 8;
             // rows past the end repeat the last one; their results are not stored
-            ra[q] = *reinterpret_cast<const uint4*>(G.A + int64_t(min(mb + row, G.M - 1)) * G.lda + k0 + kk);
-            rb[q] = *reinterpret_cast<const uint4*>(G.B + int64_t(min(nb + row, G.N - 1)) * G.ldb + k0 + kk);
+            ra[q] = *reinterpret_cast<const u32x4*>(G.A + int64_t(min(mb + row, G.M - 1)) * G.lda + k0 + kk);
+            rb[q] = *reinterpret_cast<const u32x4*>(G.B + int64_t(min(nb + row, G.N - 1)) * G.ldb + k0 + kk);
         }
     };
     f32x4 acc[F][F];
@@ -352,8 +357,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& G, int mt, int nt, int
 #pragma unroll
         for (int q = 0; q < L; ++q) {
             const int i = t + 256 * q, row = i >> 3, kk = (i & 7) * 8;
-            *reinterpret_cast<uint4*>(&sA[row * GKP + kk]) = ra[q];
-            *reinterpret_cast<uint4*>(&sB[row * GKP + kk]) = rb[q];
+            *reinterpret_cast<u32x4*>(&sA[row * GKP + kk]) = ra[q];
+            *reinterpret_cast<u32x4*>(&sB[row * GKP + kk]) = rb[q];
         }
         __syncthreads();
         if (k0 + GK < kend) fetch(k0 + GK);
@@ -393,6 +398,11 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& G, int mt, int nt, int
 #pragma unroll
             for (int q = 0; q < 4; ++q) v[q] = acc[i][j][q];
             if (EPI == EPI_OUT || EPI == EPI_PART) {
+                if (EPI == EPI_PART && G.N % 4 == 0) {  // 16-byte aligned: the layers before have whole rows of four
+                    if (m < G.M && n0 < G.N)
+                        *reinterpret_cast<float4*>(G.out + (int64_t(z) * G.M + m) * G.N + n0) = make_float4(v[0], v[1], v[2], v[3]);
+                    continue;
+                }
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                     if (m < G.M && n0 + q < G.N) G.out[(int64_t(z) * G.M + m) * G.N + n0 + q] = v[q] + bias[q];
@@ -464,33 +474,37 @@ __global__ void __launch_bounds__(256) k_gemm_grads(GradArgs W) {
 // from `splits` products, b from the row tiles' column sums.
 struct ReduceArgs {
     int n;                       // layers
-    int64_t w_off[GradArgs::MAX], b_off[GradArgs::MAX];
+    int64_t w_off[GradArgs::MAX];   // its weights, then its biases
     int64_t w_part[GradArgs::MAX];  // first partial product of the layer
     int64_t b_part[GradArgs::MAX];
     int size[GradArgs::MAX], cols[GradArgs::MAX], tiles[GradArgs::MAX];
+    int blk0[GradArgs::MAX];  // first workgroup of the layer
     int splits;
 };
-// 64 parameters per workgroup, four lanes each, so that the many row tiles of a
-// bias do not run as one serial chain; the four sums are added in lane order.
+// 64 parameters of one layer per workgroup, four lanes each, so that the many row
+// tiles of a bias do not run as one serial chain; the four sums are added in lane
+// order.  The layer is the workgroup's: its table is read by scalar loads, where a
+// search per lane read the kernel's arguments entry after entry.
 __global__ void __launch_bounds__(256) k_reduce_grads(ReduceArgs R, const float* __restrict__ wp,
-                                                      const float* __restrict__ bp, float* __restrict__ g, int64_t n) {
+                                                      const float* __restrict__ bp, float* __restrict__ g) {
     __shared__ float sh[4][64];
     const int c = threadIdx.x & 63, part = threadIdx.x >> 6;
-    const int64_t i = int64_t(blockIdx.x) * 64 + c;
+    int l = 0;
+    while (l + 1 < R.n && int(blockIdx.x) >= R.blk0[l + 1]) ++l;
+    const int i = (int(blockIdx.x) - R.blk0[l]) * 64 + c, size = R.size[l], cols = R.cols[l];
     float s = 0.f;
-    if (i < n) {
-        int l = 0;
-        while (l + 1 < R.n && i >= R.w_off[l + 1]) ++l;
-        const bool bias = i >= R.b_off[l];
+    if (i < size + cols) {
+        const bool bias = i >= size;
         const int cnt = bias ? R.tiles[l] : R.splits;
-        const int64_t stride = bias ? R.cols[l] : R.size[l];
-        const float* src = bias ? bp + R.b_part[l] + (i - R.b_off[l]) : wp + R.w_part[l] + (i - R.w_off[l]);
+        const int64_t stride = bias ? cols : size;
+        const float* src = bias ? bp + R.b_part[l] + (i - size) : wp + R.w_part[l] + i;
         const int q = (cnt + 3) / 4;
+#pragma unroll 4
         for (int z = part * q; z < min(cnt, part * q + q); ++z) s += src[z * stride];
     }
     sh[part][c] = s;
     __syncthreads();
-    if (part == 0 && i < n) g[i] = ((sh[0][c] + sh[1][c]) + sh[2][c]) + sh[3][c];
+    if (part == 0 && i < size + cols) g[R.w_off[l] + i] = ((sh[0][c] + sh[1][c]) + sh[2][c]) + sh[3][c];
 }
 
 // features [sin, cos](2 pi B x) as BF16, [row][ld] (columns past 2 n_freq zero)
@@ -540,45 +554,49 @@ __global__ void __launch_bounds__(256) k_fourier(const float* __restrict__ X, in
         for (int j = 2 * n_freq; j < ld; ++j) row[j] = 0;
 }
 
-// Squared error of 256 rows and its gradient as BF16 (both layouts), with the
-// gradient's column sums per 256 rows.  out, y: [rows][18].
+// Squared error of 64 rows and its gradient as BF16 (both layouts), with the
+// gradient's column sums per 64 rows.  out, y: [rows][18].  One wavefront per
+// workgroup: with 256 rows each, 8,192 rows were 32 workgroups and took 11 us.
 constexpr int NO = 18;
-constexpr int MSE_ROWS = 256;
-__global__ void __launch_bounds__(256) k_mse(const float* __restrict__ out, const float* __restrict__ y, int rows,
-                                             float inv_n, uint16_t* __restrict__ D, int ld, uint16_t* __restrict__ Dt,
-                                             int ldt, float* __restrict__ col, float* __restrict__ loss) {
-    __shared__ float sh[4];
-    __shared__ float sc[4][NO];
-    const int r = blockIdx.x * MSE_ROWS + threadIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    float e = 0.f;
-    for (int k = 0; k < NO; ++k) {
-        float d = 0.f;
-        if (r < rows) {
-            d = out[int64_t(r) * NO + k] - y[int64_t(r) * NO + k];
+constexpr int MSE_ROWS = 64;
+__global__ void __launch_bounds__(MSE_ROWS) k_mse(const float* __restrict__ out, const float* __restrict__ y, int rows,
+                                                  float inv_n, uint16_t* __restrict__ D, int ld, uint16_t* __restrict__ Dt,
+                                                  int ldt, float* __restrict__ col, float* __restrict__ loss) {
+    const int lane = threadIdx.x, r = blockIdx.x * MSE_ROWS + lane;
+    const bool in = r < rows;
+    float e = 0.f, c[NO];
+#pragma unroll
+    for (int k = 0; k < NO; ++k) c[k] = 0.f;
+    if (in)
+#pragma unroll
+        for (int k = 0; k < NO; ++k) {
+            const float d = out[int64_t(r) * NO + k] - y[int64_t(r) * NO + k];
             e += d * d;
-            d = 2.f * d * inv_n;
-            D[int64_t(r) * ld + k] = f2bf(d);
+            c[k] = 2.f * d * inv_n;
+            D[int64_t(r) * ld + k] = f2bf(c[k]);
         }
-        if (r < ldt) Dt[int64_t(k) * ldt + r] = f2bf(d);
-        float c = d;
-        for (int s = 32; s > 0; s >>= 1) c += __shfl_xor(c, s);
-        if (lane == 0) sc[wave][k] = c;
+    if (r < ldt)
+#pragma unroll
+        for (int k = 0; k < NO; ++k) Dt[int64_t(k) * ldt + r] = f2bf(c[k]);
+    for (int s = 32; s > 0; s >>= 1) {
+        e += __shfl_xor(e, s);
+#pragma unroll
+        for (int k = 0; k < NO; ++k) c[k] += __shfl_xor(c[k], s);
     }
-    for (int s = 32; s > 0; s >>= 1) e += __shfl_xor(e, s);
-    if (lane == 0) sh[wave] = e;
-    __syncthreads();
-    if (threadIdx.x < NO)
-        col[int64_t(blockIdx.x) * NO + threadIdx.x] =
-            ((sc[0][threadIdx.x] + sc[1][threadIdx.x]) + sc[2][threadIdx.x]) + sc[3][threadIdx.x];
-    if (threadIdx.x == 0) loss[blockIdx.x] = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+    if (lane == 0) {
+        loss[blockIdx.x] = e;
+#pragma unroll
+        for (int k = 0; k < NO; ++k) col[int64_t(blockIdx.x) * NO + k] = c[k];
+    }
 }
 
-// The batch's loss in FP64: the workgroups' sums added in order.
-__global__ void k_loss(const float* __restrict__ part, int n, double inv_n, double* __restrict__ dst) {
-    if (threadIdx.x != 0) return;
+// The batch's loss in FP64 by one wavefront: the workgroups' sums, always in the
+// same order.
+__global__ void __launch_bounds__(64) k_loss(const float* __restrict__ part, int n, double inv_n, double* __restrict__ dst) {
     double s = 0.0;
-    for (int i = 0; i < n; ++i) s += part[i];
-    *dst = s * inv_n;
+    for (int i = threadIdx.x; i < n; i += 64) s += part[i];
+    for (int x = 32; x > 0; x >>= 1) s += __shfl_xor(s, x);
+    if (threadIdx.x == 0) *dst = s * inv_n;
 }
 
 // One layer's place in the parameter array and its BF16 copies: Wt [out][ld_in]
@@ -824,7 +842,9 @@ void ensure_train(gfx_mlp& M, int rows) {
     M.train_cap = rows;
 }
 
-// One product, 128 x 128 tiles where they give every CU two workgroups, else 64 x 64.
+// One product, 128 x 128 tiles where they give every CU two workgroups, else 64 x 64:
+// a layer of 256 units over 131,072 rows takes 61 us in tiles of 128 and 66 in
+// tiles of 64; over 8,192 rows tiles of 128 would be 128 workgroups for 256 CUs.
 template <int EPI>
 int gemm(gfx_mlp& M, const GemmArgs& G) {
     const int big = ((G.M + 127) / 128) * ((G.N + 127) / 128);
@@ -936,7 +956,7 @@ void gradient(gfx_mlp& M, int rows, double* loss) {
     W.n = d + 1;
     W.kc = (T.ldt / 64 + R.splits - 1) / R.splits * 64;
     R.splits = (T.ldt + W.kc - 1) / W.kc;
-    int tiles = 0;
+    int tiles = 0, blocks = 0;
     for (int l = 0; l <= d; ++l) {
         GemmArgs& G = W.g[l];
         G.A = M.Ht.p + T.ht[l];
@@ -948,15 +968,16 @@ void gradient(gfx_mlp& M, int rows, double* loss) {
         W.tile0[l] = tiles;
         tiles += ((G.M + 63) / 64) * ((G.N + 63) / 64);
         R.w_off[l] = M.w_off[l];
-        R.b_off[l] = M.b_off[l];
         R.w_part[l] = wp;
         R.size[l] = G.M * G.N;
         R.cols[l] = G.N;
+        R.blk0[l] = blocks;
+        blocks += (R.size[l] + G.N + 63) / 64;
         wp += int64_t(R.splits) * R.size[l];
     }
     W.tile0[d + 1] = tiles;
     k_gemm_grads<<<dim3(tiles, R.splits), 256, 0, M.stream>>>(W);
-    k_reduce_grads<<<int((M.n_params + 63) / 64), 256, 0, M.stream>>>(R, M.w_part.p, M.b_part.p, M.g.p, M.n_params);
+    k_reduce_grads<<<blocks, 256, 0, M.stream>>>(R, M.w_part.p, M.b_part.p, M.g.p);
     GFX_HIP(hipGetLastError());
 }
 

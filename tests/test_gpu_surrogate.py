@@ -278,7 +278,7 @@ def test_network_serves_regions_the_zero_predictor_cannot():
 
 
 @pytest.mark.parametrize("width,depth,n_freq,rows", [(16, 1, 1, 1), (48, 2, 10, 63), (100, 3, 13, 65), (64, 2, 32, 257),
-                                                     (200, 2, 8, 1000), (320, 1, 70, 130)])
+                                                     (200, 2, 8, 1000), (320, 1, 70, 130), (50, 2, 5, 70)])
 def test_mlp_products_at_tile_edges(width, depth, n_freq, rows):
     """Widths, feature counts and rows off the products' tiles (64, 128) and
     padding (64): forward and every gradient block against the CPU model, with
