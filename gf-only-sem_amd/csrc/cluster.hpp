@@ -145,11 +145,10 @@ __device__ __forceinline__ void cluster_body(const ElemArgs& A, const ClusterHea
 #pragma unroll
     for (int c = 0; c < NG9; ++c) g[c] = *reinterpret_cast<const F5*>(A.G + (DIAG ? c * 4 : c) * A.P + pt0);
     const F5 lam = *reinterpret_cast<const F5*>(A.lam + pt0), mu = *reinterpret_cast<const F5*>(A.mu + pt0);
-    int sb = 0, se = 0;
-    if (live) {
-        sb = A.src_off[ew];
-        se = A.src_off[ew + 1];
-    }
+    // one flag per wavefront: few elements have a source, and with the lists' bounds
+    // held over the fields the kernel spilled five registers (131,072 elements,
+    // 1 field: 222 -> 212 us)
+    const bool src = __any(A.src_off[ew] < A.src_off[ew + 1]);
     const int step = A.ctr[0];
     float md[5], mt[5];  // row lane % 4 of D and of its transpose
 #pragma unroll
@@ -236,12 +235,13 @@ __device__ __forceinline__ void cluster_body(const ElemArgs& A, const ClusterHea
                 for (int c = 0; c < 3; ++c) rv.v[c] = -((rx.v[c] + ry.v[c]) + out[s].v[c]);
                 xk[s] = rv;
             }
-            for (int q = sb; q < se; ++q) {  // point sources, as add_sources
-                const int4 en = A.src_ent[q];
-                if (en.x != f || step >= A.nstf) continue;
-                const float amp = A.stf[int64_t(f) * A.nstf + step];
-                for (int s = 0; s < 5; ++s) xk[s].v[en.y] += amp * A.src_w[en.z + qd * 5 + s];
-            }
+            if (src)  // point sources, as add_sources
+                for (int q = A.src_off[ew], se = A.src_off[ew + 1]; q < se; ++q) {
+                    const int4 en = A.src_ent[q];
+                    if (en.x != f || step >= A.nstf) continue;
+                    const float amp = A.stf[int64_t(f) * A.nstf + step];
+                    for (int s = 0; s < 5; ++s) xk[s].v[en.y] += amp * A.src_w[en.z + qd * 5 + s];
+                }
             if (OUT == CL_POINTS)
                 for (int s = 0; s < 5; ++s)
                     *reinterpret_cast<F3*>(A.Rl + (int64_t(f) * A.PR + A.rdst[pt0 + s]) * 3) = xk[s];
