@@ -133,6 +133,30 @@ def test_batch_of_uneven_meshes_equals_single_runs(assembly, groups):
     batch.close()
 
 
+@pytest.mark.parametrize("pieces", [(4,), (3, 5, 4), (9, 1, 8)])
+def test_group_steps_chained_in_one_graph_equal_single_runs(pieces):
+    """A group's graph holds four steps: runs shorter, equal and longer than
+    that, one mesh ending between, give every run's state (residuals of the last
+    step included) and records bit for bit."""
+    meshes = _uneven_meshes()
+    srcs = [[mc.surface_centre_source(m, f0=1.5, t0=0.02) + (2,)] for m in meshes]
+    batched = [_solver(m, s, pygfx.GFX_ASSEMBLY_GATHER) for m, s in zip(meshes, srcs)]
+    single = [_solver(m, s, pygfx.GFX_ASSEMBLY_GATHER) for m, s in zip(meshes, srcs)]
+    until = [10 ** 6, 6, 10 ** 6]
+    batch = pygfx.Batch(batched, groups=2)
+    for n in pieces:
+        batch.run(n, until)
+        for b, s, u in zip(batched, single, until):
+            s.run(max(0, min(n, u - s.step)))
+            assert b.step == s.step and b.n_snapshots == s.n_snapshots
+            for x, y in zip(b.get_state(0), s.get_state(0)):
+                assert np.array_equal(x, y)
+            for x, y in zip(_all_records(b, b.n_snapshots), _all_records(s, s.n_snapshots)):
+                for p, q in zip(x, y):
+                    assert np.array_equal(p, q)
+    batch.close()
+
+
 def test_launch_groups_fall_back_to_branches_when_a_mesh_cannot_share():
     """An attenuating mesh runs its own element kernel form, so a batch holding
     one keeps one branch per mesh even with launch groups requested; dropping it
