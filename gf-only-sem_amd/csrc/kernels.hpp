@@ -901,8 +901,10 @@ __device__ __forceinline__ void cpml_body(const ElemArgs& A, CpmlShared& S, int 
 
 // The PML elements of up to eight ranges, one per set of damped axes, in one
 // launch: the ranges are small (a corner's has tens of elements) and one after
-// the other each left most of the device idle.  All forms hold at most the
-// registers of three waves per SIMD, so sharing a launch costs none of them any.
+// the other each left most of the device idle (12,600 elements, 3 fields: 20 steps
+// with their records 6.7 ms in a launch per range, 3.85 ms in one).  Every form runs
+// at three waves per SIMD by itself too, so a launch of many elements loses
+// nothing: 135,500 elements, 24 fields, 12.1 ms against 12.3.
 // blockIdx.y: fields [y * chunk, (y + 1) * chunk).
 struct CpmlRanges {
     int n;
@@ -913,10 +915,13 @@ template <int MODE>
 __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(3, 3)))
 k_element_cpml(ElemArgs A, CpmlRanges R, int chunk) {
     __shared__ CpmlShared S;
-    const int blk = xcd_block(blockIdx.x, gridDim.x);
+    const int blk = blockIdx.x;
     int r = 0;
     while (r + 1 < R.n && blk >= R.first[r + 1]) ++r;
-    const int e = R.e0[r] + blk - R.first[r];
+    // every XCD takes an eighth of each range: in eighths of the whole launch, the
+    // ranges of two and three axes (twice the work per element) all met on the last
+    // XCDs (135,500 elements, 24 fields: 16.5 ms)
+    const int e = R.e0[r] + xcd_block(blk - R.first[r], R.first[r + 1] - R.first[r]);
     const int f0 = blockIdx.y * chunk, f1 = min(A.nf, f0 + chunk);
     switch (R.ax[r]) {
         case 0: cpml_body<MODE, 0>(A, S, e, f0, f1); break;
