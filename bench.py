@@ -420,11 +420,11 @@ def main():
     kern_of = {"auto": pygfx.GFX_ELEMENT_AUTO, "block": pygfx.GFX_ELEMENT_BLOCK,
                "wave": pygfx.GFX_ELEMENT_WAVE, "pair": pygfx.GFX_ELEMENT_PAIR, "pencil": pygfx.GFX_ELEMENT_PENCIL}
 
-    def launch_config(n_fields):
+    def launch_config(n_fields, **kw):
         if args.assembly == "auto":
             t0 = time.perf_counter()
             pick = pygfx.autotune(mesh, n_fields=n_fields, trial_steps=3, record_capacity=0,
-                                  general_geometry=args.general_geometry)
+                                  general_geometry=args.general_geometry, **kw)
             log(f"autotune F={n_fields}: {pick} ({time.perf_counter() - t0:.1f} s)")
             return dict(assembly=pick["assembly"], element_kernel=pick["element_kernel"],
                         elems_per_block=pick["elems_per_block"], node_field_groups=pick["node_field_groups"])
@@ -494,9 +494,12 @@ def main():
               "element_kernel": knames[int(sb.query("element_kernel"))],
               "elems_per_block": int(sb.query("elems_per_block")),
               "node_field_groups": int(sb.query("node_field_groups"))}
-    kern = {"element": ({"wave": "k_element_wave", "pair": "k_element_pair",
+    clusters = launch["assembly"] == "gather" and not sb.query("n_sls")  # element and interior nodes in one kernel
+    kern = {"element": ({"wave": "k_cluster" if clusters else "k_element_wave", "pair": "k_element_pair",
                          "pencil": "k_element_pencil"}.get(launch["element_kernel"], "k_element"), 1),
             "node_special": ("k_node_special", 3), "node_regular": ("k_node_regular", 4)}
+    if clusters and launch["element_kernel"] == "wave":  # one launch for all other nodes
+        kern["node_special"], kern["node_regular"] = ("k_cluster_nodes", 3), ("k_cluster_nodes", 4)
     dom = max(kern, key=lambda k: tb[k][0])
     kname, which = kern[dom]
     ms_dom, n_dom = tb[dom]
@@ -560,7 +563,11 @@ def main():
     sb.close()
     del sb
     if want_cpml:
-        result["cpml_complete"] = cpml_complete_leg(pygfx, mesh, F, lcb, st, stf, args, value, launch, dims)
+        lcc = launch_config(F, cpml_complete=True)  # its interior elements have no cluster form
+        launch = {"assembly": names[lcc["assembly"]], "element_kernel": knames[lcc["element_kernel"]],
+                  "elems_per_block": lcc["elems_per_block"], "node_field_groups": lcc["node_field_groups"]}
+        result["cpml_complete"] = cpml_complete_leg(pygfx, mesh, F, lcc, st, stf, args, value, launch, dims)
+        result["cpml_complete"]["launch"] = launch
         log("complete C-PML:", json.dumps(result["cpml_complete"]))
     if not args.no_uneven and not args.small:
         result["uneven_batch"] = uneven_workload(pygfx, args.steps, args.warmup)

@@ -2545,7 +2545,15 @@ extern "C" double gfx_solver_algorithmic_bytes(const gfx_solver* s, int which) {
     if (s->has_cpml && s->pml_nodal) node += 56.0 * Gp + F * 96.0 * Gp;
     // the node stage split by kernel: special nodes [0, Ga) carry a and the
     // C-PML terms, regular nodes [Ga, G) only r, u~ and w
-    const double node_reg = (4.0 + F * 60.0) * (G - Ga);
+    double node_reg = (4.0 + F * 60.0) * (G - Ga);
+    if (uses_clusters(*s)) {
+        // the clusters' interior nodes are updated in the element stage: w read,
+        // u~ and w written and 1/m there in place of their residual
+        const double Gin = double(std::max<int64_t>(0, s->G - s->Gi));
+        elem += (4.0 + F * 24.0) * Gin;
+        node -= (4.0 + F * 60.0) * Gin;
+        node_reg -= (4.0 + F * 60.0) * Gin;
+    }
     if (which == 1) return elem;
     if (which == 2) return node;
     if (which == 3) return node - node_reg;
