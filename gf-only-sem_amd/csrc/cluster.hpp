@@ -18,8 +18,8 @@
 // step moves 147 bytes per node and field, of which the fused form needs about
 // 85 (a 2 x 2 x 2 block has 729 nodes for 1,000 points, 343 of them interior).
 // Measured (MI355X; element and node stages of one step, before -> now):
-// 131,072 elements, 1 field: 421 -> 339 us; 36,855 elements, 3 fields: 292 ->
-// 239 us; 23,328 elements, 24 fields: 1,386 -> 1,091 us.
+// 131,072 elements, 1 field: 421 -> 321 us; 36,855 elements, 3 fields: 292 ->
+// 230 us; 23,328 elements, 24 fields: 1,386 -> 1,072 us.
 // Bound: LDS.  At 24 fields its pipes are busy 67 % of the kernel's time (a
 // quarter of that bank conflicts, half of them the eta lines' a = 0 and a = 4
 // planes meeting; no plane padding within the LDS budget removes both theirs and
@@ -368,7 +368,8 @@ __global__ void __launch_bounds__(CLUSTER_THREADS, DIAG ? 4 : 3)
 // spec_blocks take 256 special nodes each, the others 256 regular nodes shared
 // by clusters.  A lane sums its node's entries itself: with one entry per
 // cluster most nodes have none or one beside their own, so there is nothing to
-// stage through LDS and the launch keeps eight wavefronts per SIMD.
+// stage through LDS (special nodes and their C-PML state hold 85 registers, five
+// wavefronts per SIMD; at 23,328 elements, 24 fields the launch moves 5.2 TB/s).
 // blockIdx.y: fields [y * chunk, (y + 1) * chunk).  ctr (may be null): the
 // launch closes the step as k_advance does (no record kernel follows; nothing
 // in the launch reads the counters).

@@ -1166,9 +1166,10 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
         }
     }
     // The cluster kernel (GATHER assembly, elastic, without the complete C-PML)
-    // works on elements that lie together: the curve then runs over the lattice of element-sized cells instead (the element
-    // size per axis from grad xi at the element centres), so that its lowest
-    // three bits number the elements of a 2 x 2 x 2 block
+    // works on elements that lie together: the curve then runs over the lattice
+    // of element-sized cells instead (the element size per axis from grad xi at
+    // the element centres), so that its lowest three bits number the elements of
+    // a 2 x 2 x 2 block
     const bool by_cluster = S.assembly == GFX_ASSEMBLY_GATHER && d.n_sls == 0 && !S.cpml_complete;
     if (by_cluster && d.elem_centroid) {
         double lo[3] = {1e300, 1e300, 1e300}, h[3] = {0, 0, 0};
