@@ -2584,14 +2584,14 @@ struct gfx_batch {
         gfx::DevBuf<gfx::dev::NodeArgs> ntab;
         gfx::DevBuf<gfx::dev::RecArgs> rtab;
         // per-workgroup work of each launch (general and diagonal element
-        // forms, special and regular nodes)
-        gfx::DevBuf<int4> map_gen, map_diag, map_spec, map_reg, map_rec;
+        // forms, special and regular nodes, and the nodes of solvers that take them
+        // all in one launch)
+        gfx::DevBuf<int4> map_gen, map_diag, map_spec, map_reg, map_node, map_rec;
         gfx::DevBuf<int*> ctrs;
         gfx::DevBuf<int> strides;
         // launch shape: workgroups per launch, kernel form
-        int bg = 0, bd = 0, bs = 0, br = 0, bc = 0, n_ctr = 0, rec_threads = 0;
+        int bg = 0, bd = 0, bs = 0, br = 0, bn = 0, bc = 0, n_ctr = 0, rec_threads = 0;
         int fg = 1, kernel = 0, epb = 1;
-        bool direct = false;  // one launch for all nodes
     };
     struct Cached {
         std::vector<char> active;
@@ -2668,7 +2668,7 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
     std::vector<dev::ElemArgs> et;
     std::vector<dev::NodeArgs> nt;
     std::vector<dev::RecArgs> rt;
-    std::vector<int4> eg, ed, es, er, ec;  // one entry per workgroup
+    std::vector<int4> eg, ed, es, er, en, ec;  // one entry per workgroup
     std::vector<int*> ctr;
     std::vector<int> strides;
     int fg = 1, kernel = GFX_ELEMENT_BLOCK, epb = 1;
@@ -2689,10 +2689,12 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
             }
             for (int w = 0; w < (n + S.epb - 1) / S.epb; ++w) m.push_back(make_int4(t, rg.b, n, w));
         }
-        if (args[i].direct) {  // all nodes in the one launch of c.map_spec
+        // each solver's nodes in the form its own launches take: with per-point entries
+        // that depends on its field count, so a group may hold both
+        if (args[i].direct) {
             for (int f = 0; f < S.nf; f += GROUP_CHUNK)
                 for (int w = 0; w < args[i].spec_grid + args[i].reg_grid; ++w)
-                    es.push_back(make_int4(t, args[i].spec_grid, f, w));
+                    en.push_back(make_int4(t, args[i].spec_grid, f, w));
         } else {
             for (int w = 0; w < args[i].spec_grid; ++w) es.push_back(make_int4(t, 0, 0, w));
             for (int w = 0; w < args[i].reg_grid; ++w) er.push_back(make_int4(t, 0, 0, w));
@@ -2716,6 +2718,7 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
     put(c.map_diag, ed);
     put(c.map_spec, es);
     put(c.map_reg, er);
+    put(c.map_node, en);
     put(c.rtab, rt);
     put(c.map_rec, ec);
     put(c.ctrs, ctr);
@@ -2724,12 +2727,12 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
     c.bd = int(ed.size());
     c.bs = int(es.size());
     c.br = int(er.size());
+    c.bn = int(en.size());
     c.bc = int(ec.size());
     c.n_ctr = int(ctr.size());
     c.rec_threads = args[c.members.front()].rec_threads;
     c.fg = fg;
     c.kernel = kernel;
-    c.direct = args[c.members.front()].direct;
     c.epb = epb;
 }
 
@@ -2740,9 +2743,8 @@ void enqueue_group(gfx_batch::Group& c, bool keep_r, hipStream_t st) {
     const dev::ElemArgs* const et = c.etab[keep_r ? 1 : 0].p;
     if (c.bg > 0) launch_element_grp<false>(c.kernel, c.epb, et, c.map_gen, c.bg, st);
     if (c.bd > 0) launch_element_grp<true>(c.kernel, c.epb, et, c.map_diag, c.bd, st);
-    if (c.direct && c.bs > 0)
-        dev::k_cluster_nodes_grp<<<c.bs, 256, 0, st>>>(c.ntab.p, c.map_spec.p, GROUP_CHUNK);
-    else switch (c.fg) {
+    if (c.bn > 0) dev::k_cluster_nodes_grp<<<c.bn, 256, 0, st>>>(c.ntab.p, c.map_node.p, GROUP_CHUNK);
+    switch (c.fg) {
         case 2: launch_nodes_grp<2>(c, st); break;
         case 4: launch_nodes_grp<4>(c, st); break;
         case 8: launch_nodes_grp<8>(c, st); break;

@@ -157,6 +157,35 @@ def test_group_steps_chained_in_one_graph_equal_single_runs(pieces):
     batch.close()
 
 
+@pytest.mark.parametrize("kernel", [pygfx.GFX_ELEMENT_BLOCK, pygfx.GFX_ELEMENT_WAVE])
+@pytest.mark.parametrize("n_fields", [(3, 6), (6, 3), (1, 5, 4)])
+def test_launch_group_of_different_field_counts_equals_single_runs(kernel, n_fields):
+    """One launch group of solvers with few and with many fields: each gives
+    its single run's state and records bit for bit, whichever comes first."""
+    meshes = _uneven_meshes()[:len(n_fields)]
+    batched, single = [], []
+    for m, nf in zip(meshes, n_fields):
+        cells, w, stf = mc.surface_centre_source(m, f0=1.5, t0=0.02)
+        src = [(cells, w, stf * (1.0 + f), f % 3) for f in range(nf)]
+        for to in (batched, single):
+            to.append(_solver(m, src, pygfx.GFX_ASSEMBLY_GATHER, element_kernel=kernel))
+    batch = pygfx.Batch(batched, groups=1)
+    for n in (1, 6):
+        batch.run(n)
+        assert batch.last_groups == 1
+        for b, s in zip(batched, single):
+            s.run(n)
+            assert b.step == s.step and b.n_snapshots == s.n_snapshots
+            for f in range(s.n_fields):
+                for x, y in zip(b.get_state(f), s.get_state(f)):
+                    assert np.any(y) or s.step == 1  # u after the first step is zero
+                    assert np.array_equal(x, y)
+            for x, y in zip(_all_records(b, b.n_snapshots), _all_records(s, s.n_snapshots)):
+                for p, q in zip(x, y):
+                    assert np.array_equal(p, q)
+    batch.close()
+
+
 def test_launch_groups_fall_back_to_branches_when_a_mesh_cannot_share():
     """An attenuating mesh runs its own element kernel form, so a batch holding
     one keeps one branch per mesh even with launch groups requested; dropping it
