@@ -45,7 +45,7 @@ struct ElemRange {
 // per element point (rdst[point]; every element kernel but the cluster form),
 // or one per cluster and node (the cluster kernel).
 struct GatherPlan {
-    bool ready = false;
+    bool ready = false;  // the tables are on the device
     int64_t PR = 0;  // entries per field
     std::vector<int32_t> off_host, pts_host;
     DevBuf<int32_t> off, pts, rdst;
@@ -497,6 +497,8 @@ template <int OUT>
 void launch_clusters(gfx_solver& S, const dev::ElemArgs& a, const ElemRange& rg) {
     const int grid = rg.ce - rg.cb;
     if (grid == 0) return;
+    require(S.cl_head.n >= size_t(rg.ce) && (OUT == dev::CL_POINTS || S.by_cluster.Rl.n > 0),
+            "internal: cluster tables are missing");
     if (rg.diag)
         dev::k_cluster<true, OUT><<<grid, dev::CLUSTER_THREADS, 0, S.stream>>>(a, rg.cb);
     else
@@ -590,7 +592,7 @@ struct StepArgs {
 };
 constexpr int REPB = 2;  // recording cells per workgroup
 
-void require_plan(gfx_solver& S, int which);
+void require_plan(gfx_solver& S, int which, bool entries = true);
 
 // Arguments of one step; points = true: with the residuals left per element
 // point whatever the element kernel (the per-stage entry points).
@@ -603,6 +605,8 @@ StepArgs make_step_args(gfx_solver& S, bool points = false) {
     // are (36 x 36 x 18, 24 fields: 793 us against 847)
     a.direct = clusters || (S.assembly == GFX_ASSEMBLY_GATHER && !points && S.node_fg == 1 && S.nf <= 4);
     require_plan(S, S.assembly != GFX_ASSEMBLY_GATHER ? R_ASSEMBLED : clusters ? R_CLUSTERS : R_POINTS);
+    // the cluster kernel reads its tables also where it leaves one entry per point
+    if (points && uses_clusters(S)) require_plan(S, R_CLUSTERS, false);
     const GatherPlan& gp = clusters ? S.by_cluster : S.by_point;
     const double theta = 1.0 / 8.0;  // pml.cpp:35, coefficients pml.cpp:63-64
     const float c1 = float((1.0 - 2.0 * theta) * 0.5 * S.dt);
@@ -1070,12 +1074,19 @@ HostPlan cluster_plan(const gfx_solver& S, const std::vector<uint32_t>& hib) {
     return h;
 }
 
-// Builds the residual entries a launch needs if they are not there yet (a
-// solver switched to another element kernel, or driven stage by stage).
-void require_plan(gfx_solver& S, int which) {
+// Builds the tables of a plan a launch needs, and (entries) the buffer of its
+// residual entries, if they are not there yet (a solver switched to another
+// element kernel, or driven stage by stage).
+void require_plan(gfx_solver& S, int which, bool entries) {
     if (which == R_ASSEMBLED) return;
     GatherPlan& gp = which == R_CLUSTERS ? S.by_cluster : S.by_point;
-    if (gp.ready) return;
+    if (gp.ready) {
+        if (entries && gp.Rl.n == 0) {
+            gp.Rl.alloc(size_t(S.nf) * gp.PR * 3);
+            gp.Rl.zero(S.stream);
+        }
+        return;
+    }
     std::vector<uint32_t> hib(size_t(S.E) * NP);
     GFX_HIP(hipStreamSynchronize(S.stream));
     GFX_HIP(hipMemcpy(hib.data(), S.ibool.p, hib.size() * 4, hipMemcpyDeviceToHost));
@@ -1090,12 +1101,10 @@ void require_plan(gfx_solver& S, int which) {
         S.cl_ent.upload(h.ent);
         S.cl_bdst.upload(h.bdst);
     }
-    gp.Rl.alloc(size_t(S.nf) * gp.PR * 3);
-    gp.Rl.zero(S.stream);
-    GFX_HIP(hipStreamSynchronize(S.stream));
     gp.off_host = std::move(h.off);
     gp.pts_host = std::move(h.pts);
     gp.ready = true;
+    require_plan(S, which, entries);
 }
 
 void create(const gfx_solver_desc& d, gfx_solver& S) {

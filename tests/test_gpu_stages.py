@@ -45,8 +45,8 @@ def _sources(mesh):
     return [(zc, zw, stf, 2), (bc, bw, bstf, 0)]
 
 
-def _solver(mesh, srcs, assembly, has_cpml):
-    s = pygfx.Solver(mesh, n_fields=len(srcs), assembly=assembly, record_uva=True, has_cpml=has_cpml)
+def _solver(mesh, srcs, assembly, has_cpml, **kw):
+    s = pygfx.Solver(mesh, n_fields=len(srcs), assembly=assembly, record_uva=True, has_cpml=has_cpml, **kw)
     for f, (c, w, stf, d) in enumerate(srcs):
         s.set_source(f, d, c, w, stf)
     return s
@@ -103,6 +103,26 @@ def test_gather_stages_equal_fused_run_bitwise(has_cpml):
     a.run(5)
     b.run(5)
     assert all(np.array_equal(x, y) for x, y in zip(a.get_state(1), b.get_state(1)))
+
+
+@pytest.mark.parametrize("kernel", [pygfx.GFX_ELEMENT_BLOCK, pygfx.GFX_ELEMENT_PENCIL])
+def test_stages_first_after_a_switch_to_the_wave_form(kernel):
+    """A solver made with another element kernel, switched to the wave form and
+    driven stage by stage before any whole step: bit for bit the solver made in
+    the wave form; then whole steps from there."""
+    mesh = _mesh(True)
+    srcs = _sources(mesh)
+    a = _solver(mesh, srcs, pygfx.GFX_ASSEMBLY_GATHER, True)
+    b = _solver(mesh, srcs, pygfx.GFX_ASSEMBLY_GATHER, True, element_kernel=kernel)
+    b.set_launch(pygfx.GFX_ELEMENT_WAVE)
+    for s in (a, b):
+        _drive(s, mesh, srcs, 4)
+    for f in range(2):
+        assert all(np.array_equal(x, y) for x, y in zip(a.get_state(f), b.get_state(f)))
+    a.run(3)
+    b.run(3)
+    for f in range(2):
+        assert all(np.array_equal(x, y) for x, y in zip(a.get_state(f), b.get_state(f)))
 
 
 @pytest.mark.parametrize("assembly", [pygfx.GFX_ASSEMBLY_COLORED, pygfx.GFX_ASSEMBLY_ATOMIC])
