@@ -9,6 +9,7 @@
 
 #include "device.hpp"
 #include "gfx.h"
+#include "judge_work.hpp"
 
 struct gfx_green {
     int n_time = 0, n_node = 0, n_cell = 0;
@@ -29,28 +30,8 @@ struct gfx_green {
     std::vector<double> h_xyz, h_box;
     std::vector<int32_t> h_cell;
     hipStream_t stream = nullptr;
-    // device copies of an interpolation's queries and answers, kept between calls
-    // (up to KEEP queries, 26 MB) and held by one call at a time
-    struct Work {
-        static constexpr size_t KEEP = 262144;
-        gfx::DevBuf<double> q;
-        gfx::DevBuf<int32_t> t, c;
-        gfx::DevBuf<float> o;
-        void fit(size_t n) {
-            if (q.n >= n * 3) return;
-            q.alloc(n * 3);
-            t.alloc(n);
-            c.alloc(n);
-            o.alloc(n * 18);
-        }
-        void trim() {
-            if (t.n <= KEEP) return;
-            q.release();
-            t.release();
-            c.release();
-            o.release();
-        }
-    };
+    // device copies of an interpolation's queries and answers, held by one call at a time
+    using Work = gfx::JudgeWork<gfx::DevBuf>;
     mutable std::mutex work_mu;
     mutable Work work;
     ~gfx_green() {

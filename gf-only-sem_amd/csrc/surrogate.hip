@@ -1110,6 +1110,10 @@ extern "C" gfx_status gfx_green_interpolate(const gfx_green* g, int n, const dou
         if (n == 0) return;
         std::lock_guard<std::mutex> lock(g->work_mu);
         gfx_green::Work& w = g->work;
+        struct Trim {
+            gfx_green::Work& w;
+            ~Trim() { w.trim(); }
+        } trim{w};  // also when the call fails
         w.fit(n);
         GFX_HIP(hipMemcpyAsync(w.q.p, xyz, size_t(n) * 24, hipMemcpyHostToDevice, g->stream));
         GFX_HIP(hipMemcpyAsync(w.t.p, tix, size_t(n) * 4, hipMemcpyHostToDevice, g->stream));
@@ -1119,7 +1123,6 @@ extern "C" gfx_status gfx_green_interpolate(const gfx_green* g, int n, const dou
         GFX_HIP(hipMemcpyAsync(out, w.o.p, size_t(n) * 18 * 4, hipMemcpyDeviceToHost, g->stream));
         if (cell) GFX_HIP(hipMemcpyAsync(cell, w.c.p, size_t(n) * 4, hipMemcpyDeviceToHost, g->stream));
         GFX_HIP(hipStreamSynchronize(g->stream));
-        w.trim();
     });
 }
 

@@ -5,6 +5,8 @@ per axis, cardinality at nodes, partition of unity, clipping, the outside
 error), and the CPU model of the MLP (oracle/mlp.py), pinned by central
 finite differences."""
 import os
+import shutil
+import subprocess
 import sys
 
 import numpy as np
@@ -116,3 +118,65 @@ def test_bf16_rounding_is_nearest_even():
     assert r[3] == 1.0  # below the tie
     assert r[4] == 1.0 + 2 ** -6  # tie between 1+2^-7 (odd) and 1+2^-6 (even) -> even
     assert r[5] == -2.5
+
+
+_WORK = """
+#include <cstdio>
+#include <new>
+#include <stdexcept>
+#include "judge_work.hpp"
+static int fail_at = 0;  // the fail_at-th allocation from now throws
+template <class T> struct Buf {  // as DevBuf: frees, then allocates
+    T* p = nullptr;
+    size_t n = 0;
+    void release() { delete[] p; p = nullptr; n = 0; }
+    void alloc(size_t count) {
+        release();
+        if (fail_at > 0 && --fail_at == 0) throw std::runtime_error("no memory");
+        p = new T[count];
+        n = count;
+    }
+    ~Buf() { release(); }
+};
+using Work = gfx::JudgeWork<Buf>;
+static bool holds(const Work& w, size_t n) { return w.q.n >= 3 * n && w.t.n >= n && w.c.n >= n && w.o.n >= 18 * n; }
+static bool empty(const Work& w) { return !w.q.p && !w.t.p && !w.c.p && !w.o.p; }
+int main() {
+    for (int first = 0; first <= 100; first += 100)
+        for (int k = 1; k <= 4; ++k) {
+            Work w;
+            if (first) w.fit(first);
+            fail_at = k;
+            bool threw = false;
+            try { w.fit(1000); } catch (const std::exception&) { threw = true; }
+            if (!threw || !empty(w)) return 10 * k + 1;
+            w.fit(500);  // what a caller does next: a smaller call
+            if (!holds(w, 500)) return 10 * k + 2;
+            w.fit(1000);
+            if (!holds(w, 1000)) return 10 * k + 3;
+        }
+    Work w;
+    w.fit(Work::KEEP);
+    w.trim();
+    if (!holds(w, Work::KEEP)) return 1;
+    w.fit(Work::KEEP + 1);
+    w.trim();
+    if (!empty(w)) return 2;
+    w.fit(1);
+    return holds(w, 1) ? 0 : 3;
+}
+"""
+
+
+def test_interpolation_workspace_grows_whole_or_not_at_all(tmp_path):
+    """A failed growth of any of the four buffers leaves none of them, so the
+    next, smaller call allocates all four again instead of writing through one
+    that is not there; past its bound the workspace is given back."""
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    src, exe = tmp_path / "work.cpp", tmp_path / "work"
+    src.write_text(_WORK)
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "gf-only-sem_amd", "csrc")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", csrc, str(src),
+                    "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)]).returncode == 0
