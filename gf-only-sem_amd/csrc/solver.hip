@@ -309,7 +309,9 @@ int active_plan(const gfx_solver& S) {
 }
 
 const GatherPlan& plan_of(const gfx_solver& S, int r_src) {
-    return r_src == R_CLUSTERS ? S.by_cluster : S.by_point;
+    const GatherPlan& gp = r_src == R_CLUSTERS ? S.by_cluster : S.by_point;
+    require(gp.ready && gp.Rl.n > 0, "internal: the residual's entries are not there");
+    return gp;
 }
 
 void init_state(gfx_solver& S) {
@@ -796,9 +798,11 @@ void ensure_graph(gfx_solver& S) {
 }
 
 void run_steps(gfx_solver& S, int nsteps) {
-    if (nsteps > 0) S.r_src = active_plan(S);
+    // r_src changes once everything the steps need is there: a plan that finds no
+    // memory leaves the state as it was
     if (S.use_graph && !S.timing) {
         ensure_graph(S);
+        if (nsteps > 0) S.r_src = active_plan(S);
         for (int t = 0; t < nsteps; ++t) {
             GFX_HIP(hipGraphLaunch(S.graph_exec, S.stream));
             advance_host(S);
@@ -819,6 +823,7 @@ void run_steps(gfx_solver& S, int nsteps) {
         GFX_HIP(hipEventRecord(ev[0], S.stream));
     }
     std::vector<char> did_rec(nsteps, 0);
+    if (nsteps > 0) S.r_src = active_plan(S);
     for (int t = 0; t < nsteps; ++t) {
         const bool snap = a.recording && S.step % S.stride == 0;
         a.ea.keep_r = t + 1 == nsteps;  // only the last step's residual can be asked for
@@ -2325,23 +2330,10 @@ extern "C" gfx_status gfx_solver_checkpoint_load(gfx_solver* s, const void* host
         } else {
             put(s->zeta.p, s->zeta.n);
         }
-        if (s->assembly != GFX_ASSEMBLY_GATHER) {
-            put(s->R.p, fl);
-        } else {
-            // the sum at each node's first entry (its own index), zeros elsewhere:
-            // get_state then forms the same r
-            require_plan(*s, active_plan(*s));
-            const GatherPlan& gp = plan_of(*s, active_plan(*s));
-            std::vector<float> hl(size_t(gp.PR) * 3, 0.f);
-            for (int f = 0; f < s->nf; ++f) {
-                const float* r = p + int64_t(f) * s->fstride;
-                std::copy(r, r + size_t(s->G) * 3, hl.begin());
-                GFX_HIP(hipMemcpy(gp.Rl.p + int64_t(f) * gp.PR * 3, hl.data(), hl.size() * 4, hipMemcpyHostToDevice));
-            }
-        }
+        put(s->R.p, fl);
         s->step = int(hdr[5]);
         s->n_snap = int(hdr[6]);
-        s->r_src = active_plan(*s);
+        s->r_src = R_ASSEMBLED;
         s->stage = 0;
         upload_counters(*s);
     });

@@ -8,6 +8,8 @@ Against the lane-per-point block kernel on the same mesh, which sums each
 node's points in another order: both round in FP32, so after a few dozen steps
 the states agree to some 1e-6 relative; the bars are 1e-5 for u and v and 1e-4
 for the acceleration, which is a difference of much larger element forces."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -77,4 +79,60 @@ def test_switching_the_element_kernel_keeps_the_state():
     s.set_launch(pygfx.GFX_ELEMENT_BLOCK, 1)
     s.run(5)
     for x, y in zip(s.get_state(0), after):
+        assert np.array_equal(x, y)
+
+
+class _DeviceMemory:
+    """Holds all but `left` bytes of the free device memory."""
+
+    def __init__(self, left):
+        self.hip = pygfx.lib  # its own HIP runtime
+        self.hip.hipMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
+        self.hip.hipFree.argtypes = [C.c_void_p]
+        free, total = C.c_size_t(0), C.c_size_t(0)
+        assert self.hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        self.p = C.c_void_p()
+        assert free.value > left
+        assert self.hip.hipMalloc(C.byref(self.p), free.value - left) == 0
+
+    def close(self):
+        if self.p:
+            self.hip.hipFree(self.p)
+            self.p = None
+
+
+def test_a_switch_that_finds_no_memory_leaves_the_state():
+    """The entries per point of a solver switched away from the cluster form do
+    not fit beside what the device holds: the run is refused, the state and the
+    acceleration stay readable, and the solver goes on in its earlier form."""
+    mesh = pygfx.build_box(nx=10, ny=10, nz=10, lx=6000.0, ly=6000.0, lz=6000.0,
+                           layers=[(0.0, 6200.0, 3600.0, 2800.0)], pml_xmin=0, pml_xmax=0, pml_ymin=0, pml_ymax=0,
+                           pml_zmax=0, duration=0.2, record_depth_max=0.0)
+    cells, w, stf = mc.buried_source(mesh, t0=0.02)
+    nf, last = 2048, 2047  # 3.1 GB of entries per point, 2.2 GB per cluster
+    solvers = [pygfx.Solver(mesh, n_fields=n, assembly=pygfx.GFX_ASSEMBLY_GATHER, has_cpml=False, record_capacity=0)
+               for n in (nf, 1)]
+    for s, f in zip(solvers, (last, 0)):
+        s.set_source(f, 2, cells, w, stf)
+        s.run(4)
+    s, one = solvers
+    hog = _DeviceMemory(400 << 20)
+    try:
+        s.set_launch(pygfx.GFX_ELEMENT_BLOCK, 1)
+        with pytest.raises(pygfx.GfxError) as ei:
+            s.run(1)
+        assert ei.value.status == 4 and s.step == 4
+        for x, y in zip(s.get_state(last), one.get_state(0)):
+            assert np.any(y) and np.array_equal(x, y)
+        s.set_launch(pygfx.GFX_ELEMENT_WAVE)
+        s.run(1)
+    finally:
+        hog.close()
+    one.run(1)
+    for x, y in zip(s.get_state(last), one.get_state(0)):
+        assert np.array_equal(x, y)
+    for t in (s, one):
+        t.set_launch(pygfx.GFX_ELEMENT_BLOCK, 1)
+        t.run(1)
+    for x, y in zip(s.get_state(last), one.get_state(0)):
         assert np.array_equal(x, y)
