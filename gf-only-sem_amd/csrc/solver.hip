@@ -43,14 +43,14 @@ struct ElemRange {
 // pts_host[off_host[n], off_host[n+1]) of Rl, the first being entry n itself;
 // on the device off / pts list all but that first one.  Two forms: one entry
 // per element point (rdst[point]; every element kernel but the cluster form),
-// or one per cluster and node (the cluster kernel).
+// or one per cluster and node (the cluster kernel).  Both write the solver's
+// one buffer of entries, which has the size of the largest plan run so far.
 struct GatherPlan {
     bool ready = false;  // the tables are on the device
-    int64_t PR = 0;  // entries per field
+    int64_t PR = 0;  // entries per field the plan needs
     std::vector<int32_t> off_host, pts_host;
     DevBuf<int32_t> off, pts, rdst;
     DevBuf<uint8_t> new_cluster;  // point form: slots where a node's next cluster begins
-    DevBuf<float> Rl;
 };
 
 // Which buffer holds the last step's residual.
@@ -102,8 +102,10 @@ struct gfx_solver {
     gfx::DevBuf<uint8_t> pmask;  // nodal C-PML: memory directions in use (bits x, y, z)
     gfx::DevBuf<int32_t> pml_slot, src_off;
     gfx::DevBuf<float> U, W, R, Aacc;
-    // GATHER assembly: residual entries per element point (built when a kernel
-    // needs it) and per cluster
+    // GATHER assembly: residual entries, PR per field, and where they belong: per
+    // element point or per cluster (a plan is built when a kernel needs it)
+    gfx::DevBuf<float> Rl;
+    int64_t PR = 0;
     gfx::GatherPlan by_point, by_cluster;
     // clusters of elements (GATHER): cluster c is the solver elements
     // [cl_begin[c], cl_begin[c+1]); the regular nodes of one cluster only come
@@ -310,7 +312,7 @@ int active_plan(const gfx_solver& S) {
 
 const GatherPlan& plan_of(const gfx_solver& S, int r_src) {
     const GatherPlan& gp = r_src == R_CLUSTERS ? S.by_cluster : S.by_point;
-    require(gp.ready && gp.Rl.n > 0, "internal: the residual's entries are not there");
+    require(gp.ready && S.Rl.n > 0, "internal: the residual's entries are not there");
     return gp;
 }
 
@@ -319,8 +321,7 @@ void init_state(gfx_solver& S) {
     S.W.zero(S.stream);
     S.R.zero(S.stream);
     S.Aacc.zero(S.stream);
-    S.by_point.Rl.zero(S.stream);
-    S.by_cluster.Rl.zero(S.stream);
+    S.Rl.zero(S.stream);
     S.pmem.zero(S.stream);
     S.pnew.zero(S.stream);
     S.zeta.zero(S.stream);
@@ -499,8 +500,7 @@ template <int OUT>
 void launch_clusters(gfx_solver& S, const dev::ElemArgs& a, const ElemRange& rg) {
     const int grid = rg.ce - rg.cb;
     if (grid == 0) return;
-    require(S.cl_head.n >= size_t(rg.ce) && (OUT == dev::CL_POINTS || S.by_cluster.Rl.n > 0),
-            "internal: cluster tables are missing");
+    require(S.cl_head.n >= size_t(rg.ce), "internal: cluster tables are missing");
     if (rg.diag)
         dev::k_cluster<true, OUT><<<grid, dev::CLUSTER_THREADS, 0, S.stream>>>(a, rg.cb);
     else
@@ -595,6 +595,7 @@ struct StepArgs {
 constexpr int REPB = 2;  // recording cells per workgroup
 
 void require_plan(gfx_solver& S, int which, bool entries = true);
+void drop_graph(gfx_solver& S);
 
 // Arguments of one step; points = true: with the residuals left per element
 // point whatever the element kernel (the per-stage entry points).
@@ -624,9 +625,9 @@ StepArgs make_step_args(gfx_solver& S, bool points = false) {
     ea.fstride = S.fstride;
     ea.U = S.U.p;
     ea.R = S.R.p;
-    ea.Rl = gp.Rl.p;
+    ea.Rl = S.Rl.p;
     ea.rdst = gp.rdst.p;
-    ea.PR = gp.PR;
+    ea.PR = S.PR;
     ea.cl_head = S.cl_head.p;
     ea.cl_ent = S.cl_ent.p;
     ea.cl_bdst = S.cl_bdst.p;
@@ -670,8 +671,8 @@ StepArgs make_step_args(gfx_solver& S, bool points = false) {
     na.fstride = S.fstride;
     na.astride = S.astride;
     na.gather = (S.assembly == GFX_ASSEMBLY_GATHER) ? 1 : 0;
-    na.Rl = gp.Rl.p;
-    na.PR = gp.PR;
+    na.Rl = S.Rl.p;
+    na.PR = S.PR;
     na.off = gp.off.p;
     na.pts = gp.pts.p;
     na.minv = S.minv.p;
@@ -1079,17 +1080,42 @@ HostPlan cluster_plan(const gfx_solver& S, const std::vector<uint32_t>& hib) {
     return h;
 }
 
-// Builds the tables of a plan a launch needs, and (entries) the buffer of its
-// residual entries, if they are not there yet (a solver switched to another
-// element kernel, or driven stage by stage).
+// The last step's residual moves from the entries to R, summed as get_state
+// sums them, so that the entries may be written in another form.
+void assemble_residual(gfx_solver& S) {
+    if (S.r_src == R_ASSEMBLED) return;
+    const GatherPlan& gp = plan_of(S, S.r_src);
+    dev::NodeArgs na{};
+    na.G4 = S.G4;
+    na.fstride = S.fstride;
+    na.Rl = S.Rl.p;
+    na.PR = S.PR;
+    na.off = gp.off.p;
+    na.pts = gp.pts.p;
+    na.R = S.R.p;
+    dev::k_scatter_slots<<<dim3(unsigned((S.G4 + 255) / 256), unsigned(S.nf)), 256, 0, S.stream>>>(na, nullptr);
+    GFX_HIP(hipGetLastError());
+    GFX_HIP(hipStreamSynchronize(S.stream));
+    S.r_src = R_ASSEMBLED;
+}
+
+// Builds the tables of a plan a launch needs, and (entries) makes the buffer of
+// entries large enough for it, if they are not there yet (a solver switched to
+// another element kernel, or driven stage by stage).  The old buffer is given
+// back first: 500,000 elements and 24 fields have 18 GB of entries per point and
+// 13 GB per cluster.
 void require_plan(gfx_solver& S, int which, bool entries) {
     if (which == R_ASSEMBLED) return;
     GatherPlan& gp = which == R_CLUSTERS ? S.by_cluster : S.by_point;
     if (gp.ready) {
-        if (entries && gp.Rl.n == 0) {
-            gp.Rl.alloc(size_t(S.nf) * gp.PR * 3);
-            gp.Rl.zero(S.stream);
-        }
+        if (!entries || S.PR >= gp.PR) return;
+        GFX_HIP(hipStreamSynchronize(S.stream));
+        if (S.Rl.n > 0) assemble_residual(S);
+        drop_graph(S);  // captured launches use the buffer
+        S.PR = 0;
+        S.Rl.alloc(size_t(S.nf) * gp.PR * 3);
+        S.PR = gp.PR;
+        S.Rl.zero(S.stream);
         return;
     }
     std::vector<uint32_t> hib(size_t(S.E) * NP);
@@ -1698,7 +1724,8 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
         dv.upload(S.cl_head, std::move(h.head));
         dv.upload(S.cl_ent, std::move(h.ent));
         dv.upload(S.cl_bdst, std::move(h.bdst));
-        dv.alloc(gp.Rl, size_t(S.nf) * gp.PR * 3);
+        S.PR = gp.PR;
+        dv.alloc(S.Rl, size_t(S.nf) * S.PR * 3);
         gp.ready = true;
     }
     std::vector<uint32_t>().swap(hib);
@@ -1866,7 +1893,7 @@ extern "C" gfx_status gfx_solver_get_state(const gfx_solver* s, int field, doubl
             // assembled r of the last step: fixed-order sum of the node's slots, as the
             // node kernels form it
             const GatherPlan& gp = plan_of(*s, s->r_src);
-            const std::vector<float> hl = fetch(s, gp.Rl.p + int64_t(field) * gp.PR * 3, size_t(gp.PR) * 3);
+            const std::vector<float> hl = fetch(s, s->Rl.p + int64_t(field) * s->PR * 3, size_t(s->PR) * 3);
             const std::vector<int32_t>& off = gp.off_host;
             const std::vector<int32_t>& pts = gp.pts_host;
             hR.assign(size_t(s->G4) * 3, 0.f);
@@ -1930,10 +1957,9 @@ extern "C" gfx_status gfx_solver_set_state(gfx_solver* s, int field, const doubl
             GFX_HIP(hipMemcpy(s->Aacc.p + int64_t(field) * s->astride, hA.data(), hA.size() * 4,
                               hipMemcpyHostToDevice));
         if (s->r_src != R_ASSEMBLED) {  // r = m a at the first entry of each node (the node's own index)
-            const GatherPlan& gp = plan_of(*s, s->r_src);
-            std::vector<float> hl(size_t(gp.PR) * 3, 0.f);
+            std::vector<float> hl(size_t(s->PR) * 3, 0.f);
             std::copy(hR.begin(), hR.end(), hl.begin());
-            GFX_HIP(hipMemcpy(gp.Rl.p + int64_t(field) * gp.PR * 3, hl.data(), hl.size() * 4, hipMemcpyHostToDevice));
+            GFX_HIP(hipMemcpy(s->Rl.p + int64_t(field) * s->PR * 3, hl.data(), hl.size() * 4, hipMemcpyHostToDevice));
         }
     });
 }
@@ -2033,6 +2059,7 @@ extern "C" gfx_status gfx_step_element_residual(gfx_solver* s, int ngll, int n_e
         require(s->stage_zeroed || s->assembly != GFX_ASSEMBLY_ATOMIC,
                 "ATOMIC assembly adds into the residual: call gfx_step_zero_residual first");
         StepArgs a = make_step_args(*s, true);
+        assemble_residual(*s);  // the last step's, before its entries are written over
         a.ea.nstf = 0;  // sources come from gfx_step_source_injection
         for (int i = 0; i < int(s->ranges.size());) {
             if (uses_clusters(*s))
@@ -2077,9 +2104,9 @@ extern "C" gfx_status gfx_step_source_injection(gfx_solver* s, int field, int di
         GFX_HIP(hipMemcpy(s->inj_cells.p, cells.data(), cells.size() * 4, hipMemcpyHostToDevice));
         GFX_HIP(hipMemcpy(s->inj_w.p, w.data(), w.size() * 4, hipMemcpyHostToDevice));
         const GatherPlan& gp = s->by_point;
-        dev::k_inject<<<1, 128, 0, s->stream>>>(gp.Rl.p, gp.rdst.p, s->R.p, s->ibool.p, s->inj_cells.p, s->inj_w.p,
+        dev::k_inject<<<1, 128, 0, s->stream>>>(s->Rl.p, gp.rdst.p, s->R.p, s->ibool.p, s->inj_cells.p, s->inj_w.p,
                                                int(cells.size()), direction, float(stf_val),
-                                               gp.PR, s->fstride, field,
+                                               s->PR, s->fstride, field,
                                                s->assembly == GFX_ASSEMBLY_GATHER ? 1 : 0);
         GFX_HIP(hipGetLastError());
     });
@@ -2277,7 +2304,7 @@ extern "C" gfx_status gfx_solver_checkpoint_save(const gfx_solver* s, void* host
             std::fill(p, p + fl, 0.f);
             for (int f = 0; f < s->nf; ++f) {
                 const GatherPlan& gp = plan_of(*s, s->r_src);
-                const std::vector<float> hl = fetch(s, gp.Rl.p + int64_t(f) * gp.PR * 3, size_t(gp.PR) * 3);
+                const std::vector<float> hl = fetch(s, s->Rl.p + int64_t(f) * s->PR * 3, size_t(s->PR) * 3);
                 float* r = p + int64_t(f) * s->fstride;
                 for (int64_t n = 0; n < s->G; ++n)
                     for (int q = gp.off_host[n]; q < gp.off_host[n + 1]; ++q)
@@ -2786,6 +2813,8 @@ constexpr int CHAIN = 4;
 
 // `steps` steps (1, or CHAIN if groupable) of the active solvers as a graph.
 hipGraphExec_t batch_graph(gfx_batch& B, const std::vector<char>& active, int steps) {
+    for (size_t i = 0; i < B.s.size(); ++i)  // may make earlier captures stale
+        if (active[i]) require_plan(*B.s[i], active_plan(*B.s[i]));
     std::vector<int> gens(B.s.size());
     for (size_t i = 0; i < B.s.size(); ++i) gens[i] = B.s[i]->gen;
     const int groups = (B.want_groups > 0 && groupable(B, active)) ? B.want_groups : 0;

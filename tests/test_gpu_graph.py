@@ -186,6 +186,33 @@ def test_launch_group_of_different_field_counts_equals_single_runs(kernel, n_fie
     batch.close()
 
 
+@pytest.mark.parametrize("groups", [0, 1])
+def test_batch_recaptures_after_a_member_was_driven_by_stages(groups):
+    """A member driven stage by stage between batch runs has a larger buffer of
+    residual entries afterwards; the batch's captured steps follow it."""
+    meshes = _uneven_meshes()[:2]
+    srcs = [[mc.surface_centre_source(m, f0=1.5, t0=0.02) + (2,)] for m in meshes]
+    batched = [_solver(m, s, pygfx.GFX_ASSEMBLY_GATHER) for m, s in zip(meshes, srcs)]
+    single = [_solver(m, s, pygfx.GFX_ASSEMBLY_GATHER) for m, s in zip(meshes, srcs)]
+    batch = pygfx.Batch(batched, groups=groups)
+    for n in (5, 6, 1):
+        batch.run(n)
+        m, (cells, w, stf, d), s = meshes[0], srcs[0][0], batched[0]
+        step = s.step
+        s.stage("newmark_predict", m.dt, 0.0)
+        s.stage("element_residual", 5, m.n_elem)
+        s.stage("source_injection", 0, d, float(stf[step]), np.asarray(w, np.float64), len(cells))
+        s.stage("scatter_to_rank")
+        s.stage("newmark_correct", m.dt, 0.0, 0.5)
+        single[0].run(n + 1)
+        single[1].run(n)
+        for b, t in zip(batched, single):
+            assert b.step == t.step
+            for x, y in zip(b.get_state(0), t.get_state(0)):
+                assert np.any(y) and np.array_equal(x, y)
+    batch.close()
+
+
 def test_launch_groups_fall_back_to_branches_when_a_mesh_cannot_share():
     """An attenuating mesh runs its own element kernel form, so a batch holding
     one keeps one branch per mesh even with launch groups requested; dropping it
