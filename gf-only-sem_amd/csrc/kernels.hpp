@@ -1325,6 +1325,15 @@ __global__ void __launch_bounds__(64 * WPB) k_element_wave(ElemArgs A, int e0, i
     wave_body<WPB, MODE, DIAG>(A, e0, ne, xcd_block(blockIdx.x, gridDim.x));
 }
 
+// One launch for the element ranges of several solvers, wavefront form without
+// clusters.
+template <int WPB, int MODE, bool DIAG>
+__global__ void __launch_bounds__(64 * WPB)
+    k_element_wave_grp(const ElemArgs* __restrict__ tab, const int4* __restrict__ map) {
+    const int4 E = map[xcd_block(blockIdx.x, gridDim.x)];
+    wave_body<WPB, MODE, DIAG>(const_row(tab, E.x), E.y, E.z, E.w);
+}
+
 // Fixed-order sum of a node's element contributions (GATHER assembly): the
 // node's first point (its entry at the node id) added to 0, then the other
 // points' entries (slots [kb, ke) of the node) in increasing solver order.

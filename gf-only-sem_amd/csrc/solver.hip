@@ -2612,13 +2612,13 @@ struct gfx_batch {
         gfx::DevBuf<gfx::dev::NodeArgs> ntab;
         gfx::DevBuf<gfx::dev::RecArgs> rtab;
         // per-workgroup work of each launch (general and diagonal element
-        // forms, special and regular nodes, and the nodes of solvers that take them
-        // all in one launch)
-        gfx::DevBuf<int4> map_gen, map_diag, map_spec, map_reg, map_node, map_rec;
+        // forms, by elements and by clusters; special and regular nodes, and the
+        // nodes of solvers that take them all in one launch)
+        gfx::DevBuf<int4> map_gen, map_diag, map_cl_gen, map_cl_diag, map_spec, map_reg, map_node, map_rec;
         gfx::DevBuf<int*> ctrs;
         gfx::DevBuf<int> strides;
         // launch shape: workgroups per launch, kernel form
-        int bg = 0, bd = 0, bs = 0, br = 0, bn = 0, bc = 0, n_ctr = 0, rec_threads = 0;
+        int bg = 0, bd = 0, kg = 0, kd = 0, bs = 0, br = 0, bn = 0, bc = 0, n_ctr = 0, rec_threads = 0;
         int fg = 1, kernel = 0, epb = 1;
     };
     struct Cached {
@@ -2658,7 +2658,7 @@ bool groupable(const gfx_batch& B, const std::vector<char>& active) {
         if (!active[i]) continue;
         const gfx_solver& S = *B.s[i];
         if (S.assembly != GFX_ASSEMBLY_GATHER || (S.has_cpml && !S.pml_nodal) || S.n_sls > 0) return false;
-        if (S.kernel != GFX_ELEMENT_BLOCK && !uses_clusters(S)) return false;
+        if (S.kernel != GFX_ELEMENT_BLOCK && S.kernel != GFX_ELEMENT_WAVE) return false;
         if (first && (S.kernel != first->kernel || S.epb != first->epb || S.node_fg != first->node_fg)) return false;
         if (!first) first = &S;
     }
@@ -2670,7 +2670,12 @@ void launch_element_grp(int kernel, int epb, const dev::ElemArgs* etab, const gf
                         hipStream_t st) {
     constexpr int M = dev::ASM_GATHER;
     if (kernel == GFX_ELEMENT_WAVE) {
-        dev::k_cluster_grp<DIAG><<<grid, dev::CLUSTER_THREADS, 0, st>>>(etab, map.p);
+        switch (epb) {
+            case 1: dev::k_element_wave_grp<1, M, DIAG><<<grid, 64, 0, st>>>(etab, map.p); break;
+            case 2: dev::k_element_wave_grp<2, M, DIAG><<<grid, 128, 0, st>>>(etab, map.p); break;
+            case 4: dev::k_element_wave_grp<4, M, DIAG><<<grid, 256, 0, st>>>(etab, map.p); break;
+            default: dev::k_element_wave_grp<8, M, DIAG><<<grid, 512, 0, st>>>(etab, map.p); break;
+        }
     } else {
         constexpr auto T = [](int e) { return ((e * NP + 63) / 64) * 64; };
         switch (epb) {
@@ -2696,7 +2701,7 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
     std::vector<dev::ElemArgs> et;
     std::vector<dev::NodeArgs> nt;
     std::vector<dev::RecArgs> rt;
-    std::vector<int4> eg, ed, es, er, en, ec;  // one entry per workgroup
+    std::vector<int4> eg, ed, kg, kd, es, er, en, ec;  // one entry per workgroup
     std::vector<int*> ctr;
     std::vector<int> strides;
     int fg = 1, kernel = GFX_ELEMENT_BLOCK, epb = 1;
@@ -2710,11 +2715,11 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
         epb = S.epb;
         for (const auto& rg : S.ranges) {
             const int n = rg.e - rg.b;
-            auto& m = rg.diag ? ed : eg;
-            if (kernel == GFX_ELEMENT_WAVE) {
-                for (int cl = rg.cb; cl < rg.ce; ++cl) m.push_back(make_int4(t, cl, 0, 0));
+            if (uses_clusters(S)) {
+                for (int cl = rg.cb; cl < rg.ce; ++cl) (rg.diag ? kd : kg).push_back(make_int4(t, cl, 0, 0));
                 continue;
             }
+            auto& m = rg.diag ? ed : eg;
             for (int w = 0; w < (n + S.epb - 1) / S.epb; ++w) m.push_back(make_int4(t, rg.b, n, w));
         }
         // each solver's nodes in the form its own launches take: with per-point entries
@@ -2744,6 +2749,8 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
     put(c.ntab, nt);
     put(c.map_gen, eg);
     put(c.map_diag, ed);
+    put(c.map_cl_gen, kg);
+    put(c.map_cl_diag, kd);
     put(c.map_spec, es);
     put(c.map_reg, er);
     put(c.map_node, en);
@@ -2753,6 +2760,8 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
     put(c.strides, strides);
     c.bg = int(eg.size());
     c.bd = int(ed.size());
+    c.kg = int(kg.size());
+    c.kd = int(kd.size());
     c.bs = int(es.size());
     c.br = int(er.size());
     c.bn = int(en.size());
@@ -2771,6 +2780,8 @@ void enqueue_group(gfx_batch::Group& c, bool keep_r, hipStream_t st) {
     const dev::ElemArgs* const et = c.etab[keep_r ? 1 : 0].p;
     if (c.bg > 0) launch_element_grp<false>(c.kernel, c.epb, et, c.map_gen, c.bg, st);
     if (c.bd > 0) launch_element_grp<true>(c.kernel, c.epb, et, c.map_diag, c.bd, st);
+    if (c.kg > 0) dev::k_cluster_grp<false><<<c.kg, dev::CLUSTER_THREADS, 0, st>>>(et, c.map_cl_gen.p);
+    if (c.kd > 0) dev::k_cluster_grp<true><<<c.kd, dev::CLUSTER_THREADS, 0, st>>>(et, c.map_cl_diag.p);
     if (c.bn > 0) dev::k_cluster_nodes_grp<<<c.bn, 256, 0, st>>>(c.ntab.p, c.map_node.p, GROUP_CHUNK);
     switch (c.fg) {
         case 2: launch_nodes_grp<2>(c, st); break;

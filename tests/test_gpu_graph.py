@@ -186,6 +186,39 @@ def test_launch_group_of_different_field_counts_equals_single_runs(kernel, n_fie
     batch.close()
 
 
+def _with_a_repeated_node(mesh):
+    """The mesh with one element that has a node twice (a corner it shared with
+    other elements replaced by the next point): no clusters then."""
+    ib = mesh.ibool.reshape(-1, 125).copy()
+    e = mesh.n_elem // 2
+    corner = next(p for p in (0, 20, 100, 120) if np.count_nonzero(ib == ib[e, p]) > 1)
+    ib[e, corner] = ib[e, corner + 1]
+    return mesh.derive(ibool=ib)
+
+
+@pytest.mark.parametrize("repeated", [(True, True), (True, False)])
+def test_wave_solvers_without_clusters_share_launch_groups(repeated):
+    """Solvers in the wave form whose mesh allows no clusters share launches, with
+    each other and with cluster solvers, and equal their single runs."""
+    meshes = [_with_a_repeated_node(m) if r else m for m, r in zip(_uneven_meshes(), repeated)]
+    batched, single = [], []
+    for m in meshes:
+        cells, w, stf = mc.surface_centre_source(m, f0=1.5, t0=0.02)
+        for to in (batched, single):
+            to.append(_solver(m, [(cells, w, stf, 2), (cells, w, stf, 0)], pygfx.GFX_ASSEMBLY_GATHER,
+                              element_kernel=pygfx.GFX_ELEMENT_WAVE))
+    batch = pygfx.Batch(batched, groups=1)
+    for n in (1, 6):
+        batch.run(n)
+        assert batch.last_groups == 1
+        for b, s in zip(batched, single):
+            s.run(n)
+            for f in range(2):
+                for x, y in zip(b.get_state(f), s.get_state(f)):
+                    assert np.isfinite(y).all() and np.array_equal(x, y)
+    batch.close()
+
+
 @pytest.mark.parametrize("groups", [0, 1])
 def test_batch_recaptures_after_a_member_was_driven_by_stages(groups):
     """A member driven stage by stage between batch runs has a larger buffer of
