@@ -5,8 +5,11 @@
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
+#include <exception>
+#include <mutex>
 #include <stdexcept>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -57,7 +60,9 @@ struct GLL {
 };
 
 // Static-partitioned parallel loop over [0, n) with up to `threads` workers of at
-// least `grain` items each (starting a worker costs tens of microseconds).
+// least `grain` items each (starting a worker costs tens of microseconds).  An
+// exception of fn (the first one) comes out of the call once every worker has
+// ended; parts whose worker cannot be started run in the caller.
 template <typename Fn>
 void parallel_for(int64_t n, Fn&& fn, int threads = 0, int64_t grain = 1) {
     if (threads <= 0) {
@@ -70,15 +75,29 @@ void parallel_for(int64_t n, Fn&& fn, int threads = 0, int64_t grain = 1) {
         return;
     }
     std::vector<std::thread> pool;
+    pool.reserve(threads);
+    std::exception_ptr failed;
+    std::mutex mu;
     const int64_t chunk = (n + threads - 1) / threads;
     for (int t = 0; t < threads; ++t) {
         const int64_t b = t * chunk, e = std::min(n, b + chunk);
         if (b >= e) break;
-        pool.emplace_back([b, e, &fn] {
-            for (int64_t i = b; i < e; ++i) fn(i);
-        });
+        auto part = [b, e, &fn, &failed, &mu] {
+            try {
+                for (int64_t i = b; i < e; ++i) fn(i);
+            } catch (...) {
+                std::lock_guard<std::mutex> lock(mu);
+                if (!failed) failed = std::current_exception();
+            }
+        };
+        try {
+            pool.emplace_back(part);
+        } catch (const std::system_error&) {
+            part();
+        }
     }
     for (auto& th : pool) th.join();
+    if (failed) std::rethrow_exception(failed);
 }
 
 }  // namespace gfx

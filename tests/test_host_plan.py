@@ -7,6 +7,10 @@ call, so on a machine with no HIP device the call must end in
 GFX_ERR_DEVICE ("no HIP device available"), never in an internal check or a
 crash.  A numbering that is not a permutation of the nodes (a node queued
 once per element that touches it) fails the plan's own check instead."""
+import os
+import shutil
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -85,3 +89,39 @@ def test_cluster_tables_plan_at_every_size(nx, ny, nz, morton):
     with pytest.raises(pygfx.GfxError) as ei:
         pygfx.Solver(mesh, assembly=pygfx.GFX_ASSEMBLY_GATHER, has_cpml=False, morton=morton, record_capacity=0)
     assert ei.value.status == GFX_ERR_DEVICE, str(ei.value)
+
+
+_LOOP = """
+#include <atomic>
+#include "common.hpp"
+int main() {
+    using gfx::parallel_for;
+    std::atomic<int> done{0};
+    bool caught = false;
+    try {  // two workers fail, the others finish
+        parallel_for(8192, [&](int64_t i) {
+            if (i == 5 || i == 8000) throw gfx::Error(GFX_ERR_NOMEM, "no memory");
+            ++done;
+        }, 8);
+    } catch (const gfx::Error& e) {
+        caught = e.code == GFX_ERR_NOMEM;
+    }
+    if (!caught || done < 6 * 1024) return 1;
+    done = 0;
+    parallel_for(8191, [&](int64_t) { ++done; }, 5);
+    return done == 8191 ? 0 : 2;
+}
+"""
+
+
+def test_an_exception_in_a_worker_reaches_the_caller(tmp_path):
+    """The host plan's loops allocate inside their workers: a failure there is an
+    error of the call, not the end of the process."""
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    src, exe = tmp_path / "loop.cpp", tmp_path / "loop"
+    src.write_text(_LOOP)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-pthread", "-I", os.path.join(root, "include"), "-I",
+                    os.path.join(root, "gf-only-sem_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)]).returncode == 0
