@@ -60,7 +60,8 @@ struct GLL {
 };
 
 // Static-partitioned parallel loop over [0, n) with up to `threads` workers of at
-// least `grain` items each (starting a worker costs tens of microseconds).  An
+// least `grain` items each (starting a worker costs tens of microseconds; without
+// a grain, loops of fewer than 4,096 items run in the caller).  An
 // exception of fn (the first one) comes out of the call once every worker has
 // ended; parts whose worker cannot be started run in the caller.
 template <typename Fn>
@@ -70,7 +71,7 @@ void parallel_for(int64_t n, Fn&& fn, int threads = 0, int64_t grain = 1) {
         threads = (int)std::min<unsigned>(hc ? hc : 1, 16);
     }
     threads = int(std::min<int64_t>(threads, std::max<int64_t>(1, n / grain)));
-    if (n < 4096 || threads == 1) {
+    if (threads == 1 || (grain <= 1 && n < 4096)) {
         for (int64_t i = 0; i < n; ++i) fn(i);
         return;
     }

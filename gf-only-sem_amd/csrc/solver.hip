@@ -907,6 +907,9 @@ struct DeviceWork {
     }
 };
 
+// Clusters per host thread: the lists of one take about 0.1 ms, a thread's start less.
+constexpr int64_t CLUSTER_GRAIN = 16;
+
 // Clusters of the solver elements [b, e), appended to `begin`: up to CE elements
 // whose keys differ in the lowest three bits only (a 2 x 2 x 2 block of the
 // element lattice), blocks with fewer joined while they fit.  Where that leaves
@@ -1050,7 +1053,7 @@ HostPlan cluster_plan(const gfx_solver& S, const std::vector<uint32_t>& hib) {
         for (size_t t = 0; t < list[0].size(); ++t)
             if (list[0][t].id != H.ibase + int32_t(t)) bad = true;
         for (const Node& x : list[1]) shared[c].push_back(x.id);
-    });
+    }, 0, CLUSTER_GRAIN);
     require(!bad, "internal: cluster lists do not match the node numbering");
     std::vector<int32_t>&off = h.off, &pts = h.pts;
     off.assign(G4 + 1, 0);
@@ -1398,7 +1401,7 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
             }
             std::sort(uniq.begin(), uniq.end());
             for (const uint64_t u : uniq) lists[c].push_back(ids[u & 0xffff]);
-        }, 0, 64);
+        }, 0, CLUSTER_GRAIN);
         S.cl_ok = !repeated;
         cl_first.assign(nc + 1, 0);
         for (int c = 0; c < nc; ++c) cl_first[c + 1] = cl_first[c] + int64_t(lists[c].size());

@@ -109,7 +109,10 @@ int main() {
     if (!caught || done < 6 * 1024) return 1;
     done = 0;
     parallel_for(8191, [&](int64_t) { ++done; }, 5);
-    return done == 8191 ? 0 : 2;
+    if (done != 8191) return 2;
+    done = 0;  // few items of much work each: workers by the grain
+    parallel_for(70, [&](int64_t) { ++done; }, 4, 16);
+    return done == 70 ? 0 : 3;
 }
 """
 
