@@ -114,6 +114,13 @@ struct gfx_solver {
     bool cl_ok = false;
     int64_t Gi = 0;
     std::vector<int32_t> cl_begin;
+    // with the clusters' order: what the order without clusters follows from, in
+    // which earlier builds took their images (caller elements' places on the
+    // centroids' curve, bit 63 for general geometry; memory directions of the C-PML
+    // nodes; number of special nodes)
+    std::vector<uint64_t> curve;
+    std::vector<uint8_t> pml_dirs;
+    int64_t n_special = 0;
     gfx::DevBuf<gfx::dev::ClusterHead> cl_head;
     gfx::DevBuf<uint16_t> cl_ent;
     gfx::DevBuf<int32_t> cl_bdst;
@@ -1214,6 +1221,7 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
     // the element centres), so that its lowest three bits number the elements of
     // a 2 x 2 x 2 block
     const bool by_cluster = S.assembly == GFX_ASSEMBLY_GATHER && d.n_sls == 0 && !S.cpml_complete;
+    if (by_cluster) S.curve = key;
     if (by_cluster && d.elem_centroid) {
         double lo[3] = {1e300, 1e300, 1e300}, h[3] = {0, 0, 0};
         for (int e = 0; e < E; ++e)
@@ -1249,6 +1257,7 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
             diag_el[e] = ok;
         }
     }
+    for (size_t e = 0; e < S.curve.size(); ++e) S.curve[e] |= diag_el[e] ? 0 : uint64_t(1) << 63;
     // complete C-PML: PML elements run their own kernel, after the others
     // and are grouped by the axes their stretch profiles damp (d != 0 at some
     // point), so that each launch carries only the memories those axes use
@@ -1464,9 +1473,13 @@ void create(const gfx_solver_desc& d, gfx_solver& S) {
             hit[n] = 1;
         }
     }
-    int64_t n_special = 0;
-    for (int g = 0; g < G; ++g) n_special += cls[g] > 0 ? 1 : 0;
-    S.Ga = std::min<int64_t>(((n_special + 3) / 4) * 4, ((int64_t(G) + 3) / 4) * 4);
+    for (int g = 0; g < G; ++g) S.n_special += cls[g] > 0 ? 1 : 0;
+    if (by_cluster) {
+        S.pml_dirs.resize(S.Gpml);
+        for (int g = 0; g < G; ++g)
+            if (cls[g] == 2) S.pml_dirs[S.node_new_of_old[g]] = pm_old[g];
+    }
+    S.Ga = std::min<int64_t>(((S.n_special + 3) / 4) * 4, ((int64_t(G) + 3) / 4) * 4);
     S.G4 = ((int64_t(G) + 3) / 4) * 4;
     S.Gi = std::min<int64_t>((S.Gi + 3) / 4 * 4, S.G4);
 
@@ -2240,17 +2253,77 @@ namespace {
 constexpr int64_t CKPT_MAGIC = 0x31544b5043584647LL;  // "GFXCPKT1"
 constexpr int CKPT_WORDS = 16;
 
-uint64_t layout_signature(const gfx_solver& S) {
+uint64_t layout_signature(const gfx_solver& S, const std::vector<int32_t>& node_new_of_old,
+                          const std::vector<int32_t>& int_of_elem) {
     uint64_t h = 1469598103934665603ULL;  // FNV-1a over the solver's numbering
     auto mix = [&](const void* p, size_t n) {
         const unsigned char* c = static_cast<const unsigned char*>(p);
         for (size_t i = 0; i < n; ++i) h = (h ^ c[i]) * 1099511628211ULL;
     };
-    mix(S.node_new_of_old.data(), S.node_new_of_old.size() * sizeof(int32_t));
-    mix(S.int_of_elem.data(), S.int_of_elem.size() * sizeof(int32_t));
+    mix(node_new_of_old.data(), node_new_of_old.size() * sizeof(int32_t));
+    mix(int_of_elem.data(), int_of_elem.size() * sizeof(int32_t));
     const int64_t k[7] = {S.E, S.G, S.nf, S.Ga, S.Gpml, int64_t(S.assembly), int64_t(S.cpml_complete)};
     mix(k, sizeof(k));
     return h;
+}
+uint64_t layout_signature(const gfx_solver& S) { return layout_signature(S, S.node_new_of_old, S.int_of_elem); }
+
+// Where an image in the order without clusters keeps what this solver's order
+// has at a node or C-PML point (empty: the image has the solver's own order).
+struct ImageOrder {
+    std::vector<int32_t> node;   // [G]
+    std::vector<int64_t> point;  // element-local C-PML: [Ppml]
+};
+
+// That order: elements along the curve of their centroids, axis-aligned ones
+// first; nodes by class (C-PML, other special, regular) at their first touch in
+// element order, C-PML nodes by their memory directions first.  False when the
+// image of signature `sig` is not in it.
+bool plain_image_order(const gfx_solver& S, uint64_t sig, ImageOrder& out) {
+    if (S.curve.empty()) return false;
+    const int E = S.E, G = S.G;
+    std::vector<int32_t> elem(E), new_elem(E), caller(G);
+    std::iota(elem.begin(), elem.end(), 0);
+    std::stable_sort(elem.begin(), elem.end(), [&](int a, int b) { return S.curve[a] < S.curve[b]; });
+    for (int i = 0; i < E; ++i) new_elem[elem[i]] = i;
+    for (int g = 0; g < G; ++g) caller[S.node_new_of_old[g]] = g;
+    std::vector<uint32_t> hib(size_t(E) * NP);
+    GFX_HIP(hipMemcpy(hib.data(), S.ibool.p, hib.size() * 4, hipMemcpyDeviceToHost));
+    auto cls = [&](int32_t n) { return n < S.Gpml ? 2 : n < S.n_special ? 1 : 0; };
+    std::vector<int32_t> node(G, -1), number(G);
+    int next = 0;
+    for (int pass = 2; pass >= 0; --pass) {
+        std::vector<int32_t> order;
+        for (int i = 0; i < E; ++i)
+            for (int p = 0; p < NP; ++p) {
+                const int32_t n = int32_t(hib[size_t(S.int_of_elem[elem[i]]) * NP + p]);
+                if (cls(n) == pass && node[n] == -1) {
+                    node[n] = -2;
+                    order.push_back(n);
+                }
+            }
+        if (pass == 2)
+            std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return S.pml_dirs[a] < S.pml_dirs[b]; });
+        for (const int32_t n : order) {
+            node[n] = next;
+            number[caller[n]] = next++;
+        }
+    }
+    if (next != G || layout_signature(S, number, new_elem) != sig) return false;
+    if (ref_elem_pml(S)) {
+        std::vector<int32_t> slot(E);
+        GFX_HIP(hipMemcpy(slot.data(), S.pml_slot.p, size_t(E) * 4, hipMemcpyDeviceToHost));
+        out.point.resize(S.Ppml);
+        int64_t at = 0;
+        for (int i = 0; i < E; ++i) {
+            const int64_t q = slot[S.int_of_elem[elem[i]]];
+            if (q < 0) continue;
+            for (int p = 0; p < NP; ++p) out.point[q * NP + p] = at * NP + p;
+            ++at;
+        }
+    }
+    out.node = std::move(node);
+    return true;
 }
 
 size_t checkpoint_bytes(const gfx_solver& S) {
@@ -2326,10 +2399,14 @@ extern "C" gfx_status gfx_solver_checkpoint_load(gfx_solver* s, const void* host
         // earlier images hold the solids' memories z and the previous deviatoric
         // strain of every point instead of the carry a z + b dev
         const int64_t n_dev = s->n_sls > 0 ? int64_t(s->nf) * 5 * s->E * NP : 0;
+        const char* const other_solver =
+            "checkpoint was taken from a solver with another mesh, field count, assembly or attenuation";
         require(hdr[1] == s->E && hdr[2] == s->G && hdr[3] == s->nf && hdr[4] == s->assembly &&
-                    hdr[7] == int64_t(layout_signature(*s)) && hdr[8] == int64_t(s->pmem.n) &&
-                    hdr[9] == int64_t(s->pnew.n) && hdr[10] == int64_t(s->zeta.n) && (hdr[11] == 0 || hdr[11] == n_dev),
-                "checkpoint was taken from a solver with another mesh, field count, assembly or attenuation");
+                    hdr[8] == int64_t(s->pmem.n) && hdr[9] == int64_t(s->pnew.n) && hdr[10] == int64_t(s->zeta.n) &&
+                    (hdr[11] == 0 || hdr[11] == n_dev),
+                other_solver);
+        ImageOrder order;  // earlier images of solvers with clusters hold the order without
+        require(hdr[7] == int64_t(layout_signature(*s)) || plain_image_order(*s, uint64_t(hdr[7]), order), other_solver);
         require(bytes >= checkpoint_bytes(*s) + size_t(hdr[11]) * 4, "checkpoint image truncated");
         const float* p = reinterpret_cast<const float*>(static_cast<const char*>(host) + CKPT_WORDS * 8);
         const size_t fl = size_t(s->nf) * s->fstride, al = size_t(s->nf) * s->astride;
@@ -2338,11 +2415,43 @@ extern "C" gfx_status gfx_solver_checkpoint_load(gfx_solver* s, const void* host
             if (n) GFX_HIP(hipMemcpy(d, p, n * 4, hipMemcpyHostToDevice));
             p += n;
         };
-        put(s->U.p, fl);
-        put(s->W.p, fl);
-        put(s->Aacc.p, al);
-        put(s->pmem.p, s->pmem.n);
-        put(s->pnew.p, s->pnew.n);
+        // nodes [0, n) of every field, `stride` apart; rows of one value per C-PML node or point
+        const bool own = order.node.empty();
+        std::vector<float> h;
+        auto put_nodes = [&](float* d, int64_t stride, int64_t n, const float* r) {
+            if (own) return put(d, size_t(s->nf) * stride);
+            for (int f = 0; f < s->nf; ++f, p += stride) {
+                h.assign(stride, 0.f);
+                for (int64_t g = 0; g < n; ++g) {
+                    const int64_t j = order.node[g];
+                    // a is kept at nodes [0, Ga): the last three may be regular ones, of which
+                    // the image has others and keeps r = m a instead
+                    const double m = s->mass_node[g];
+                    for (int c = 0; c < 3; ++c)
+                        h[g * 3 + c] = !r || j < n ? p[j * 3 + c]
+                                       : m > 0.0   ? r[int64_t(f) * s->fstride + j * 3 + c] * float(1.0 / m)
+                                                   : 0.f;
+                }
+                GFX_HIP(hipMemcpy(d + int64_t(f) * stride, h.data(), h.size() * 4, hipMemcpyHostToDevice));
+            }
+        };
+        auto put_rows = [&](float* d, size_t n, int64_t rows) {
+            if (own || n == 0) return put(d, n);
+            const int64_t len = int64_t(n) / (s->nf * rows), used = s->pml_nodal ? s->Gpml : s->Ppml;
+            h.resize(n);
+            std::copy(p, p + n, h.begin());
+            for (int64_t k = 0; k < s->nf * rows; ++k)
+                for (int64_t q = 0; q < used; ++q)
+                    h[k * len + q] = p[k * len + (s->pml_nodal ? int64_t(order.node[q]) : order.point[q])];
+            GFX_HIP(hipMemcpy(d, h.data(), n * 4, hipMemcpyHostToDevice));
+            p += n;
+        };
+        const float* const r = p + 2 * fl + al + s->pmem.n + s->pnew.n + s->zeta.n + size_t(hdr[11]);
+        put_nodes(s->U.p, s->fstride, s->G, nullptr);
+        put_nodes(s->W.p, s->fstride, s->G, nullptr);
+        put_nodes(s->Aacc.p, s->astride, std::min<int64_t>(s->Ga, s->G), r);
+        put_rows(s->pmem.p, s->pmem.n, 9);
+        put_rows(s->pnew.p, s->pnew.n, 3);
         if (hdr[11] != 0) {
             const int64_t P = int64_t(s->E) * NP, L = s->n_sls;
             const std::vector<float> a = fetch(s, s->att_a.p, size_t(L * P)), b = fetch(s, s->att_b.p, size_t(L * P));
@@ -2360,7 +2469,7 @@ extern "C" gfx_status gfx_solver_checkpoint_load(gfx_solver* s, const void* host
         } else {
             put(s->zeta.p, s->zeta.n);
         }
-        put(s->R.p, fl);
+        put_nodes(s->R.p, s->fstride, s->G, nullptr);
         s->step = int(hdr[5]);
         s->n_snap = int(hdr[6]);
         s->r_src = R_ASSEMBLED;

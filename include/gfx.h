@@ -300,9 +300,11 @@ gfx_status gfx_solver_get_record(const gfx_solver* s, int field, int snap, doubl
  * displacement, velocity, acceleration where kept, C-PML memory, the last
  * assembled residual, step and snapshot counters).  Loading it into a solver
  * built from the same inputs, field count and assembly continues the run bit
- * for bit; any other solver rejects it (GFX_ERR_INVALID).  This goes beyond
- * the reference's restart file (forward/share/src/restart.cpp:120-152), which
- * keeps neither the C-PML memory nor the exact step state. */
+ * for bit; any other solver rejects it (GFX_ERR_INVALID).  Images of GATHER
+ * solvers from before the cluster kernel hold another element and node order
+ * and are converted: the state is exact, and the run goes on with the cluster
+ * kernel's order of sums.  This goes beyond the reference's restart file
+ * (forward/share/src/restart.cpp:120-152), which keeps neither the C-PML memory nor the exact step state. */
 gfx_status gfx_solver_checkpoint_size(const gfx_solver* s, size_t* bytes);
 gfx_status gfx_solver_checkpoint_save(const gfx_solver* s, void* host, size_t bytes);
 gfx_status gfx_solver_checkpoint_load(gfx_solver* s, const void* host, size_t bytes);

@@ -9,6 +9,7 @@ node's points in another order: both round in FP32, so after a few dozen steps
 the states agree to some 1e-6 relative; the bars are 1e-5 for u and v and 1e-4
 for the acceleration, which is a difference of much larger element forces."""
 import ctypes as C
+import os
 
 import numpy as np
 import pytest
@@ -17,6 +18,8 @@ import meshcases as mc
 import pygfx
 
 pytestmark = pytest.mark.gpu
+
+GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "images_without_clusters.npz")
 
 
 def _run(mesh, nf, kernel, has_cpml, morton, steps=30):
@@ -202,3 +205,59 @@ def test_both_forms_share_one_buffer_of_entries():
         for x, y in zip(s.get_state(nf - 1), ref.get_state(nf - 1)):
             assert np.array_equal(x, y)
         del s, ref
+
+
+def image_case(form):
+    """The solver of the stored images (tests/golden/README.md): axis-aligned and
+    general elements, C-PML nodes of several direction sets, one recorded cell, a
+    number of special nodes that is no multiple of four; memory per node or, with
+    one element's coefficient changed, per element."""
+    nx = 4 if form == "nodal" else 3
+    mesh = pygfx.build_box(nx=nx, ny=2, nz=2, lx=700.0 * nx, ly=1500.0, lz=1300.0,
+                           layers=[(700.0, 5000.0, 2900.0, 2500.0), (0.0, 6200.0, 3600.0, 2800.0)], pml_xmin=1,
+                           pml_xmax=0, pml_ymin=0, pml_ymax=0, pml_zmax=1, f0_pml=1.5, duration=1.0,
+                           record_depth_max=0.0)
+    dd = mesh.dxi_dx.reshape(-1, 125, 9).copy()
+    dd[::3, :, 1] = 1e-9 * dd[::3, :, 0]  # every third element takes the general form
+    mesh = mesh.derive(dxi_dx=dd.reshape(-1))
+    if form == "element":
+        al = mesh.coef_alpha.reshape(-1, 125, 9).copy()
+        use = (mesh.pml_region[:, None] != 0) & (mesh.coef_abar.reshape(-1, 125, 5)[:, :, 2] != 0)
+        ids, n = np.unique(mesh.ibool.reshape(-1, 125)[use], return_counts=True)
+        e, q = (int(x[0]) for x in np.nonzero(use & (mesh.ibool.reshape(-1, 125) == ids[n >= 2][0])))
+        al[e, q, 0] *= 0.999
+        mesh = mesh.derive(coef_alpha=al.reshape(-1))
+    cells, w, stf = mc.buried_source(mesh, depth=500.0, t0=0.05)
+    s = pygfx.Solver(mesh, n_fields=1, assembly=pygfx.GFX_ASSEMBLY_GATHER, record_capacity=1,
+                     rec_cell=np.array([mesh.n_elem - 1], np.int32))
+    s.set_source(0, 2, cells, w, stf)
+    return mesh, s
+
+
+@pytest.mark.parametrize("form", ["nodal", "element"])
+def test_images_in_the_order_without_clusters_load(form):
+    """An image taken before elements and nodes were ordered by clusters loads
+    into the solver of the same inputs: the state it was taken at bit for bit,
+    and five steps on from there the displacement that build reached, to the
+    rounding of another order of sums (1e-5)."""
+    mesh, s = image_case(form)
+    assert s.query("pml_nodal") == (form == "nodal")
+    assert form == "element" or 0 < s.query("diag_elements") < mesh.n_elem
+    with np.load(GOLDEN) as z:
+        image, at, later = (z[f"{form}_{k}"] for k in ("image", "at", "later"))
+    s.restore(image.tobytes())
+    assert s.step == 6
+    for x, y in zip(s.get_state(0), at):
+        assert np.any(y) and np.array_equal(x, y.astype(np.float64))
+    own = s.checkpoint()  # from here on in this solver's own order
+    s.run(5)
+    after = s.get_state(0)
+    assert mc.rel_l2(after[0], later) <= 1e-5
+    s.restore(own)
+    s.run(5)
+    for x, y in zip(s.get_state(0), after):
+        assert np.array_equal(x, y)
+    bad = image.copy()
+    bad[56] ^= 1  # another numbering is refused
+    with pytest.raises(pygfx.GfxError):
+        s.restore(bad.tobytes())
