@@ -152,6 +152,7 @@ struct gfx_solver {
     double t_elem = 0, t_elem_pml = 0, t_spec = 0, t_reg = 0, t_rec = 0, t_total = 0;
     int n_elem_launch = 0, n_elem_pml_launch = 0, n_spec_launch = 0, n_reg_launch = 0, n_rec_launch = 0,
         n_total_launch = 0;
+    int elem_launches = 0, elem_pml_launches = 0;  // element launches of the last enqueued step
     // complete C-PML: index of the first range when the PML ranges close the
     // element launches (one colour), else -1 (their time is then not split out)
     int pml_tail = -1;
@@ -743,8 +744,11 @@ void enqueue_step(gfx_solver& S, const StepArgs& a, bool record, hipEvent_t* ev)
         dev::k_zero<<<a.zero_grid, 256, 0, S.stream>>>(reinterpret_cast<float4*>(S.R.p), a.r4);
     const int nr = int(S.ranges.size());
     const int pml_tail = S.pml_tail >= 0 ? S.pml_tail : nr;
+    S.elem_launches = S.elem_pml_launches = 0;
     for (int i = 0; i < nr;) {
         if (ev && i == pml_tail) GFX_HIP(hipEventRecord(ev[0], S.stream));
+        ++S.elem_launches;
+        if (i >= pml_tail) ++S.elem_pml_launches;
         i = launch_element(S, a.ea, i);
     }
     if (ev && pml_tail == nr) GFX_HIP(hipEventRecord(ev[0], S.stream));
@@ -843,7 +847,6 @@ void run_steps(gfx_solver& S, int nsteps) {
     if (S.timing) {
         S.t_elem = S.t_elem_pml = S.t_spec = S.t_reg = S.t_rec = S.t_total = 0;
         S.n_elem_launch = S.n_elem_pml_launch = S.n_spec_launch = S.n_reg_launch = S.n_rec_launch = 0;
-        const int n_pml_ranges = S.pml_tail >= 0 ? int(S.ranges.size()) - S.pml_tail : 0;
         for (int t = 0; t < nsteps; ++t) {
             float e = 0, ep = 0, b = 0, c = 0, d = 0;
             const size_t o = size_t(t) * EV;
@@ -857,8 +860,8 @@ void run_steps(gfx_solver& S, int nsteps) {
             S.t_spec += b;
             S.t_reg += c;
             S.t_rec += d;
-            S.n_elem_launch += int(S.ranges.size());
-            S.n_elem_pml_launch += n_pml_ranges;
+            S.n_elem_launch += S.elem_launches;
+            S.n_elem_pml_launch += S.elem_pml_launches;
             S.n_spec_launch += a.spec_grid > 0;
             S.n_reg_launch += a.reg_grid > 0;
             S.n_rec_launch += did_rec[t];

@@ -311,15 +311,18 @@ gfx_status gfx_solver_checkpoint_load(gfx_solver* s, const void* host, size_t by
 
 /* Per-kernel device time of the last gfx_solver_run (HIP events on the
  * solver's stream).  name is "element", "node" (both node kernels),
- * "node_special", "node_regular", "record" or "total"; returns milliseconds
- * summed over the run and the launch count. */
+ * "node_special", "node_regular", "record" or "total", or "element_pml" (the
+ * complete C-PML's element launches, within "element"; 0 under COLORED
+ * assembly); returns milliseconds summed over the run and the launch count. */
 gfx_status gfx_solver_kernel_time(const gfx_solver* s, const char* name, double* ms,
                                   int* launches);
 /* Enable/disable per-kernel event timing (default off). */
 gfx_status gfx_solver_set_timing(gfx_solver* s, int enable);
 
 /* Switch the element kernel form and elements per workgroup of an existing
- * solver (same contract as the descriptor fields; results do not depend on it). */
+ * solver (same contract as the descriptor fields).  Results are the same up to
+ * the rounding of sums: under GATHER assembly the wave form of elastic elements
+ * sums a node's points cluster by cluster, the other forms one after the other. */
 gfx_status gfx_solver_set_launch(gfx_solver* s, int element_kernel, int elems_per_block);
 /* Capture one whole step into a HIP graph and replay it for every step of
  * gfx_solver_run (1), or launch kernel by kernel (0, default).  The step and
@@ -347,8 +350,8 @@ gfx_status gfx_autotune(const gfx_solver_desc* base, int trial_steps, gfx_solver
  * (elements on the diagonal-geometry form), "n_sls"; with the complete C-PML
  * "cpml_complete", "cpml_points" (PML element points), "cpml_memories"
  * (memories in use per field, summed over those points) and "cpml_groups"
- * (launches of the PML element kernel per step: one per set of damped axes,
- * and per colour under COLORED assembly). */
+ * (groups of PML elements with one set of damped axes, per colour under COLORED
+ * assembly; up to eight groups of a colour share a launch). */
 gfx_status gfx_solver_query(const gfx_solver* s, const char* key, double* value);
 
 /* Algorithmic HBM bytes per step for the current problem (each array counted

@@ -107,6 +107,21 @@ def _check(mesh, c, w, stf, direction, assembly, n_mid, sensitivity=False):
                 assert mc.rel_l2(other[k], mid[k]) > 100 * TOL, k
 
 
+def test_kernel_times_count_the_launches_made():
+    """The groups of PML elements share one launch per step (one colour): the
+    launch counts beside the kernel times are those of the launches."""
+    mesh = mc.small_layered(nx=6, ny=5, nz=5, pml=1, jitter=0.0, duration=0.5, want_profiles=True)
+    c, w, stf = mc.surface_centre_source(mesh)
+    s = _gpu(mesh, [(c, w, stf, 2)], pygfx.GFX_ASSEMBLY_GATHER)
+    assert s.query("cpml_groups") == 7
+    s.set_timing(True)
+    s.run(4)
+    ms, n = s.kernel_time("element_pml")
+    assert n == 4 and ms > 0
+    assert s.kernel_time("element")[1] == 8  # the interior elements' and the PML's
+    assert s.kernel_time("node_special")[1] <= 4 and s.kernel_time("total")[1] == 4
+
+
 @pytest.mark.parametrize("assembly", [pygfx.GFX_ASSEMBLY_COLORED, pygfx.GFX_ASSEMBLY_ATOMIC,
                                       pygfx.GFX_ASSEMBLY_GATHER])
 def test_halfspace_matches_oracle(assembly):
