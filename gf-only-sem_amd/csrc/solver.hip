@@ -610,11 +610,17 @@ void drop_graph(gfx_solver& S);
 StepArgs make_step_args(gfx_solver& S, bool points = false) {
     StepArgs a;
     const bool clusters = !points && uses_clusters(S);
-    // entries per element point: with few fields the one launch without LDS staging
-    // is faster (28 x 26 x 15 elements, 3 fields: 67 us against 77 in two launches;
-    // 4,000 elements, 1 field: 21 us a step against 28), with many the staged sums
-    // are (36 x 36 x 18, 24 fields: 793 us against 847)
-    a.direct = clusters || (S.assembly == GFX_ASSEMBLY_GATHER && !points && S.node_fg == 1 && S.nf <= 4);
+    // Entries per element point: on a small mesh the one launch without LDS staging
+    // is faster, on a large one, whose entries no cache holds, the staged sums are.
+    // A step in us, direct against two staged launches, block kernel, 1 / 4 fields:
+    //   0.3 M nodes  22 / 49  against  32 / 72     2.4 M nodes  113 / 373  against  120 / 375
+    //   1.5 M nodes  76 / 241 against  83 / 247    4.2 M nodes  221 / 632  against  218 / 626
+    // (131,072 elements, 8.5 M nodes, 1 field: 430 against 427); with three solids
+    // 0.7 M nodes 77 / 270 against 81 / 279, 2.4 M nodes 297 / 866 against 295 / 854.
+    // More fields bring the line down (24 fields: between 1.1 M and 1.5 M nodes).
+    constexpr int64_t DIRECT_NODES = 2000000;
+    a.direct = clusters || (S.assembly == GFX_ASSEMBLY_GATHER && !points && S.node_fg == 1 && S.nf <= 4 &&
+                            S.G <= DIRECT_NODES);
     require_plan(S, S.assembly != GFX_ASSEMBLY_GATHER ? R_ASSEMBLED : clusters ? R_CLUSTERS : R_POINTS);
     // the cluster kernel reads its tables also where it leaves one entry per point
     if (points && uses_clusters(S)) require_plan(S, R_CLUSTERS, false);
@@ -2838,7 +2844,7 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
             for (int w = 0; w < (n + S.epb - 1) / S.epb; ++w) m.push_back(make_int4(t, rg.b, n, w));
         }
         // each solver's nodes in the form its own launches take: with per-point entries
-        // that depends on its field count, so a group may hold both
+        // that depends on its fields and nodes, so a group may hold both
         if (args[i].direct) {
             for (int f = 0; f < S.nf; f += GROUP_CHUNK)
                 for (int w = 0; w < args[i].spec_grid + args[i].reg_grid; ++w)

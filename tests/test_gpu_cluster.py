@@ -59,6 +59,26 @@ def test_cluster_kernel_matches_block_kernel(nx, ny, nz, nf, jitter, has_cpml, m
             assert mc.rel_l2(p, q) <= bar
 
 
+@pytest.mark.parametrize("nf,has_cpml,n_sls", [(1, True, 0), (4, False, 0), (3, True, 2)])
+def test_one_node_launch_equals_staged_launches(nf, has_cpml, n_sls):
+    """Entries per element point: small meshes of few fields take all nodes in one
+    launch; two field groups per workgroup keep the two staged launches.  The
+    same sums in the same order: bit for bit."""
+    mesh = mc.small_layered(duration=0.8, n_sls=n_sls, q_mu=[60.0, 90.0, 120.0], att_fmin=0.1, att_fmax=4.0)
+    cells, w, stf = mc.buried_source(mesh)
+    states = []
+    for groups in (1, 2):
+        s = pygfx.Solver(mesh, n_fields=nf, assembly=pygfx.GFX_ASSEMBLY_GATHER, element_kernel=pygfx.GFX_ELEMENT_BLOCK,
+                         has_cpml=has_cpml, node_field_groups=groups)
+        for f in range(nf):
+            s.set_source(f, f % 3, cells, w, stf)
+        s.run(25)
+        states.append([s.get_state(f) for f in range(nf)])
+    for a, b in zip(*states):
+        for x, y in zip(a, b):
+            assert np.any(y) and np.array_equal(x, y)
+
+
 def test_switching_the_element_kernel_keeps_the_state():
     """A solver moved between the cluster and the block form mid-run (each has
     its own residual entries) continues from the same state, and the
