@@ -367,9 +367,12 @@ __global__ void __launch_bounds__(CLUSTER_THREADS, DIAG ? 4 : 3)
 // The nodes the cluster kernel leaves, in one launch: workgroups below
 // spec_blocks take 256 special nodes each, the others 256 regular nodes shared
 // by clusters.  A lane sums its node's entries itself: with one entry per
-// cluster most nodes have none or one beside their own, so there is nothing to
+// cluster most nodes have none or one beside their own, so little is left to
 // stage through LDS (special nodes and their C-PML state hold 85 registers, five
-// wavefronts per SIMD; at 23,328 elements, 24 fields the launch moves 5.2 TB/s).
+// wavefronts per SIMD; at 23,328 elements, 24 fields the launch moves 5.2 TB/s,
+// at 500,000 the special nodes by themselves 4.5: 8.3 ms, where sums staged
+// through LDS over entries per point took 7.5; the shared regular nodes 3.2
+// against 7.3).
 // blockIdx.y: fields [y * chunk, (y + 1) * chunk).  ctr (may be null): the
 // launch closes the step as k_advance does (no record kernel follows; nothing
 // in the launch reads the counters).

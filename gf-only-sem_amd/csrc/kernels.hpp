@@ -904,7 +904,8 @@ __device__ __forceinline__ void cpml_body(const ElemArgs& A, CpmlShared& S, int 
 // the other each left most of the device idle (12,600 elements, 3 fields: 20 steps
 // with their records 6.7 ms in a launch per range, 3.85 ms in one).  Every form runs
 // at three waves per SIMD by itself too, so a launch of many elements loses
-// nothing: 135,500 elements, 24 fields, 12.1 ms against 12.3.
+// nothing: 135,500 elements, 24 fields, in turn on one box 13.09 and 13.10 ms against
+// 13.22 and 13.23.
 // blockIdx.y: fields [y * chunk, (y + 1) * chunk).
 struct CpmlRanges {
     int n;

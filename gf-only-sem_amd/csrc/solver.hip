@@ -2936,11 +2936,12 @@ std::vector<std::vector<int>> split_groups(const gfx_batch& B, const std::vector
 }
 
 // Steps of a group's launches in one graph: the groups share no data, so that
-// only the whole graph joins them again.  One step a graph left the device idle
-// for 23 of 300 us between steps (20 meshes of 500 to 4,000 elements, 3 fields, 4
-// groups: 20 steps with their records 9.07 -> 8.24 ms; graphs of eight steps 8.47, as
-// the last four run alone); the steps before the last also store no interior
-// residuals.
+// only the whole graph joins them again; one step a graph leaves the device idle
+// between steps.  The steps before the last also store no interior residuals.
+// 20 meshes of 500 to 4,000 elements, 3 fields, 4 groups, us a step in runs of 20
+// / of 400: one step a graph 261 / 259, two 239 / 238, four 229 / 228, eight
+// 233 / 223, sixteen 231 / 221.  Four has most of it without the longer graphs'
+// loss where a run's last steps are too few for them and run one by one.
 constexpr int CHAIN = 4;
 
 // `steps` steps (1, or CHAIN if groupable) of the active solvers as a graph.
