@@ -498,6 +498,8 @@ def main():
     kern = {"element": ({"wave": "k_cluster" if clusters else "k_element_wave", "pair": "k_element_pair",
                          "pencil": "k_element_pencil"}.get(launch["element_kernel"], "k_element"), 1),
             "node_special": ("k_node_special", 3), "node_regular": ("k_node_regular", 4)}
+    if sb.query("n_sls"):
+        kern["element"] = ("k_element_att", 1)
     if clusters and launch["element_kernel"] == "wave":  # one launch for all other nodes
         kern["node_special"], kern["node_regular"] = ("k_cluster_nodes", 3), ("k_cluster_nodes", 4)
     dom = max(kern, key=lambda k: tb[k][0])
