@@ -2860,8 +2860,9 @@ void build_group(gfx_batch& B, gfx_batch::Group& c, const std::vector<StepArgs>&
         strides.push_back(S.stride);
     }
     auto put = [](auto& buf, const auto& v) {
-        buf.alloc(std::max<size_t>(v.size(), 1));
-        if (!v.empty()) GFX_HIP(hipMemcpy(buf.p, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice));
+        if (v.empty()) return;  // a launch of no workgroups is not made
+        buf.alloc(v.size());
+        GFX_HIP(hipMemcpy(buf.p, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice));
     };
     for (int keep = 0; keep < 2; ++keep) {
         for (auto& a : et) a.keep_r = keep;
