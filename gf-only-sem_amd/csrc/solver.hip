@@ -1135,6 +1135,7 @@ void require_plan(gfx_solver& S, int which, bool entries) {
         S.Rl.alloc(size_t(S.nf) * gp.PR * 3);
         S.PR = gp.PR;
         S.Rl.zero(S.stream);
+        GFX_HIP(hipStreamSynchronize(S.stream));  // a batch launches on other streams
         return;
     }
     std::vector<uint32_t> hib(size_t(S.E) * NP);

@@ -246,6 +246,32 @@ def test_batch_recaptures_after_a_member_was_driven_by_stages(groups):
     batch.close()
 
 
+@pytest.mark.parametrize("groups", [0, 1])
+def test_batch_after_a_switch_of_the_element_kernel(groups):
+    """The entries of another element form are made by the batch's first run: many
+    fields, so that clearing them takes as long as the first launches."""
+    meshes = _uneven_meshes()[:2]
+    batched, single = [], []
+    for m in meshes:
+        cells, w, stf = mc.surface_centre_source(m, f0=1.5, t0=0.02)
+        for to in (batched, single):
+            s = pygfx.Solver(m, n_fields=256, assembly=pygfx.GFX_ASSEMBLY_GATHER, record_capacity=0)
+            for f in (0, 255):
+                s.set_source(f, f % 3, cells, w, stf)
+            s.run(3)
+            to.append(s)
+    batch = pygfx.Batch(batched, groups=groups)
+    for s in batched + single:
+        s.set_launch(pygfx.GFX_ELEMENT_BLOCK, 1)
+    batch.run(4)
+    for b, s in zip(batched, single):
+        s.run(4)
+        for f in (0, 255):
+            for x, y in zip(b.get_state(f), s.get_state(f)):
+                assert np.any(y) and np.array_equal(x, y)
+    batch.close()
+
+
 def test_launch_groups_fall_back_to_branches_when_a_mesh_cannot_share():
     """An attenuating mesh runs its own element kernel form, so a batch holding
     one keeps one branch per mesh even with launch groups requested; dropping it
