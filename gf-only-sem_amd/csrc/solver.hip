@@ -115,7 +115,7 @@ struct gfx_solver {
     int64_t Gi = 0;
     std::vector<int32_t> cl_begin;
     // with the clusters' order: what the order without clusters follows from, in
-    // which earlier builds took their images (caller elements' places on the
+    // which images were taken before (caller elements' places on the
     // centroids' curve, bit 63 for general geometry; memory directions of the C-PML
     // nodes; number of special nodes)
     std::vector<uint64_t> curve;

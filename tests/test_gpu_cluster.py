@@ -258,7 +258,7 @@ def image_case(form):
 def test_images_in_the_order_without_clusters_load(form):
     """An image taken before elements and nodes were ordered by clusters loads
     into the solver of the same inputs: the state it was taken at bit for bit,
-    and five steps on from there the displacement that build reached, to the
+    and five steps on from there the displacement reached then, to the
     rounding of another order of sums (1e-5)."""
     mesh, s = image_case(form)
     assert s.query("pml_nodal") == (form == "nodal")
